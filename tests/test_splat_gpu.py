@@ -97,6 +97,26 @@ def test_depth_ranks_follow_the_depths_of_each_call(gpu, oracle):
     ctx.close()
 
 
+@pytest.mark.parametrize("logit", [-1.0, 2.0, None])  # None: alpha0 from 0.981 to 0.9895 and one that is clamped
+@pytest.mark.parametrize("G,W,H", [
+    (1, 16, 8), (2, 17, 9), (3, 1, 1),  # one entry, one pair, a pair and a half; halves of a tile outside the image
+    (15, 16, 16), (16, 18, 16), (17, 16, 24), (33, 40, 40), (63, 16, 16), (64, 33, 7), (65, 16, 16), (130, 31, 33),
+])
+def test_compositing_at_the_edges_of_pairs_chunks_and_halves(gpu, oracle, G, W, H, logit):
+    """Lists as long as a pair, a piece of the split walk or a chunk and one more or less, pixels that stop behind either
+    entry of a pair, and, every third Gaussian, one so wide (50 000 pixels) that a stopped pixel is within its reach."""
+    params, depth = random_scene(G, W, H, seed=100 + G, scale_px=(6.0, 14.0))
+    if logit is None:
+        # two clamped layers on one pixel would leave (1 - 0.99)^2, which is below the threshold in fp32 and not in fp64
+        params[8] = np.random.default_rng(G + 7).uniform(3.95, 4.55, G)
+        params[8, G // 2] = 8.0
+    else:
+        params[8] += logit
+    params[2:4, ::3] = np.log(5e4)
+    target = np.random.default_rng(G).uniform(0, 1, (H, W, 3)).astype(np.float32)
+    _check_against_oracle(oracle, _gpu_step(gpu, W, H, params, depth, target), W, H, params, depth, target)
+
+
 def test_more_than_65536_tiles(gpu, oracle):
     """256 x 257 tiles: the pair keys (tile indices) take the 32-bit path.  Small Gaussians keep
     the oracle fast."""

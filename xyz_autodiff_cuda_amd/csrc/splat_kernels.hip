@@ -160,12 +160,10 @@ __device__ __forceinline__ int ordered_tile_of_block(int block, int tiles, const
 }
 
 // ---------------------------------------------------------------------------
-// Compositing kernels.  One wavefront per tile; lane l owns the four
-// horizontally adjacent pixels x = 4 (l % 4) .. +3 of row y = l / 4.  Four
-// pixels per lane amortise everything that is per Gaussian (the LDS reads of
-// its record, and in the backward pass the wavefront reduction of its
-// gradient) over four times the arithmetic, and a one-wavefront block needs no
-// block barrier.
+// Compositing kernels.  Blocks are single wavefronts, so no wait at a barrier is a wait for another one.  In the
+// backward pass one takes a tile: lane l owns the four horizontally adjacent pixels x = 4 (l % 4) .. +3 of row
+// y = l / 4, which amortises what is per Gaussian (the LDS reads of its record, and above all the wavefront
+// reduction of its gradient) over four times the arithmetic; in the forward pass, which reduces nothing, half a tile.
 //
 // The tile's list is staged through LDS 64 records at a time, in a form made
 // for the inner loop: the inverse covariance is pre-multiplied by
@@ -210,6 +208,34 @@ __device__ __forceinline__ std::uint32_t segment_length(std::uint32_t entries, i
     return kPark * ((groups + static_cast<std::uint32_t>(segments) - 1) / static_cast<std::uint32_t>(segments));
 }
 
+// Forward: a wavefront (a block of its own) walks the list of a tile for one 16 x 8 half of it, two horizontally adjacent
+// pixels per lane: lane l has pixels x = 2 (l % 8) and the next of row y = l / 8.
+//
+// What bounds it: the time the SIMDs take to issue its vector instructions (few wavefronts: their latency).  A
+// wavefront's fp32 add, multiply or fma takes a SIMD 2.5 cycles, a minimum, a compare, a select, a DPP form or any
+// instruction with a scalar-register operand 4.5, an exponential 8.3 (measured at eight wavefronts per SIMD).  So the
+// inner loop has only the first kind and the exponential:
+//   - no minimum against kAlphaMax where an entry cannot reach it (needs_care(), decided when it is staged);
+//   - a pixel that has stopped is moved out of every Gaussian's reach (kFarAway): alpha comes out as 0 by itself;
+//   - whether a pixel stops is tested once for two entries and all the lane's pixels, on the transmittance behind
+//     both; what has to be done then is in a branch.
+// Two entries per trip also overlap their loads and exponentials, which a wavefront alone on its SIMD needs.  (The
+// colour sums on v_mfma_f32_4x4x1_16b_f32, one instruction for three fma: no gain, it takes the SIMD 8.9 cycles and
+// nothing else issues meanwhile.)
+// Pixels per lane: one costs twice the LDS reads of two and is bound by them, four leaves half the wavefronts and can
+// leave out no half tile.  Measured with 1 / 2 / 4 (us, without the split into segments): 200 000 Gaussians at
+// 2048 x 2048 374 / 269 / 270, 100 000 at 1920 x 1080 184 / 135 / 137, 50 000 at 1277 x 719 87 / 65 / 71, 10 000 at
+// 512 x 512 26.6 / 24.7 / 32.1, 1000 at 640 x 427 6.3 / 5.9 / 6.8.
+constexpr int kForwardPixels = 2;
+constexpr int kForwardHigh = 8;
+constexpr int kForwardParts = kTile / kForwardHigh;       // wavefronts per tile
+constexpr int kForwardAcross = kTile / kForwardPixels;    // lanes across the tile
+static_assert(kForwardAcross * kForwardHigh == kChunk, "a wavefront covers its part of the tile");
+
+// Floats that are not negative compare as their bits do: a minimum of bits is one instruction, where one of floats
+// would be canonicalised first.
+__device__ __forceinline__ std::uint32_t bits_of(float x) { return __builtin_bit_cast(std::uint32_t, x); }
+
 template <bool kSplit>
 __global__ void __launch_bounds__(kChunk) render_forward_kernel(
     int width, int height, int tiles_x, int tiles, const std::uint32_t* __restrict__ range_begin,
@@ -217,136 +243,173 @@ __global__ void __launch_bounds__(kChunk) render_forward_kernel(
     const Record* __restrict__ records, float* __restrict__ image, float* __restrict__ final_T,
     std::uint32_t* __restrict__ n_contrib, int segments, float4* __restrict__ segment_state,
     const std::uint32_t* __restrict__ tile_order) {
-    __shared__ Staged staged[kChunk];
-    const int tile = ordered_tile_of_block(blockIdx.x, tiles, tile_order);
+    constexpr int kPx = kForwardPixels;
+    __shared__ Staged staged[kChunk + 1];  // the last one stands for "no entry"
+    // kSplit: transmittance behind and colour of the finished segments, [segment][pixel of the lane][lane]
+    extern __shared__ __attribute__((aligned(16))) float4 finished[];
+    const int block = static_cast<int>(blockIdx.x);
+    const int part = (block >> 3) % kForwardParts;
+    const int tile = ordered_tile_of_block((block & 7) + 8 * ((block >> 3) / kForwardParts), tiles, tile_order);
     if (tile >= tiles) return;
     const int lane = threadIdx.x;
-    const int x0 = (tile % tiles_x) * kTile + (lane & 3) * kLanePixels;
-    const int y = (tile / tiles_x) * kTile + (lane >> 2);
+    const int part_x = (tile % tiles_x) * kTile, part_y = (tile / tiles_x) * kTile + part * kForwardHigh;
+    const int x0 = part_x + (lane % kForwardAcross) * kPx;
+    const int y = part_y + lane / kForwardAcross;
     const float py = static_cast<float>(y);
-    const float px0 = static_cast<float>(x0);
 
     // the same for every lane: said so, which keeps the loop counters in scalar registers
     const std::uint32_t first = __builtin_amdgcn_readfirstlane(range_begin[tile]);
     const std::uint32_t last = __builtin_amdgcn_readfirstlane(range_end[tile]);
-    float T[kLanePixels], red[kLanePixels], green[kLanePixels], blue[kLanePixels];
-    std::uint32_t used[kLanePixels];
+    // px: kFarAway for a pixel that has stopped; T: transmittance, 1 for a pixel that has stopped (its own is in stopped_T)
+    float px[kPx], T[kPx], stopped_T[kPx], red[kPx], green[kPx], blue[kPx];
+    std::uint32_t used[kPx];  // list entries up to and with the one a pixel stopped behind
 #pragma unroll
-    for (int p = 0; p < kLanePixels; ++p) {
-        // pixels outside the image start out finished (see below) and are never stored
-        T[p] = (x0 + p < width && y < height) ? 1.f : 0.f;
+    for (int p = 0; p < kPx; ++p) {
+        // pixels outside the image start out stopped and are never stored
+        px[p] = (x0 + p < width && y < height) ? static_cast<float>(x0 + p) : kFarAway;
+        T[p] = stopped_T[p] = 1.f;
         red[p] = green[p] = blue[p] = 0.f;
         used[p] = 0;
     }
 
-    // kSplit: colour of the finished segments; red, green and blue hold the current segment's own
-    float done_red[kLanePixels], done_green[kLanePixels], done_blue[kLanePixels];
-#pragma unroll
-    for (int p = 0; p < kLanePixels; ++p) done_red[p] = done_green[p] = done_blue[p] = 0.f;
     const std::uint32_t seg_len = kSplit ? segment_length(last - first, segments) : 0u;
     std::uint32_t boundary = seg_len;
     int segment = 0;
-    auto leave_segment_state = [&]() {
+    // they wait until the colours of all later segments are known
+    auto close_segment = [&]() {
 #pragma unroll
-        for (int p = 0; p < kLanePixels; ++p)
-            if (x0 + p < width && y < height)
-                segment_state[(static_cast<std::size_t>(y) * width + x0 + p) * static_cast<std::size_t>(segments) + segment] =
-                    float4{T[p], red[p], green[p], blue[p]};  // the states of a pixel lie next to each other
+        for (int p = 0; p < kPx; ++p) {
+            finished[(segment * kPx + p) * kChunk + lane] = float4{T[p], red[p], green[p], blue[p]};
+            red[p] = green[p] = blue[p] = 0.f;
+        }
+        ++segment;
+        boundary += seg_len;
     };
 
-    const float tile_x = static_cast<float>((tile % tiles_x) * kTile), tile_y = static_cast<float>((tile / tiles_x) * kTile);
-    for (std::uint32_t base = first; base < last; base += kChunk) {
+    if (lane == 0) staged[kChunk] = Staged{};  // alpha0 = 0: reaches no pixel
+    bool live = accumulate::wave::ballot(px[0] != kFarAway) != 0;  // a lane's first pixel is inside if any of them is
+    for (std::uint32_t base = first; base < last && live; base += kChunk) {
         __syncthreads();
-        bool visible = false;
+        bool visible = false, careful = false;
         if (base + lane < last) {
             const Staged mine = stage_record(records, sorted_ids[base + lane]);
             staged[lane] = mine;
-            visible = !negligible_in_tile(mine, tile_x, tile_y);
+            visible = !negligible_in_rectangle<kTile, kForwardHigh>(mine, static_cast<float>(part_x), static_cast<float>(part_y));
+            careful = needs_care(mine);
         }
         __syncthreads();
-        // the staged entries that can be seen from this tile, front to back
-        for (std::uint64_t todo = accumulate::wave::ballot(visible); todo != 0; todo &= todo - 1) {
-            const int j = __builtin_ctzll(todo);
+        const std::uint64_t with_care = accumulate::wave::ballot(careful);
+        // the staged entries that can be seen from here, front to back, two at a time
+        for (std::uint64_t todo = accumulate::wave::ballot(visible); todo != 0 && live;) {
+            const std::uint64_t before = todo;
+            const int j0 = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            int j1 = todo != 0 ? __builtin_ctzll(todo) : kChunk;
+            const std::uint32_t at0 = base - first + j0 + 1, at1 = base - first + j1 + 1;
+            bool second = todo != 0;
             if constexpr (kSplit) {
                 // the first entry at or beyond a boundary closes the segments before it (the same for every lane)
-                while (base - first + j >= boundary) {
-                    leave_segment_state();
+                while (at0 > boundary) close_segment();
+                if (at1 > boundary) second = false;
+            }
+            if (second)
+                todo &= todo - 1;
+            else
+                j1 = kChunk;
+            const Staged r[2] = {staged[j0], staged[j1]};
+            float a[2][kPx];
 #pragma unroll
-                    for (int p = 0; p < kLanePixels; ++p) {
-                        done_red[p] += red[p];
-                        done_green[p] += green[p];
-                        done_blue[p] += blue[p];
-                        red[p] = green[p] = blue[p] = 0.f;
-                    }
-                    ++segment;
-                    boundary += seg_len;
+            for (int k = 0; k < 2; ++k) {
+                // exponent of the falloff as a polynomial in dx: (a_s dx + e) dx + f
+                const float dy = py - r[k].cy;
+                const float e = r[k].b2_s * dy;
+                const float f = r[k].c_s * dy * dy;
+#pragma unroll
+                for (int p = 0; p < kPx; ++p) {
+                    const float dx = px[p] - r[k].cx;
+                    a[k][p] = math::fp32::exp2_raw(::fmaf(::fmaf(r[k].a_s, dx, e), dx, f)) * r[k].alpha0;
                 }
             }
-            const Staged r = staged[j];
-            // exponent of the falloff as a polynomial in dx: (a_s dx + e) dx + f
-            const float dy = py - r.cy;
-            const float e = r.b2_s * dy;
-            const float f = r.c_s * dy * dy;
-            const float dx0 = px0 - r.cx;
+            if (((before ^ todo) & with_care) != 0) {
 #pragma unroll
-            for (int p = 0; p < kLanePixels; ++p) {
-                // A pixel stops, for good, before the first Gaussian it meets with T below the
-                // threshold: from then on alpha = 0 leaves T where it is, so the test stays true.
-                const bool done = T[p] < kMinTransmittance;
-                const float dx = dx0 + static_cast<float>(p);
-                const float a = math::fp32::exp2_raw(::fmaf(::fmaf(r.a_s, dx, e), dx, f)) * r.alpha0;
-                const float alpha = done ? 0.f : __builtin_fminf(a, kAlphaMax);  // a is finite: non-finite Gaussians are not binned
-                const float weight = T[p] * alpha;
-                red[p] = ::fmaf(weight, r.red, red[p]);
-                green[p] = ::fmaf(weight, r.green, green[p]);
-                blue[p] = ::fmaf(weight, r.blue, blue[p]);
-                T[p] *= 1.f - alpha;
-                used[p] = done ? used[p] : base - first + j + 1;
+                for (int p = 0; p < kPx; ++p) {
+                    const bool stopped = px[p] == kFarAway;
+                    a[0][p] = stopped ? 0.f : __builtin_fminf(a[0][p], kAlphaMax);  // finite: non-finite Gaussians are not binned
+                    a[1][p] = stopped ? 0.f : __builtin_fminf(a[1][p], kAlphaMax);
+                }
+            }
+            float behind0[kPx], behind1[kPx];  // transmittance behind the first and the second entry
+            std::uint32_t lowest = bits_of(1.f);
+#pragma unroll
+            for (int p = 0; p < kPx; ++p) {
+                behind0[p] = ::fmaf(-a[0][p], T[p], T[p]);
+                behind1[p] = ::fmaf(-a[1][p], behind0[p], behind0[p]);
+                lowest = __builtin_elementwise_min(lowest, bits_of(behind1[p]));
+            }
+            bool stops_here = false;
+            // A pixel stops, for good, behind the Gaussian that takes its transmittance below the threshold.
+            if (accumulate::wave::ballot(lowest < bits_of(kMinTransmittance)) != 0) {
+                stops_here = true;
+#pragma unroll
+                for (int p = 0; p < kPx; ++p) {
+                    if (behind1[p] < kMinTransmittance) {
+                        asm volatile("");  // a branch: moves are cheaper than as many selects
+                        used[p] = at1;
+                        stopped_T[p] = behind1[p];
+                        if (behind0[p] < kMinTransmittance) {
+                            asm volatile("");
+                            used[p] = at0;
+                            stopped_T[p] = behind0[p];
+                            a[1][p] = 0.f;
+                        }
+                        px[p] = kFarAway;
+                        behind1[p] = 1.f;
+                    }
+                }
+            }
+#pragma unroll
+            for (int p = 0; p < kPx; ++p) {
+                const float weight0 = T[p] * a[0][p], weight1 = behind0[p] * a[1][p];
+                red[p] = ::fmaf(weight1, r[1].red, ::fmaf(weight0, r[0].red, red[p]));
+                green[p] = ::fmaf(weight1, r[1].green, ::fmaf(weight0, r[0].green, green[p]));
+                blue[p] = ::fmaf(weight1, r[1].blue, ::fmaf(weight0, r[0].blue, blue[p]));
+                T[p] = behind1[p];
+            }
+            if (stops_here) {
+                bool any = false;
+#pragma unroll
+                for (int p = 0; p < kPx; ++p) any |= px[p] != kFarAway;
+                live = accumulate::wave::ballot(any) != 0;
             }
         }
-        const bool all_done = T[0] < kMinTransmittance && T[1] < kMinTransmittance && T[2] < kMinTransmittance &&
-                              T[3] < kMinTransmittance;
-        if (accumulate::wave::ballot(!all_done) == 0) break;
     }
     if constexpr (kSplit) {
-        leave_segment_state();  // of the segment the walk ended in
-#pragma unroll
-        for (int p = 0; p < kLanePixels; ++p) {
-            red[p] += done_red[p];
-            green[p] += done_green[p];
-            blue[p] += done_blue[p];
-        }
-        // What the backward walk of a segment needs is the colour behind it: the sum of the later segments'
-        // own colours.  Each state's colour is replaced by that sum (all loads first, then one pass).
-#pragma unroll
-        for (int p = 0; p < kLanePixels; ++p) {
-            if (x0 + p < width && y < height) {
-                float4* mine = segment_state + (static_cast<std::size_t>(y) * width + x0 + p) * static_cast<std::size_t>(segments);
-                float4 state[kMaxSegments];
-#pragma unroll
-                for (int k = 0; k < kMaxSegments; ++k) state[k] = mine[k < segment ? k : segment];
-                float behind[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-                for (int k = kMaxSegments - 1; k >= 0; --k) {
-                    if (k <= segment) {  // the same for every lane
-                        mine[k] = float4{state[k].x, behind[0], behind[1], behind[2]};
-                        behind[0] += state[k].y;
-                        behind[1] += state[k].z;
-                        behind[2] += state[k].w;
-                    }
-                }
-            }
-        }
+        while (live && boundary < last - first) close_segment();  // of entries that cannot be seen from here
     }
 #pragma unroll
-    for (int p = 0; p < kLanePixels; ++p) {
-        if (x0 + p < width && y < height) {
-            const std::size_t at = static_cast<std::size_t>(y) * width + x0 + p;
-            image[at * 3 + 0] = red[p];
-            image[at * 3 + 1] = green[p];
-            image[at * 3 + 2] = blue[p];
-            final_T[at] = T[p];
-            n_contrib[at] = used[p];
+    for (int p = 0; p < kPx; ++p) {
+        const bool inside = x0 + p < width && y < height;
+        const std::size_t at = static_cast<std::size_t>(y) * width + x0 + p;
+        float sum[3] = {red[p], green[p], blue[p]};
+        if constexpr (kSplit) {
+            // What the backward walk of a segment needs is the colour behind it: the sum of the later segments' own
+            // colours (a difference of running totals would cancel).
+            for (int k = segment - 1; k >= 0; --k) {
+                const float4 own = finished[(k * kPx + p) * kChunk + lane];
+                if (inside)
+                    segment_state[k * static_cast<std::size_t>(width) * height + at] = float4{own.x, sum[0], sum[1], sum[2]};
+                sum[0] += own.y;
+                sum[1] += own.z;
+                sum[2] += own.w;
+            }
+        }
+        if (inside) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) image[at * 3 + c] = sum[c];
+            const bool stopped = px[p] == kFarAway;
+            final_T[at] = stopped ? stopped_T[p] : T[p];
+            // (a pixel that has not stopped used the whole list: the backward pass leaves out less, whole tiles' entries)
+            n_contrib[at] = stopped ? used[p] : last - first;
         }
     }
 }
@@ -441,6 +504,10 @@ __global__ void __launch_bounds__(kChunk) render_backward_kernel(
     const int segment = kSplit ? static_cast<int>(blockIdx.x / blocks_per_segment) : 0;
     const int tile = ordered_tile_of_block(static_cast<int>(blockIdx.x % blocks_per_segment), tiles, tile_order);
     if (tile >= tiles) return;
+    const std::uint32_t first = __builtin_amdgcn_readfirstlane(range_begin[tile]);
+    const std::uint32_t seg_len = kSplit ? segment_length(range_end[tile] - first, segments) : 0u;
+    // a segment behind the end of the list (most of them where lists are short) leaves before it loads anything else
+    if (kSplit && segment > 0 && static_cast<std::uint32_t>(segment) * seg_len >= range_end[tile] - first) return;
     const int lane = threadIdx.x;
     const int x0 = (tile % tiles_x) * kTile + (lane & 3) * kLanePixels;
     const int y = (tile / tiles_x) * kTile + (lane >> 2);
@@ -480,12 +547,10 @@ __global__ void __launch_bounds__(kChunk) render_backward_kernel(
     }
     const std::uint32_t deepest = wave_max(my_max);  // entries [0, deepest) were composited by some pixel
     if (deepest == 0) return;
-    const std::uint32_t first = range_begin[tile];
     const float px0 = static_cast<float>(x0);
     // this block walks entries [walk_first, walk_last) of the list, back to front
     std::uint32_t walk_first = 0, walk_last = deepest;
     if constexpr (kSplit) {
-        const std::uint32_t seg_len = segment_length(range_end[tile] - first, segments);
         walk_first = static_cast<std::uint32_t>(segment) * seg_len;
         if (walk_first >= deepest) return;
         walk_last = walk_first + seg_len < deepest ? walk_first + seg_len : deepest;
@@ -494,9 +559,8 @@ __global__ void __launch_bounds__(kChunk) render_backward_kernel(
 #pragma unroll
         for (int p = 0; p < kLanePixels; ++p) {
             if (used[p] > walk_last) {
-                // the states of a pixel lie next to each other
-                const float4* mine = segment_state + (static_cast<std::size_t>(y) * width + x0 + p) * static_cast<std::size_t>(segments);
-                const float4 state = mine[segment];
+                const std::size_t pixels = static_cast<std::size_t>(width) * height;
+                const float4 state = segment_state[segment * pixels + static_cast<std::size_t>(y) * width + x0 + p];
                 T[p] = state.x;
                 const float behind[3] = {state.y, state.z, state.w};
                 D[p] = -::fmaf(dC[p][2], behind[2], ::fmaf(dC[p][1], behind[1], dC[p][0] * behind[0]));
@@ -698,14 +762,15 @@ int launch_render_forward(hipStream_t s, int width, int height, const std::uint3
     // the order both compositing kernels of this step take the tiles in
     hipLaunchKernelGGL(tile_order_kernel, dim3(8), dim3(1024), 0, s, tiles, range_begin, range_end, tile_order);
     XAD_HIP_TRY(hipGetLastError());
-    XAD_REQUIRE(segments >= 1 && (segments == 1 || segment_state), "splat: a split walk needs its per-segment state");
+    XAD_REQUIRE(segments >= 1 && segments <= kMaxSegments && (segments == 1 || segment_state), "splat: a split walk needs its per-segment state");
+    const dim3 grid(padded_tile_blocks(tiles) * kForwardParts), block(kChunk);
     if (segments > 1)
-        hipLaunchKernelGGL(render_forward_kernel<true>, dim3(padded_tile_blocks(tiles)), dim3(kChunk), 0, s, width, height,
-                           tiles_x, tiles, range_begin, range_end, sorted_ids, records, image, final_T, n_contrib, segments,
-                           segment_state, tile_order);
+        hipLaunchKernelGGL(render_forward_kernel<true>, grid, block, (segments - 1) * kForwardPixels * kChunk * sizeof(float4), s,
+                           width, height, tiles_x, tiles, range_begin, range_end, sorted_ids, records, image, final_T, n_contrib,
+                           segments, segment_state, tile_order);
     else
-        hipLaunchKernelGGL(render_forward_kernel<false>, dim3(padded_tile_blocks(tiles)), dim3(kChunk), 0, s, width, height,
-                           tiles_x, tiles, range_begin, range_end, sorted_ids, records, image, final_T, n_contrib, 1, nullptr, tile_order);
+        hipLaunchKernelGGL(render_forward_kernel<false>, grid, block, 0, s, width, height, tiles_x, tiles, range_begin, range_end,
+                           sorted_ids, records, image, final_T, n_contrib, 1, nullptr, tile_order);
     XAD_HIP_TRY(hipGetLastError());
     return XAD_OK;
 }

@@ -17,8 +17,8 @@ constexpr float kHalfLog2e = 0.72134752044448170368f;  // log2(e) / 2
 
 struct alignas(16) Staged {
     float cx, cy, a_s, b2_s;          // centre; a' and 2b'
-    float c_s, alpha0, red, green;    // c'; sigmoid(opacity); colour
-    float blue, a, b, c;              // colour; inverse covariance as stored
+    float c_s, alpha0, a, b;          // c'; sigmoid(opacity); inverse covariance as stored
+    float red, green, blue, c;        // colour (a lane takes the channel of its number modulo 4); inverse covariance
 };
 static_assert(sizeof(Staged) == 48, "Staged must be three float4");
 
@@ -52,22 +52,43 @@ XAD_INLINE Staged stage_record(const Record* __restrict__ records, std::uint32_t
 // counts are not affected.  Comparisons with NaN are false, so an odd record is kept.
 constexpr float kNegligibleAlpha = 1e-8f;
 
-XAD_INLINE bool negligible_in_tile(const Staged& s, float tile_x, float tile_y) {
-    const float x0 = tile_x - s.cx, x1 = x0 + static_cast<float>(kTile - 1);
-    const float y0 = tile_y - s.cy, y1 = y0 + static_cast<float>(kTile - 1);
+template <int kWide, int kHigh>
+XAD_INLINE bool negligible_in_rectangle(const Staged& s, float left, float top) {
+    const float x0 = left - s.cx, x1 = x0 + static_cast<float>(kWide - 1);
+    const float y0 = top - s.cy, y1 = y0 + static_cast<float>(kHigh - 1);
     float q_min = 0.f;
     if (!(x0 <= 0.f && x1 >= 0.f && y0 <= 0.f && y1 >= 0.f)) {
+        const float x_of_y = -s.b / s.a, y_of_x = -s.b / s.c;  // where q is least along a line
         auto along_x = [&](float y) {  // min over x in [x0, x1] of a x^2 + 2 b x y + c y^2
-            const float x = __builtin_fminf(__builtin_fmaxf(-s.b * y / s.a, x0), x1);
+            const float x = __builtin_fminf(__builtin_fmaxf(x_of_y * y, x0), x1);
             return ::fmaf(::fmaf(s.a, x, 2.f * s.b * y), x, s.c * y * y);
         };
         auto along_y = [&](float x) {
-            const float y = __builtin_fminf(__builtin_fmaxf(-s.b * x / s.c, y0), y1);
+            const float y = __builtin_fminf(__builtin_fmaxf(y_of_x * x, y0), y1);
             return ::fmaf(::fmaf(s.c, y, 2.f * s.b * x), y, s.a * x * x);
         };
         q_min = __builtin_fminf(__builtin_fminf(along_x(y0), along_x(y1)), __builtin_fminf(along_y(x0), along_y(x1)));
     }
     return s.alpha0 * math::fp32::exp2_raw(-kHalfLog2e * q_min) < kNegligibleAlpha;
+}
+
+XAD_INLINE bool negligible_in_tile(const Staged& s, float tile_x, float tile_y) {
+    return negligible_in_rectangle<kTile, kTile>(s, tile_x, tile_y);
+}
+
+// Entries for which the compositing loops have to make sure of two things themselves.  For all others
+//   - alpha stays below kAlphaMax at every pixel: alpha0 does by a margin, and q cannot come out negative by more
+//     than rounding.  (q >= (1 - |b| / sqrt(ac)) (a dx^2 + c dy^2), the rounding of its three terms is at most
+//     5e-7 (a dx^2 + c dy^2), and 1 - |b| / sqrt(ac) >= (ac - b^2) / 2ac > 5e-6);
+//   - a pixel whose x is kFarAway gets alpha = 0: there a dx^2 >= 1e-9 1e36, and neither 2 |b dx dy| <=
+//     2 sqrt(ac) 1e18 |dy| nor c dy^2 comes near it (|dy| < 1e6).
+// Comparisons with NaN are false, so an odd record is taken with care.
+constexpr float kFarAway = 1e18f;
+
+XAD_INLINE bool needs_care(const Staged& s) {
+    const float ac = s.a * s.c;
+    return !(s.alpha0 <= 0.98f && s.a >= 1e-9f && s.a <= 1e9f && s.c >= 1e-9f && s.c <= 1e9f && ac - s.b * s.b >= 1e-5f * ac &&
+             s.cx >= -1e6f && s.cx <= 1e6f && s.cy >= -5e5f && s.cy <= 5e5f);
 }
 
 }  // namespace xad_splat
