@@ -174,7 +174,7 @@ __device__ __forceinline__ int ordered_tile_of_block(int block, int tiles, const
 // (examples/mini-gaussian-splatting/gaussian_splatting_kernel.cu:45-55) in fused form.
 constexpr int kLanePixels = 4;
 constexpr int kChunk = 64;
-constexpr int kPark = 16;  // list entries whose gradient sums are finished and written out together
+constexpr int kPark = 16;  // (even) list entries whose gradient sums are finished and written out together
 __device__ __forceinline__ std::uint32_t wave_max(std::uint32_t v) {
     // 64-lane maximum through the LDS crossbar-free DPP path: rows, then row heads
     auto step = [](std::uint32_t x, auto ctrl) {
@@ -414,63 +414,85 @@ __global__ void __launch_bounds__(kChunk) render_forward_kernel(
     }
 }
 
-// Sum of nine per-lane values over each row of 16 lanes, cheaper than nine separate
-// reductions.  v[0..7] go through a reduce-scatter: at each of three steps a lane
-// keeps half of its values, the half chosen by one bit of its lane number, and
-// adds the copies held by the partner lane that differs in that bit.  For bits 2
-// and 3 (partners 4 and 8 lanes away) the choice is made by the bank mask of the
-// DPP add itself: one instruction serves the lanes whose bit is clear, a second
-// one the others, and no select is needed.  Bit 0 takes the ordinary select and
-// quad swap; a last quad swap over bit 1 completes the row.  v[8] takes the
-// ordinary four row steps.
-// Result: lane l of a row holds the row's sum of v[reduced_index(l)].
-__device__ __forceinline__ int reduced_index(int lane) {
-    const int r = lane & 15;
-    return (r & 2) ? 8 : ((r & 1) << 2) | ((r >> 3) << 1) | ((r >> 2) & 1);
-}
+// Sums of nine per-lane values of each of two list entries over each row of 16 lanes, cheaper than eighteen separate
+// reductions.  The first eight of both go through a reduce-scatter: at each of four steps a lane keeps half of its
+// values, the half chosen by one bit of its lane number, and adds the copies held by the partner lane that differs
+// in that bit.  For bits 2 and 3 (partners 4 and 8 lanes away) the choice is made by the bank mask of the DPP add
+// itself: one instruction serves the lanes whose bit is clear, a second one the others, and no select is needed.
+// Bits 0 and 1 take the ordinary select and quad swap.  The two ninth values share their first step and are then
+// added up along the row.  38 instructions for two entries (2 x 22 one by one), and their waits are shared.
+// Result: lane l of a row holds the row's sum of value reduced_index(l) of entry reduced_entry(l) in .scattered, and in
+// .ninth that of the ninth value of the first entry (bit 2 of l clear) or the second.
+__device__ __forceinline__ int reduced_index(int lane) { return ((lane & 1) << 2) | (((lane >> 3) & 1) << 1) | ((lane >> 2) & 1); }
+__device__ __forceinline__ int reduced_entry(int lane) { return (lane >> 1) & 1; }
 
-__device__ __forceinline__ float reduce_scatter9(const float (&v)[9], int lane) {
+struct RowSums {
+    float scattered, ninth;
+};
+
+__device__ __forceinline__ RowSums reduce_scatter_pair(const float (&a)[9], const float (&b)[9], int lane) {
     // bit 2: banks 0 and 2 (lanes 0-3, 8-11 of a row) keep the even value and read lane + 4,
     // banks 1 and 3 keep the odd one and read lane - 4.  The leading wait covers the two idle
     // cycles a DPP read needs after a vector write of the same register.
-    float w0, w1, w2, w3;
+    float w[8], x;
     asm volatile(
         "s_nop 1\n\t"
-        "v_add_f32_dpp %0, %4, %4 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
-        "v_add_f32_dpp %0, %5, %5 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
-        "v_add_f32_dpp %1, %6, %6 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
-        "v_add_f32_dpp %1, %7, %7 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
-        "v_add_f32_dpp %2, %8, %8 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
-        "v_add_f32_dpp %2, %9, %9 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
-        "v_add_f32_dpp %3, %10, %10 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
-        "v_add_f32_dpp %3, %11, %11 row_shr:4 row_mask:0xf bank_mask:0xa"
-        : "=&v"(w0), "=&v"(w1), "=&v"(w2), "=&v"(w3)
-        : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]));
+        "v_add_f32_dpp %0, %9, %9 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %0, %10, %10 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %1, %11, %11 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %1, %12, %12 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %2, %13, %13 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %2, %14, %14 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %3, %15, %15 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %3, %16, %16 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %4, %17, %17 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %4, %18, %18 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %5, %19, %19 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %5, %20, %20 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %6, %21, %21 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %6, %22, %22 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %7, %23, %23 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %7, %24, %24 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %8, %25, %25 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %8, %26, %26 row_shr:4 row_mask:0xf bank_mask:0xa"
+        : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]), "=&v"(w[4]), "=&v"(w[5]), "=&v"(w[6]), "=&v"(w[7]), "=&v"(x)
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]),
+          "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]), "v"(a[8]), "v"(b[8]));
     // bit 3: banks 0 and 1 (lanes 0-7) keep the even value, banks 2 and 3 the odd one; the partner is 8 lanes round the row
-    float u0, u1;
+    float u[4], y;
     asm volatile(
         "s_nop 1\n\t"
-        "v_add_f32_dpp %0, %2, %2 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-        "v_add_f32_dpp %0, %3, %3 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-        "v_add_f32_dpp %1, %4, %4 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-        "v_add_f32_dpp %1, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xc"
-        : "=&v"(u0), "=&v"(u1)
-        : "v"(w0), "v"(w1), "v"(w2), "v"(w3));
-    const bool b0 = lane & 1;
-    const float keep = b0 ? u1 : u0;
-    const float send = b0 ? u0 : u1;
-    float t = keep + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, send), 0xB1, 0xF, 0xF, true));
-    t = accumulate::wave::dpp_add<0x4E>(t);  // bit 1
-
-    float x = v[8];
-    x = accumulate::wave::dpp_add<0xB1>(x);
-    x = accumulate::wave::dpp_add<0x4E>(x);
-    x = accumulate::wave::dpp_add<0x141>(x);
-    x = accumulate::wave::dpp_add<0x140>(x);
-    return (lane & 2) ? x : t;
+        "v_add_f32_dpp %0, %5, %5 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %0, %6, %6 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %1, %7, %7 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %1, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %2, %9, %9 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %2, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %3, %11, %11 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %3, %12, %12 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %4, %13, %13 row_ror:8 row_mask:0xf bank_mask:0xf"
+        : "=&v"(u[0]), "=&v"(u[1]), "=&v"(u[2]), "=&v"(u[3]), "=&v"(y)
+        : "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(x));
+    auto swapped = [](float v, auto ctrl) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xF, 0xF, true));
+    };
+    const bool b0 = lane & 1, b1 = lane & 2;
+    constexpr std::integral_constant<int, 0xB1> bit0{};
+    constexpr std::integral_constant<int, 0x4E> bit1{};
+    const float t0 = (b0 ? u[1] : u[0]) + swapped(b0 ? u[0] : u[1], bit0);
+    const float t1 = (b0 ? u[3] : u[2]) + swapped(b0 ? u[2] : u[3], bit0);
+    y = accumulate::wave::dpp_add<0xB1>(y);
+    return {(b1 ? t1 : t0) + swapped(b1 ? t0 : t1, bit1), accumulate::wave::dpp_add<0x4E>(y)};
 }
 
-// Compositing backward.  Lists are walked back to front.  For every Gaussian
+// Compositing backward.  What bounds it is, as in the forward pass, the time its vector instructions take to issue, and
+// where there are few wavefronts their latency; so here, too, idle pixels are out of reach instead of masked, the
+// clamp is applied to entries that can reach it, entries go two at a time, and what lies behind a Gaussian is kept
+// divided by the transmittance there, which needs one multiplication less than absolute colours.  Before / after
+// (us): 200 000 Gaussians at 2048 x 2048 820 / 730, 50 000 at 1277 x 719 185 / 157, 10 000 at 512 x 512 52 / 47.
+// (82 registers, five wavefronts per SIMD; held to 80 and six it spills: 722 / 164 / 51.  One entry at a time, also 80
+// registers: 754 / 161 / 48.  Without its atomics it takes the same time.)
+// Lists are walked back to front.  For every Gaussian
 // each lane adds up, over its four pixels, the nine sums that determine
 // d loss / d record:
 //   S_x, S_y, S_xx, S_xy, S_yy = sum of g_q {dx, dy, dx^2, dx dy, dy^2},  g_q = d loss / d q
@@ -478,7 +500,7 @@ __device__ __forceinline__ float reduce_scatter9(const float (&v)[9], int lane) 
 // (the Mahalanobis backward rule, d centre = -g_q (2a dx + 2b dy, 2b dx + 2c dy),
 // d inv = g_q (dx^2, 2 dx dy, dy^2), is linear in those sums, so it is applied
 // once per Gaussian instead of once per pixel).  The nine values are reduced
-// over each row of 16 lanes by reduce_scatter9 and parked in LDS; after every kPark
+// over each row of 16 lanes by reduce_scatter_pair and parked in LDS; after every kPark
 // list entries lane j finishes entry j of the group, and the group's record
 // gradients are added to the global accumulator with consecutive lanes on
 // consecutive fields of consecutive entries: one atomic per (tile, Gaussian,
@@ -491,12 +513,13 @@ __global__ void __launch_bounds__(kChunk) render_backward_kernel(
     const float* __restrict__ final_T, const std::uint32_t* __restrict__ n_contrib, float* __restrict__ record_grads,
     double* __restrict__ loss, int segments, const float4* __restrict__ segment_state,
     const std::uint32_t* __restrict__ tile_order) {
-    __shared__ Staged staged[kChunk];
+    __shared__ Staged staged[kChunk + 1];  // the last one stands for "no entry"
     __shared__ std::uint32_t staged_id[kChunk];
     // Row sums wait here until a group of kPark list entries is complete.  Small on purpose: LDS per
     // block, not registers, is what limits the number of resident wavefronts.
-    __shared__ float parked[kPark][4][9];  // [list entry within its group][row of 16 lanes][value]
+    __shared__ float parked[kPark][4][9];  // [list entry within its group][row of 16 lanes][value]; 36 to an entry
     __shared__ int parked_entry[kPark];    // which staged entry that is
+    __shared__ std::uint32_t wakes[2];     // a bit per staged entry
 
     // kSplit: all tiles' first segments, then all second ones, ...: every XCD gets its band of tiles of every
     // segment (the late segments are the ones that often have nothing to walk)
@@ -514,16 +537,15 @@ __global__ void __launch_bounds__(kChunk) render_backward_kernel(
     const float py = static_cast<float>(y);
 
     // Per pixel: dC = d loss / d colour, T = transmittance behind the Gaussian the walk is at,
-    // D = -dC . (colour composited behind that Gaussian), in absolute (not normalised) terms.  (Kept
-    // negated so that no negated reciprocal is needed: the compiler would compute one separately.)
-    float dC[kLanePixels][3], T[kLanePixels], D[kLanePixels];
+    // R = dC . (colour composited behind that Gaussian) / T.
+    float dC[kLanePixels][3], T[kLanePixels], R[kLanePixels];
     std::uint32_t used[kLanePixels];
     float my_loss = 0.f;
     std::uint32_t my_max = 0;
 #pragma unroll
     for (int p = 0; p < kLanePixels; ++p) {
         T[p] = 1.f;
-        D[p] = 0.f;
+        R[p] = 0.f;
         used[p] = 0;
 #pragma unroll
         for (int c = 0; c < 3; ++c) dC[p][c] = 0.f;
@@ -563,7 +585,7 @@ __global__ void __launch_bounds__(kChunk) render_backward_kernel(
                 const float4 state = segment_state[segment * pixels + static_cast<std::size_t>(y) * width + x0 + p];
                 T[p] = state.x;
                 const float behind[3] = {state.y, state.z, state.w};
-                D[p] = -::fmaf(dC[p][2], behind[2], ::fmaf(dC[p][1], behind[1], dC[p][0] * behind[0]));
+                R[p] = ::fmaf(dC[p][2], behind[2], ::fmaf(dC[p][1], behind[1], dC[p][0] * behind[0])) / state.x;
             }
         }
     }
@@ -571,86 +593,163 @@ __global__ void __launch_bounds__(kChunk) render_backward_kernel(
     // wait for those loads ends up there, where it also waits, at every entry, for the atomics issued
     // since; a use of the values here settles them before the loop.
 #pragma unroll
-    for (int p = 0; p < kLanePixels; ++p) asm volatile("" : "+v"(T[p]), "+v"(D[p]));
-    // which of the nine row sums this lane ends up with; eight lanes and one more per row park theirs
-    const int park_index = reduced_index(lane);
-    const bool parks = !(lane & 2) || (lane & 15) == 2;
+    for (int p = 0; p < kLanePixels; ++p) asm volatile("" : "+v"(T[p]), "+v"(R[p]));
+    // A pixel is idle until the walk reaches the last Gaussian it composited: until then it is out of every Gaussian's
+    // reach (kFarAway), so that alpha and with it everything it would add comes out as 0 by itself.
+    float px[kLanePixels];
+#pragma unroll
+    for (int p = 0; p < kLanePixels; ++p) px[p] = used[p] >= walk_last ? px0 + static_cast<float>(p) : kFarAway;
+    // which of the eighteen row sums this lane parks, and which ninth value if any
+    float* const park_scattered = &parked[reduced_entry(lane)][lane >> 4][reduced_index(lane)];
+    float* const park_ninth = &parked[(lane >> 2) & 1][lane >> 4][8];
+    const bool parks_ninth = (lane & 11) == 0;
+    if (lane == 0) {
+        Staged none{};  // out of reach of every pixel: its falloff is 0
+        none.cx = 2.f * kFarAway;
+        none.a_s = -1.f;
+        staged[kChunk] = none;
+    }
 
     const float tile_x = static_cast<float>((tile % tiles_x) * kTile), tile_y = static_cast<float>((tile / tiles_x) * kTile);
     for (std::uint32_t chunk = (walk_last - walk_first + kChunk - 1) / kChunk; chunk-- > 0;) {
         const std::uint32_t chunk_first = walk_first + chunk * kChunk;
         const int count = static_cast<int>(walk_last - chunk_first < kChunk ? walk_last - chunk_first : kChunk);
         __syncthreads();
-        bool visible = false;
+        if (lane < 2) wakes[lane] = 0;
+        bool visible = false, careful = false;
         if (lane < count) {
             const std::uint32_t id = sorted_ids[first + chunk_first + lane];
             staged_id[lane] = id;
             const Staged mine = stage_record(records, id);
             staged[lane] = mine;
-            visible = !negligible_in_tile(mine, tile_x, tile_y);  // the forward pass left the same entries out
+            visible = !negligible_in_tile(mine, tile_x, tile_y);  // what the forward pass left out and what reaches its other half
+            careful = needs_care(mine);
         }
         __syncthreads();
+        // the entries of this chunk at which a pixel wakes up: the last one it composited
+#pragma unroll
+        for (int p = 0; p < kLanePixels; ++p) {
+            const std::uint32_t entry = used[p] - 1 - chunk_first;  // of a pixel that composited nothing: far beyond
+            if (used[p] < walk_last && entry < static_cast<std::uint32_t>(kChunk)) atomicOr(&wakes[entry >> 5], 1u << (entry & 31));
+        }
+        __syncthreads();
+        std::uint64_t waking = static_cast<std::uint64_t>(__builtin_amdgcn_readfirstlane(wakes[1])) << 32 |
+                               static_cast<std::uint32_t>(__builtin_amdgcn_readfirstlane(wakes[0]));
+        const std::uint64_t with_care = accumulate::wave::ballot(careful);
 
         // the staged entries that can be seen from this tile, back to front, in groups of up to kPark
         std::uint64_t todo = accumulate::wave::ballot(visible);
         while (todo != 0) {
             int members = 0;
-            for (; todo != 0 && members < kPark; ++members) {
-                const int j = 63 - __builtin_clzll(todo);
-                todo &= ~(std::uint64_t(1) << j);
-                const std::uint32_t position = chunk_first + j;
-                const Staged r = staged[j];
-                // exponent of the falloff as a polynomial in dx: (a_s dx + e) dx + f
-                const float dy = py - r.cy;
-                const float e = r.b2_s * dy;
-                const float f = r.c_s * dy * dy;
-                const float dx0 = px0 - r.cx;
-                float through[kLanePixels];  // d loss / d alpha0 of this Gaussian, per pixel
-                float colour[3] = {0.f, 0.f, 0.f};
+            const std::uint64_t before = todo;
+            // two at a time: their loads and exponentials overlap, and they share the reduction
+            while (todo != 0 && members < kPark) {
+                const int j0 = 63 - __builtin_clzll(todo);
+                todo &= ~(std::uint64_t(1) << j0);
+                const bool second = todo != 0;
+                const int j1 = second ? 63 - __builtin_clzll(todo) : kChunk;
+                const std::uint64_t pair = std::uint64_t(1) << j0 | (second ? std::uint64_t(1) << j1 : 0);
+                todo &= ~pair;
+                const Staged r[2] = {staged[j0], staged[j1]};
+                const int lower = second ? j1 : j0;
+                // pixels wake up at or above the lower of the two entries (one that is not visible is made up for here)
+                const bool wake = (waking >> lower) != 0;
+                if (wake) {
 #pragma unroll
-                for (int p = 0; p < kLanePixels; ++p) {
-                    // A pixel is idle until the walk reaches the last Gaussian it composited, and
-                    // active from there on.  While idle, alpha = 0 leaves T and D at their initial
-                    // values, so no branch is needed.
-                    const bool active = position < used[p];
-                    const float dx = dx0 + static_cast<float>(p);
-                    const float falloff = math::fp32::exp2_raw(::fmaf(::fmaf(r.a_s, dx, e), dx, f));
-                    const float a = falloff * r.alpha0;
-                    const bool clamped = a > kAlphaMax;
-                    const float alpha = active ? __builtin_fminf(a, kAlphaMax) : 0.f;
-                    // 1 / (1 - alpha): v_rcp_f32 and one Newton step.  The hardware reciprocal alone leans one way,
-                    // and T is rebuilt from the back by one such factor per entry, so over lists of hundreds of
-                    // entries every gradient leaned with it (measured at 200 000 Gaussians: the sum of
-                    // sign(g) (gpu - exact) over the sum of the terms' magnitudes 6.1e-7, with the step 3.5e-7,
-                    // the median error of the colour gradients 7.0e-7 -> 4.8e-7 of that mass; +2 % on the kernel).
-                    const float keep = 1.f - alpha;
-                    float inv = __builtin_amdgcn_rcpf(keep);
-                    inv = ::fmaf(::fmaf(-keep, inv, 1.f), inv, inv);
-                    const float T_front = T[p] * inv;  // transmittance in front of this Gaussian
-                    const float dot = ::fmaf(dC[p][2], r.blue, ::fmaf(dC[p][1], r.green, dC[p][0] * r.red));
-                    // d loss / d alpha = T_front (dC . colour) - (dC . colour behind) / (1 - alpha)
-                    //                  = T_front dot + D inv
-                    const float d_alpha = ::fmaf(D[p], inv, T_front * dot);
-                    const float weight = alpha * T_front;
-                    D[p] = ::fmaf(-weight, dot, D[p]);
-                    T[p] = T_front;
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) colour[c] = ::fmaf(weight, dC[p][c], colour[c]);
-                    through[p] = (active && !clamped) ? d_alpha * falloff : 0.f;
+                    for (int p = 0; p < kLanePixels; ++p) {
+                        if (chunk_first + lower < used[p]) {
+                            asm volatile("");  // a branch: one move instead of a select
+                            px[p] = px0 + static_cast<float>(p);
+                        }
+                    }
+                    waking &= (std::uint64_t(1) << lower) - 1;
                 }
-                // Moments of `through` over the lane's four pixels (offsets 0..3 from dx0) give the five
-                // sums  sum t dx^i dy^j  the Mahalanobis backward rule needs; their common factor
-                // d alpha / d q / falloff = -alpha0 / 2 is applied once per Gaussian below.
-                const float m0 = (through[0] + through[1]) + (through[2] + through[3]);
-                const float m1 = ::fmaf(3.f, through[3], ::fmaf(2.f, through[2], through[1]));
-                const float m2 = ::fmaf(9.f, through[3], ::fmaf(4.f, through[2], through[1]));
-                const float sx = ::fmaf(dx0, m0, m1);
-                const float sy = dy * m0;
-                const float v[9] = {sx, sy, ::fmaf(dx0, sx + m1, m2), dy * sx, dy * sy, colour[0], colour[1], colour[2], m0};
-                const float mine = reduce_scatter9(v, lane);
-                if (parks) parked[members][lane >> 4][park_index] = mine;
-                if (lane == 0) parked_entry[members] = j;
+                float dy[2], dx0[2], falloff[2][kLanePixels], alpha[2][kLanePixels];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    // exponent of the falloff as a polynomial in dx: (a_s dx + e) dx + f
+                    dy[k] = py - r[k].cy;
+                    dx0[k] = px0 - r[k].cx;
+                    const float e = r[k].b2_s * dy[k];
+                    const float f = r[k].c_s * dy[k] * dy[k];
+#pragma unroll
+                    for (int p = 0; p < kLanePixels; ++p) {
+                        const float dx = px[p] - r[k].cx;
+                        falloff[k][p] = math::fp32::exp2_raw(::fmaf(::fmaf(r[k].a_s, dx, e), dx, f));
+                        alpha[k][p] = falloff[k][p] * r[k].alpha0;
+                    }
+                }
+                if (wake) {  // those that woke up for the second entry only
+#pragma unroll
+                    for (int p = 0; p < kLanePixels; ++p) {
+                        if (chunk_first + j0 >= used[p]) {
+                            asm volatile("");
+                            falloff[0][p] = alpha[0][p] = 0.f;
+                        }
+                    }
+                }
+                if ((with_care & pair) != 0) {
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+                        for (int p = 0; p < kLanePixels; ++p) {
+                            const bool idle = px[p] == kFarAway, clamped = alpha[k][p] > kAlphaMax;
+                            falloff[k][p] = idle || clamped ? 0.f : falloff[k][p];  // a clamped alpha passes no gradient on
+                            alpha[k][p] = idle ? 0.f : __builtin_fminf(alpha[k][p], kAlphaMax);
+                        }
+                    }
+                }
+                float v[2][9];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    float through[kLanePixels];  // d loss / d alpha0 of this Gaussian, per pixel
+                    float colour[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int p = 0; p < kLanePixels; ++p) {
+                        // Transmittance in front of this Gaussian, T / (1 - alpha): v_rcp_f32 and one correction of the
+                        // quotient.  The hardware reciprocal alone leans one way, and T is rebuilt from the back by one
+                        // such factor per entry, so over lists of hundreds of entries every gradient leaned with it
+                        // (measured at 200 000 Gaussians: the sum of sign(g) (gpu - exact) over the sum of the terms'
+                        // magnitudes 6.1e-7, with the reciprocal corrected 3.5e-7).
+                        const float keep = 1.f - alpha[k][p];
+                        const float inv = __builtin_amdgcn_rcpf(keep);
+                        float T_front = T[p] * inv;
+                        T_front = ::fmaf(::fmaf(-keep, T_front, T[p]), inv, T_front);
+                        // d loss / d alpha = T_front (dC . colour - dC . colour behind, normalised)
+                        const float apart = ::fmaf(dC[p][2], r[k].blue, ::fmaf(dC[p][1], r[k].green, ::fmaf(dC[p][0], r[k].red, -R[p])));
+                        const float d_alpha = T_front * apart;
+                        const float weight = alpha[k][p] * T_front;
+                        R[p] = ::fmaf(alpha[k][p], apart, R[p]);
+                        T[p] = T_front;
+#pragma unroll
+                        for (int c = 0; c < 3; ++c) colour[c] = ::fmaf(weight, dC[p][c], colour[c]);
+                        through[p] = d_alpha * falloff[k][p];
+                    }
+                    // Moments of `through` over the lane's four pixels (offsets 0..3 from dx0) give the five
+                    // sums  sum t dx^i dy^j  the Mahalanobis backward rule needs; their common factor
+                    // d alpha / d q / falloff = -alpha0 / 2 is applied once per Gaussian below.
+                    const float m0 = (through[0] + through[1]) + (through[2] + through[3]);
+                    const float m1 = ::fmaf(3.f, through[3], ::fmaf(2.f, through[2], through[1]));
+                    const float m2 = ::fmaf(9.f, through[3], ::fmaf(4.f, through[2], through[1]));
+                    const float sx = ::fmaf(dx0[k], m0, m1);
+                    const float sy = dy[k] * m0;
+                    v[k][0] = sx;
+                    v[k][1] = sy;
+                    v[k][2] = ::fmaf(dx0[k], sx + m1, m2);
+                    v[k][3] = dy[k] * sx;
+                    v[k][4] = dy[k] * sy;
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) v[k][5 + c] = colour[c];
+                    v[k][8] = m0;
+                }
+                const RowSums sums = reduce_scatter_pair(v[0], v[1], lane);
+                park_scattered[members * 36] = sums.scattered;
+                if (parks_ninth) park_ninth[members * 36] = sums.ninth;
+                members += second ? 2 : 1;  // (a missing second entry parks zeros, into rows that nobody reads)
             }
+            // member m is the m-th of the group's entries from the back
+            const std::uint64_t taken = (before & ~todo) >> lane;
+            if (taken & 1) parked_entry[__builtin_popcountll(taken) - 1] = lane;
             __syncthreads();
             if (lane < members) {
                 float s[9];
