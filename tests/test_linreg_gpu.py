@@ -131,6 +131,23 @@ def test_sgd_trajectory_matches_oracle(gpu, oracle, batch, epochs):
     assert hist[-1] < (0.5 if epochs >= 300 else 1.0) * hist[0]
 
 
+@pytest.mark.parametrize("batch,epochs", [
+    (1, 130), (63, 64), (1023, 65), (1024, 3), (1025, 64),  # one sample a lane and a few more; whole launches of steps and one more
+    (2048, 1), (2049, 65), (4097, 43), (8192, 22), (8193, 5),  # the largest batch one block takes, and the first it does not
+])
+def test_sgd_where_the_ways_of_taking_steps_meet(gpu, oracle, batch, epochs):
+    import torch
+
+    total = 5003
+    x1, x2, y = linreg.synthetic_data(total, seed=8)
+    rows = np.concatenate([linreg.batch_rows(3, e, batch, total) for e in range(epochs)])
+    want_p, want_hist = oracle.linreg_sgd(x1, x2, y, rows, linreg.INITIAL_PARAMS, batch, epochs, 1e-4, 1e-6)
+    params = torch.tensor(linreg.INITIAL_PARAMS, dtype=torch.float64, device=gpu)
+    hist = linreg.sgd(*_device(gpu, x1, x2, y), params, batch, epochs, 1e-4, 1e-6, seed=3, want_history=True).cpu().numpy()
+    np.testing.assert_allclose(hist, want_hist, rtol=1e-9)
+    np.testing.assert_allclose(params.cpu().numpy(), want_p, rtol=1e-9, atol=1e-10)
+
+
 def test_sgd_reference_hyperparameters_converge(gpu):
     # linear_regression_sgd.cu:23-28: 100 000 samples, batch 8192, 10 000 steps, lr 1e-4 -> 1e-6, noise 0.5
     import torch
