@@ -471,6 +471,29 @@ def test_tile_lists_equal_what_rectangles_and_depths_imply(gpu, oracle, G, W, H,
     ctx.close()
 
 
+@pytest.mark.parametrize("G,W,H", [
+    (63, 40, 24), (64, 40, 24), (65, 40, 24), (511, 16, 16), (2049, 90, 50),  # every tile against every Gaussian: chunk edges
+    (16384, 40, 33), (16385, 40, 33),  # the most Gaussians that are taken so, and the first number that goes by supertiles
+    (300, 1024, 512), (300, 1030, 512),  # 2048 tiles, and 2080
+    (9600, 720, 704), (13000, 720, 720),  # 297 000 tests, and 411 000
+])
+def test_tile_lists_on_both_sides_of_the_binning_rule(gpu, oracle, G, W, H):
+    import torch
+
+    from xyz_autodiff_cuda_amd import splat
+
+    params, depth = random_scene(G, W, H, seed=G + 5, scale_px=(0.5, 12.0))
+    depth[::3] = depth[1]
+    params[2:4, 2] = np.log(5000.0)  # one Gaussian over the whole image
+    p, d = torch.from_numpy(params).to(gpu), torch.from_numpy(depth).to(gpu)
+    # room for a tenth of the pairs: the first call enlarges the lists; the second takes the kept order
+    ctx = splat.SplatContext(W, H, G, pair_capacity_hint=max(8, G // 10))
+    for _ in range(2):
+        ctx.forward(p, d)
+        _assert_lists(ctx, oracle, W, H, params, depth)
+    ctx.close()
+
+
 @pytest.mark.parametrize("mode", ["static", "every_step"])
 def test_steps_that_do_not_wait(gpu, oracle, mode):
     """Without a loss read-back a step only queues work; results equal those of the default mode."""

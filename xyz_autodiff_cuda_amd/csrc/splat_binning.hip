@@ -507,6 +507,118 @@ int launch_scan(hipStream_t s, std::uint32_t* data, std::size_t n, const BinScra
 
 }  // namespace
 
+// ---------------------------------------------------------------------------
+// Small scenes in two launches.  The two levels above take seven, 3 to 10 us each however little there is to do.  Here a
+// block tests one tile against all Gaussians, 64 rectangles to a wavefront at a time and in depth order, and leaves
+// one bit per Gaussian and their count; a second launch adds up the counts of the tiles before its own, and the set
+// bits, in order, are the list.  (In one launch, with room for the lists taken from a counter: 28 us with 1080 tiles
+// and next to no Gaussians, for the atomics on one address.)
+// What bounds it: the tests, tiles x Gaussians of them, and the latency of a wavefront's chain of loads.
+// The rule (bins_by_tests) is where the two ways cross.  A forward call, us, two levels / so: 1000 Gaussians at
+// 640 x 427 43.6 / 21.4, 2000 at 720 x 700 45.5 / 25.5, 10 000 at 512 x 512 69.8 / 53.6, 12 000 at 640 x 640 (301 000
+// tests) 68.3 / 58.2, 16 384 at 512 x 288 99.9 / 90.1, 16 000 at 128 x 128 119 / 102; but 20 000 at 512 x 512
+// (321 000) 91.0 / 89.3, 20 000 at 768 x 768 (721 000) 75.8 / 88.0, 60 000 at 256 x 256, where a wavefront's chain of
+// chunks is long, 108 / 148, and 10 000 at 1024 x 1024 (4096 tiles) 61.9 / 67.6.
+constexpr int kTestWaves = 4;
+
+__device__ __forceinline__ std::uint32_t sum_over_block(std::uint32_t v, std::uint32_t (&per_wave)[kTestWaves]) {
+    for (int step = 32; step > 0; step /= 2) v += __shfl_xor(v, step, 64);
+    if ((threadIdx.x & 63) == 0) per_wave[threadIdx.x >> 6] = v;
+    __syncthreads();
+    std::uint32_t total = 0;
+#pragma unroll
+    for (int w = 0; w < kTestWaves; ++w) total += per_wave[w];
+    return total;
+}
+
+__global__ void __launch_bounds__(64 * kTestWaves) test_tiles_kernel(BinPlan p, const TileRect* __restrict__ rects_by_depth,
+                                                                     std::uint64_t* __restrict__ covering,
+                                                                     std::uint32_t* __restrict__ counts) {
+    __shared__ std::uint32_t per_wave[kTestWaves];
+    const int wave = static_cast<int>(threadIdx.x) >> 6, lane = static_cast<int>(threadIdx.x) & 63;
+    const int tile = static_cast<int>(blockIdx.x), tx = tile % p.tiles_x, ty = tile / p.tiles_x;
+    const int chunks = (p.G + 63) / 64;
+    std::uint64_t* mine = covering + static_cast<std::size_t>(tile) * chunks;
+    constexpr int kAhead = 8;  // loads in flight
+    std::uint32_t count = 0;   // of this lane's Gaussians
+    for (int c0 = wave * kAhead; c0 < chunks; c0 += kTestWaves * kAhead) {
+        TileRect r[kAhead];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            const int i = (c0 + k) * 64 + lane;
+            r[k] = TileRect{1, 1, 0, 0};  // covers nothing
+            if (i < p.G) r[k] = rects_by_depth[i];
+        }
+        std::uint64_t answer = 0;
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            const bool covers = tx >= r[k].x0 && tx <= r[k].x1 && ty >= r[k].y0 && ty <= r[k].y1;
+            const std::uint64_t mask = ballot(covers);
+            count += covers ? 1u : 0u;
+            if (lane == k) answer = mask;
+        }
+        if (lane < kAhead && c0 + lane < chunks) mine[c0 + lane] = answer;
+    }
+    const std::uint32_t total = sum_over_block(count, per_wave);
+    if (threadIdx.x == 0) counts[tile] = total;
+}
+
+__global__ void __launch_bounds__(64 * kTestWaves) write_lists_kernel(
+    BinPlan p, const std::uint32_t* __restrict__ by_depth, const std::uint64_t* __restrict__ covering,
+    const std::uint32_t* __restrict__ counts, std::uint32_t* __restrict__ list, std::uint32_t* __restrict__ range_begin,
+    std::uint32_t* __restrict__ range_end, std::uint32_t* __restrict__ status, bool clear_depth_flag) {
+    __shared__ std::uint32_t per_wave[kTestWaves];
+    __shared__ std::uint32_t found[kTestWaves];
+    const int wave = static_cast<int>(threadIdx.x) >> 6, lane = static_cast<int>(threadIdx.x) & 63;
+    const int tile = static_cast<int>(blockIdx.x);
+    const int chunks = (p.G + 63) / 64, share = (chunks + kTestWaves - 1) / kTestWaves;
+    const int begin = wave * share, end = begin + share < chunks ? begin + share : chunks;
+    const std::uint64_t* mine = covering + static_cast<std::size_t>(tile) * chunks;
+
+    std::uint32_t before = 0, here = 0;
+    for (int t = static_cast<int>(threadIdx.x); t < tile; t += 64 * kTestWaves) before += counts[t];
+    for (int c = begin + lane; c < end; c += 64) here += static_cast<std::uint32_t>(__builtin_popcountll(mine[c]));
+    for (int step = 32; step > 0; step /= 2) here += __shfl_xor(here, step, 64);
+    if (lane == 0) found[wave] = here;
+    const std::uint32_t first = sum_over_block(before, per_wave);
+    std::uint32_t at = first;
+    for (int w = 0; w < wave; ++w) at += found[w];
+
+    for (int c = begin; c < end; c += 64) {
+        const std::uint64_t answers = c + lane < end ? mine[c + lane] : 0;
+        for (std::uint64_t todo = ballot(answers != 0); todo != 0; todo &= todo - 1) {
+            const int k = __builtin_ctzll(todo);
+            const std::uint64_t mask =
+                static_cast<std::uint64_t>(static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(answers >> 32), k))) << 32 |
+                static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(answers), k));
+            if ((mask >> lane) & 1) {
+                const std::uint32_t to = at + static_cast<std::uint32_t>(__builtin_popcountll(mask & ((std::uint64_t(1) << lane) - 1)));
+                if (to < p.capacity) list[to] = by_depth[(c + k) * 64 + lane];
+            }
+            at += static_cast<std::uint32_t>(__builtin_popcountll(mask));
+        }
+    }
+    if (threadIdx.x == 0) {
+        // a list that does not fit is cut short; the pair count stays exact
+        const std::uint32_t behind = first + counts[tile];
+        range_begin[tile] = first < p.capacity ? first : p.capacity;
+        range_end[tile] = behind < p.capacity ? behind : p.capacity;
+        if (blockIdx.x == gridDim.x - 1) {
+            const bool overflow = behind > p.capacity;
+            status[kStatusPairs] = behind;
+            status[kStatusSuperPairs] = 0;
+            status[kStatusOverflow] = overflow ? 1u : 0u;
+            if (overflow) atomicMax(status + kStatusOverflowSticky, behind);
+            if (clear_depth_flag) status[kStatusDepthChanged] = 0;
+        }
+    }
+}
+
+bool bins_by_tests(int G, int tiles) {
+    const long long chunks = (static_cast<long long>(G) + 63) / 64;
+    return tiles <= kBinTestTiles && chunks <= kBinTestChunks && chunks * tiles <= kBinTests;
+}
+
 int launch_binning(hipStream_t s, const BinPlan& p, const std::uint32_t* by_depth, const TileRect* rects_by_depth,
                    const TileRect* rects, BinScratch& scratch,
                    std::uint32_t* list, std::uint32_t* range_begin, std::uint32_t* range_end, std::uint32_t* status,
@@ -514,6 +626,15 @@ int launch_binning(hipStream_t s, const BinPlan& p, const std::uint32_t* by_dept
     XAD_REQUIRE(p.G > 0 && p.supers > 0 && p.ranges_a > 0 && p.capacity > 0, "splat binning: empty plan");
     XAD_REQUIRE(range_end == range_begin + static_cast<std::size_t>(p.tiles_x) * p.tiles_y,
                 "splat binning: the two halves of the tile ranges must be adjacent");
+    if (scratch.covering) {
+        const dim3 grid(static_cast<unsigned>(p.tiles_x) * static_cast<unsigned>(p.tiles_y)), block(64 * kTestWaves);
+        hipLaunchKernelGGL(test_tiles_kernel, grid, block, 0, s, p, rects_by_depth, scratch.covering, scratch.counts);
+        XAD_HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(write_lists_kernel, grid, block, 0, s, p, by_depth, scratch.covering, scratch.counts, list, range_begin,
+                           range_end, status, clear_depth_flag);
+        XAD_HIP_TRY(hipGetLastError());
+        return XAD_OK;
+    }
     const unsigned waves_a = static_cast<unsigned>(p.ranges_a) * static_cast<unsigned>(p.groups);
     hipLaunchKernelGGL(super_kernel<false>, dim3(waves_a), dim3(64), 0, s, p, by_depth, rects_by_depth, scratch.matrix_a,
                        scratch.list_a);

@@ -103,6 +103,10 @@ void carve_fixed(xad_splat_context* c, char* base, std::size_t* bytes) {
     c->record_grads = k.take<float>(G * kRecordGradStride);
     c->loss = k.take<double>(kLossWords);
     c->status = k.take<std::uint32_t>(kStatusWords);
+    if (bins_by_tests(c->G, c->tiles)) {
+        c->bin.covering = k.take<std::uint64_t>((G + 63) / 64 * static_cast<std::size_t>(c->tiles));
+        c->bin.counts = k.take<std::uint32_t>(static_cast<std::size_t>(c->tiles));
+    }
     c->bin.scan_control = k.take<std::uint32_t>(kScanControlWords);
     c->depth_sort_temp = k.take<char>(c->depth_sort_bytes ? c->depth_sort_bytes : 16);
     *bytes = k.used;

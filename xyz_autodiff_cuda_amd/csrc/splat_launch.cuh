@@ -47,10 +47,18 @@ struct BinScratch {
     std::uint32_t* list_a = nullptr;      // capacity: the supertiles' lists
     std::uint32_t* first_wave = nullptr;  // supers + 1
     std::uint64_t* scan_state = nullptr;  // bin_scan_state_words, zero before the first launch
+    // scenes that bins_by_tests accepts, null for others: a bit per (tile, Gaussian), tiles x ceil(G / 64) words; a count per tile
+    std::uint64_t* covering = nullptr;
+    std::uint32_t* counts = nullptr;
     std::uint32_t* scan_control = nullptr;  // kScanControlWords: tickets given out, blocks finished (both zero between launches), epoch (never zero)
 };
 // The buffers are sized by a plan with capacity_a = capacity; a plan with a smaller capacity_a (once the host
 // has seen how many supertile pairs a scene produces) uses less of them and launches fewer wavefronts.
+// Whether tiles and Gaussians are few enough for the lists to be made by testing every tile against every Gaussian, 64
+// Gaussians (a chunk) a test.
+constexpr int kBinTestTiles = 2048, kBinTestChunks = 256;
+constexpr long long kBinTests = 300'000;
+bool bins_by_tests(int G, int tiles);
 BinPlan make_bin_plan(int G, int tiles_x, int tiles_y, std::uint32_t capacity, std::uint32_t capacity_a);
 std::size_t bin_matrix_a_words(const BinPlan& p);
 std::size_t bin_matrix_b_words(const BinPlan& p);
