@@ -430,7 +430,7 @@ int xad_linreg_sgd_f64(size_t total, const double* x1, const double* x2, const d
                        uint64_t seed, double* loss_history, void* stream);
 /* xad_linreg_sgd_f64 for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  No
- * counterpart in the reference.  Same arguments, same kernels and same results
+ * counterpart in the reference.  Same arguments, same draws and same results
  * as xad_linreg_sgd_f64, with two differences:
  *   - the gradient sums of a step live in a 256-byte array that is part of the
  *     library's device image (one copy per device, held until the process ends)

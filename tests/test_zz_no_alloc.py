@@ -1,8 +1,8 @@
 """The allocation-free SGD entry point against the allocating one, through the C ABI.
 
 xad_linreg_sgd_f64_static keeps the gradient sums of a step in an array inside
-the library's device image instead of allocating them.  Both entry points run
-the same kernels on the same rows, so their results differ only by the order
+the library's device image instead of allocating them.  Both entry points take
+the same steps on the same rows, so their results differ only by the order
 of the fp64 sums inside a step (1e-16 relative per step; the iteration
 contracts): parameters and loss history must agree to 1e-9 relative, the bound
 the trajectory test of the allocating entry point uses against the CPU
