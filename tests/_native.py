@@ -90,6 +90,41 @@ def negligible_in_tile(fields, tiles, device=False):
     return out.astype(bool)
 
 
+def compositing_choice(fields, tiles):
+    """What the two compositing passes make of (record, tile) pairs, on the host (fields and tiles as above):
+    (needs care, is ill shaped, left out by the backward pass, left out by the forward pass of the upper and the lower half
+    (n, 2), largest alpha the loops compute in each half (n, 2))."""
+    fields = np.ascontiguousarray(fields, np.float32)
+    tiles = np.ascontiguousarray(tiles, np.float32)
+    n = fields.shape[0]
+    assert fields.shape == (n, 6) and tiles.shape == (n, 2)
+    flags, largest = np.zeros(n, np.int32), np.zeros((n, 2), np.float32)
+    fn = load().xad_test_compositing_choice
+    fn.argtypes = [ctypes.c_int] + [ctypes.c_void_p] * 4
+    assert fn(n, fields.ctypes.data, tiles.ctypes.data, flags.ctypes.data, largest.ctypes.data) == 0
+    return (flags & 1) != 0, (flags & 16) != 0, (flags & 2) != 0, np.stack([(flags & 4) != 0, (flags & 8) != 0], axis=1), largest
+
+
+def composited_alpha(fields, pixels):
+    """alpha of records (n, 6) at one pixel each (n, 2) as the compositing loops compute it, before the clamp; on the host."""
+    fields = np.ascontiguousarray(fields, np.float32)
+    pixels = np.ascontiguousarray(pixels, np.float32)
+    n = fields.shape[0]
+    assert fields.shape == (n, 6) and pixels.shape == (n, 2)
+    out = np.zeros(n, np.float32)
+    fn = load().xad_test_composited_alpha
+    fn.argtypes = [ctypes.c_int] + [ctypes.c_void_p] * 3
+    assert fn(n, fields.ctypes.data, pixels.ctypes.data, out.ctypes.data) == 0
+    return out
+
+
+def far_away():
+    """The x that the compositing loops give to a pixel no Gaussian is to reach."""
+    fn = load().xad_test_far_away
+    fn.restype = ctypes.c_float
+    return np.float32(fn())
+
+
 def parallel_accumulation(threads, block):
     out = np.zeros(3, np.float64)
     rc = load().xad_test_parallel_accumulation(ctypes.c_size_t(threads), ctypes.c_int(block), out.ctypes.data_as(ctypes.c_void_p))

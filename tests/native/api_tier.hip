@@ -169,7 +169,7 @@ bool ok(hipError_t e) { return e == hipSuccess; }
 // The test that leaves a list entry out of a tile's compositing (csrc/splat_staged.cuh), on n (record, tile)
 // pairs; fields: n x 6 floats (centre x, y; inverse covariance a, b, c; alpha0), tiles: n x 2 floats (the
 // tile's first pixel).
-XAD_HD int negligible_pair(const float* fields, const float* tiles, int i) {
+XAD_HD xad_splat::Staged staged_record(const float* fields, int i) {
     xad_splat::Record record{};
     record.cx = fields[6 * i];
     record.cy = fields[6 * i + 1];
@@ -177,8 +177,18 @@ XAD_HD int negligible_pair(const float* fields, const float* tiles, int i) {
     record.b = fields[6 * i + 3];
     record.c = fields[6 * i + 4];
     record.alpha0 = fields[6 * i + 5];
-    const xad_splat::Staged staged = xad_splat::stage_record(&record, 0);
-    return xad_splat::negligible_in_tile(staged, tiles[2 * i], tiles[2 * i + 1]) ? 1 : 0;
+    return xad_splat::stage_record(&record, 0);
+}
+
+XAD_HD int negligible_pair(const float* fields, const float* tiles, int i) {
+    return xad_splat::negligible_in_tile(staged_record(fields, i), tiles[2 * i], tiles[2 * i + 1]) ? 1 : 0;
+}
+
+// alpha as the compositing loops compute it, before the clamp
+float composited_alpha(const xad_splat::Staged& r, float px, float py) {
+    const float dy = py - r.cy, dx = px - r.cx;
+    const float e = r.b2_s * dy, f = r.c_s * dy * dy;
+    return xyz_autodiff::math::fp32::exp2_raw(::fmaf(::fmaf(r.a_s, dx, e), dx, f)) * r.alpha0;
 }
 
 __global__ void negligible_kernel(int n, const float* fields, const float* tiles, int* out) {
@@ -236,6 +246,36 @@ extern "C" int xad_test_negligible_in_tile(int side, int n, const float* fields,
     (void)hipFree(d_out);
     return rc;
 }
+
+// Host.  What the two compositing passes make of n (record, tile) pairs.  flags, n ints: 1 the entry needs care, 2 the
+// backward pass leaves it out, 4 and 8 the forward pass leaves it out of the upper and the lower half of the tile, 16 it
+// is ill shaped.
+// largest: n x 2 floats, the largest alpha that the loops compute at a pixel of each half.
+extern "C" int xad_test_compositing_choice(int n, const float* fields, const float* tiles, int* flags, float* largest) {
+    constexpr int kHigh = xad_splat::kTile / 2;
+    for (int i = 0; i < n; ++i) {
+        const xad_splat::Staged r = staged_record(fields, i);
+        const float left = tiles[2 * i], top = tiles[2 * i + 1];
+        flags[i] = (xad_splat::needs_care(r) ? 1 : 0) | (xad_splat::ill_shaped(r) ? 16 : 0) | (xad_splat::negligible_in_tile(r, left, top) ? 2 : 0);
+        for (int half = 0; half < 2; ++half) {
+            if (xad_splat::negligible_in_part(r, left, top, top + half * kHigh, kHigh)) flags[i] |= 4 << half;
+            float best = 0.f;
+            for (int y = 0; y < kHigh; ++y)
+                for (int x = 0; x < xad_splat::kTile; ++x)
+                    best = ::fmaxf(best, composited_alpha(r, left + x, top + half * kHigh + y));
+            largest[2 * i + half] = best;
+        }
+    }
+    return 0;
+}
+
+// Host.  alpha of n records at one pixel each (n x 2 floats) as the compositing loops compute it, unclamped.
+extern "C" int xad_test_composited_alpha(int n, const float* fields, const float* pixels, float* alpha) {
+    for (int i = 0; i < n; ++i) alpha[i] = composited_alpha(staged_record(fields, i), pixels[2 * i], pixels[2 * i + 1]);
+    return 0;
+}
+
+extern "C" float xad_test_far_away(void) { return xad_splat::kFarAway; }
 
 extern "C" int xad_test_run_case_host(int id, double* out) { return xad_test::run_case(id, out); }
 

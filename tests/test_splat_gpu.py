@@ -117,6 +117,42 @@ def test_compositing_at_the_edges_of_pairs_chunks_and_halves(gpu, oracle, G, W, 
     _check_against_oracle(oracle, _gpu_step(gpu, W, H, params, depth, target), W, H, params, depth, target)
 
 
+@pytest.mark.parametrize("W,H,needles,short_px,long_px,seed", [
+    (1040, 1040, 300, 0.01, 60.0, 31), (1040, 1040, 100, 0.05, 400.0, 32),  # one walk per tile
+    (500, 510, 600, 0.01, 60.0, 32), (500, 510, 100, 0.02, 200.0, 32),      # a walk in pieces
+    (1040, 1040, 0, 1.0, 1.0, 33),
+])
+def test_gradients_use_the_weights_of_the_image(gpu, W, H, needles, short_px, long_px, seed):
+    """With d loss / d pixel = 1 everywhere a colour gradient is the sum of the weights that the Gaussian has in the image,
+    and these are what is seen when it alone is white (three at a time, one per channel).  Among ordinary Gaussians long thin
+    ones, whose inverse covariance is at the limit of fp32: both passes have to see the same of them, however little that
+    has to do with the ellipse.  1e-4: a few hundred fp32 roundings (6e-8 each) of the transmittance and the sum; 2e-5 is seen."""
+    import torch
+
+    from xyz_autodiff_cuda_amd import splat
+
+    G = 900
+    params, depth = random_scene(G, W, H, seed=seed, scale_px=(2.0, 12.0))
+    r = np.random.default_rng(seed + 1)
+    params[2, :needles] = r.uniform(np.log(short_px / 3), np.log(short_px), needles)
+    params[3, :needles] = r.uniform(np.log(long_px / 3), np.log(long_px), needles)
+    p, d = torch.from_numpy(params).to(gpu), torch.from_numpy(depth).to(gpu)
+    ctx = splat.SplatContext(W, H, G, depth_mode="static")
+    image = ctx.forward(p, d)
+    grads = ctx.step(p, d, image - 0.5)[1][5:8].double().cpu().numpy()
+    one = p.clone()
+    want = np.zeros(G)
+    for g in range(0, G, 3):
+        one[5:8] = 0.0
+        for k in range(3):
+            one[5 + k, g + k] = 1.0
+        want[g:g + 3] = ctx.forward(one, d).double().sum(dim=(0, 1)).cpu().numpy()
+    ctx.close()
+    assert (want > 1.0).sum() > 50
+    error = (np.abs(grads - want) / (want + 1e-2)).max()
+    assert error < 1e-4, error
+
+
 def test_more_than_65536_tiles(gpu, oracle):
     """256 x 257 tiles: the pair keys (tile indices) take the 32-bit path.  Small Gaussians keep
     the oracle fast."""

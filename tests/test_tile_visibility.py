@@ -1,10 +1,12 @@
-"""The test by which both compositing kernels leave a list entry out of a tile (negligible_in_tile,
-csrc/splat_staged.cuh) against brute force over the tile's 256 pixel centres, on the host build of the same
-code and, on the GPU, the device build against the host's.
+"""The tests by which the compositing kernels leave a list entry out (csrc/splat_staged.cuh): of a tile in the
+backward pass (negligible_in_tile), of half a tile in the forward pass (negligible_in_part), and which entries take
+their general path (needs_care).  Against brute force over the pixel centres, on the host build of the same code and,
+on the GPU, the device build of the first against the host's.
 
 What must hold: an entry that is left out reaches no pixel of the tile with alpha >= 1e-8 (the criterion is a
 lower bound of q over the pixels' bounding box, so it may keep entries it could have dropped, never the
-reverse); and it is worth having: nearly every entry that is far below the threshold at every pixel is found.
+reverse); it is worth having: nearly every entry that is far below the threshold at every pixel is found; and the two
+passes leave out the same, up to entries that change no pixel.
 """
 import numpy as np
 import pytest
@@ -91,6 +93,78 @@ def test_fraction_of_the_large_benchmark_scene():
     fields = np.stack([cx, cy, a, b, cc, alpha0], axis=1).astype(np.float32)[g]
     fraction = _native.negligible_in_tile(fields, tiles).mean()
     assert 0.17 < fraction < 0.27, fraction
+
+
+def _needles(n, seed, short_px, long_px):
+    """Long thin Gaussians, each paired with a tile that its ridge passes through or close by."""
+    r = np.random.default_rng(seed)
+    sx, sy = np.exp(r.uniform(np.log(short_px / 3), np.log(short_px), n)), np.exp(r.uniform(np.log(long_px / 3), np.log(long_px), n))
+    theta = r.uniform(-np.pi, np.pi, n)
+    tiles = (np.floor(r.uniform(0, 64, (n, 2))) * 16).astype(np.float32)
+    c, s = np.cos(theta), np.sin(theta)
+    along = r.uniform(-3, 3, n) * sy
+    cx = tiles[:, 0] + r.uniform(-2, 17, n) + along * s
+    cy = tiles[:, 1] + r.uniform(-2, 17, n) - along * c
+    a, b, cc = c * c / sx**2 + s * s / sy**2, c * s * (1 / sx**2 - 1 / sy**2), s * s / sx**2 + c * c / sy**2
+    alpha0 = 1 / (1 + np.exp(-r.standard_normal(n)))
+    return np.stack([cx, cy, a, b, cc, alpha0], axis=1).astype(np.float32), tiles
+
+
+@pytest.mark.parametrize("short_px,long_px", [(20, 40), (0.5, 40), (0.5, 300), (0.3, 1000), (0.5, 10000), (0.3, 3000), (0.1, 1000), (0.02, 200)])
+def test_both_passes_leave_out_the_same(short_px, long_px):
+    fields, tiles = _needles(200_000, 11, short_px, long_px)
+    careful, ill, backward_out, forward_out, largest = _native.compositing_choice(fields, tiles)
+    assert careful[ill].all()
+    # ill shaped entries: one answer, the tile's, whatever rounding has made of q
+    assert (forward_out[ill] == backward_out[ill, None]).all()
+    # others: what one pass takes and the other does not has an alpha below 1e-8^(1/1.44) at every pixel of that half
+    differ = forward_out != backward_out[:, None]
+    assert not differ.any() or largest[differ].max() < 3e-6, largest[differ].max()
+    # and the halves are worth having: of what is far below the threshold in a half most is left out of it (ridges of less
+    # than a third of a pixel pass between pixel centres, which a minimum over the pixels' box cannot know)
+    clearly = (largest < THRESHOLD * 1e-3) & ~ill[:, None]
+    if clearly.sum() > 1000 and short_px >= 0.3:
+        assert forward_out[clearly].mean() > 0.9, forward_out[clearly].mean()
+
+
+def test_entries_without_care_at_the_limits():
+    """Just inside the limits of needs_care(): alpha stays below the clamp wherever q cancels most, and is exactly 0 at
+    the place of a pixel that no Gaussian is to reach, in every row of the tallest image."""
+    r = np.random.default_rng(12)
+    n = 400_000
+    a, c = (np.exp(r.uniform(np.log(1e-9), np.log(1e9), n)) for _ in range(2))
+    a[: n // 4], c[: n // 8], c[n // 8 : n // 4] = 1.0001e-9, 0.9999e9, 1.0001e-9
+    a[n // 4 : n // 3] = 0.9999e9
+    b = np.sqrt(a * c * (1 - 1e-5 * (1 + np.exp(r.uniform(np.log(1e-3), np.log(1e4), n))))) * r.choice([-1.0, 1.0], n)
+    pixel = np.stack([np.floor(r.uniform(0, 524272, n)), np.floor(r.uniform(0, 524272, n))], axis=1)
+    # centres at all distances, the pixel on the ridge as seen along x: dx = -(b / a) dy, or along y
+    reach = np.exp(r.uniform(np.log(1e-2), np.log(4e5), n)) * r.choice([-1.0, 1.0], n)
+    steep = r.uniform(size=n) < 0.5
+    dx, dy = np.where(steep, -b / a * reach, reach), np.where(steep, reach, -b / c * reach)
+    cx, cy = np.clip(pixel[:, 0] - dx, -1e6, 1e6), np.clip(pixel[:, 1] - dy, -5e5, 5e5)
+    fields = np.stack([cx, cy, a, b, c, np.full(n, 0.98)], axis=1).astype(np.float32)
+    fields[:, 5] = np.minimum(fields[:, 5], np.float32(0.98))
+    careful = _native.compositing_choice(fields, np.zeros((n, 2), np.float32))[0]
+    assert 0.01 < careful.mean() < 0.5
+    fields, pixel = fields[~careful], pixel[~careful].astype(np.float32)
+    alpha = _native.composited_alpha(fields, pixel)
+    assert (alpha > 0.5).sum() > 1000  # the ridge is met
+    assert alpha.max() <= 0.98 * (1 + 1e-6)
+    pixel[:, 0] = _native.far_away()
+    assert (_native.composited_alpha(fields, pixel) == 0).all()
+    pixel[:, 1] = np.where(fields[:, 4] > 0, 524271.0, 0.0)
+    assert (_native.composited_alpha(fields, pixel) == 0).all()
+
+
+@pytest.mark.parametrize("field,value", [
+    (5, 0.9801), (5, np.nan), (2, 0.9e-9), (2, 1.1e9), (2, -1.0), (2, np.nan), (4, 0.9e-9), (4, 1.1e9), (4, -1.0), (3, 0.999999), (3, np.nan),
+    (0, 1.1e6), (0, -1.1e6), (0, np.inf), (1, 5.1e5), (1, -5.1e5), (1, np.nan),
+])
+def test_entries_beyond_a_limit_need_care(field, value):
+    fields = np.array([[5.0, 6.0, 1.0, 0.2, 1.0, 0.5]] * 2, np.float32)
+    fields[1, field] = value
+    careful = _native.compositing_choice(fields, np.zeros((2, 2), np.float32))[0]
+    assert not careful[0] and careful[1]
 
 
 @pytest.mark.gpu

@@ -294,7 +294,8 @@ __global__ void __launch_bounds__(kChunk) render_forward_kernel(
         if (base + lane < last) {
             const Staged mine = stage_record(records, sorted_ids[base + lane]);
             staged[lane] = mine;
-            visible = !negligible_in_rectangle<kTile, kForwardHigh>(mine, static_cast<float>(part_x), static_cast<float>(part_y));
+            visible = !negligible_in_part(mine, static_cast<float>(part_x), static_cast<float>(part_y - part * kForwardHigh),
+                                          static_cast<float>(part_y), kForwardHigh);
             careful = needs_care(mine);
         }
         __syncthreads();
@@ -598,7 +599,7 @@ __global__ void __launch_bounds__(kChunk) render_backward_kernel(
     // reach (kFarAway), so that alpha and with it everything it would add comes out as 0 by itself.
     float px[kLanePixels];
 #pragma unroll
-    for (int p = 0; p < kLanePixels; ++p) px[p] = used[p] >= walk_last ? px0 + static_cast<float>(p) : kFarAway;
+    for (int p = 0; p < kLanePixels; ++p) px[p] = kFarAway;
     // which of the eighteen row sums this lane parks, and which ninth value if any
     float* const park_scattered = &parked[reduced_entry(lane)][lane >> 4][reduced_index(lane)];
     float* const park_ninth = &parked[(lane >> 2) & 1][lane >> 4][8];
@@ -622,15 +623,21 @@ __global__ void __launch_bounds__(kChunk) render_backward_kernel(
             staged_id[lane] = id;
             const Staged mine = stage_record(records, id);
             staged[lane] = mine;
-            visible = !negligible_in_tile(mine, tile_x, tile_y);  // what the forward pass left out and what reaches its other half
+            visible = !negligible_in_tile(mine, tile_x, tile_y);  // all that the forward pass took for either half, see negligible_in_part()
             careful = needs_care(mine);
         }
         __syncthreads();
-        // the entries of this chunk at which a pixel wakes up: the last one it composited
+        // A pixel that composited the whole chunk is awake from its start on, whatever chunks behind it held; the others wake
+        // up at an entry of this chunk, the last one they composited, if not in front of it.
+        const std::uint32_t chunk_last = chunk_first + static_cast<std::uint32_t>(count);
 #pragma unroll
         for (int p = 0; p < kLanePixels; ++p) {
-            const std::uint32_t entry = used[p] - 1 - chunk_first;  // of a pixel that composited nothing: far beyond
-            if (used[p] < walk_last && entry < static_cast<std::uint32_t>(kChunk)) atomicOr(&wakes[entry >> 5], 1u << (entry & 31));
+            if (used[p] >= chunk_last) {
+                px[p] = px0 + static_cast<float>(p);
+            } else {
+                const std::uint32_t entry = used[p] - 1 - chunk_first;  // of a pixel that composited nothing: far beyond
+                if (entry < static_cast<std::uint32_t>(kChunk)) atomicOr(&wakes[entry >> 5], 1u << (entry & 31));
+            }
         }
         __syncthreads();
         std::uint64_t waking = static_cast<std::uint64_t>(__builtin_amdgcn_readfirstlane(wakes[1])) << 32 |

@@ -1,7 +1,8 @@
 #pragma once
-// A Gaussian's record as the compositing kernels stage it in LDS, and the test that leaves an entry
-// of a tile's list out of both compositing passes.  In a header of its own, and callable on the host
-// as well, so that the test can be checked against brute force over a tile's pixels without a GPU.
+// A Gaussian's record as the compositing kernels stage it in LDS, the tests that leave an entry of a
+// tile's list out of the compositing passes, and the one that sends an entry to their general path.  In
+// a header of its own, and callable on the host as well, so that the tests can be checked against brute
+// force over a tile's pixels without a GPU.
 #include <cstdint>
 
 #include <xyz_autodiff/detail/config.cuh>
@@ -47,15 +48,16 @@ XAD_INLINE Staged stage_record(const Record* __restrict__ records, std::uint32_t
 // an entry is recognised when its record is staged: the minimum of q over the tile's pixel centres
 // is bounded from below by the minimum over their bounding box, which for a convex quadratic whose
 // centre lies outside the box is attained on one of the four edges.  If even there alpha stays below
-// kNegligibleAlpha, the entry is left out of the compositing loops of this tile, forward and backward
-// alike: it would change a pixel by less than 1e-8 (an fp32 ulp of 0.5 is 6e-8).  Lists and pair
-// counts are not affected.  Comparisons with NaN are false, so an odd record is kept.
+// kNegligibleAlpha, the entry is left out of the compositing loop: it would change a pixel by less than
+// 1e-8 (an fp32 ulp of 0.5 is 6e-8).  The backward pass asks about a whole tile, the forward pass about
+// the half that a wavefront walks (see negligible_in_part() for what keeps the two together).  Lists and
+// pair counts are not affected.  Comparisons with NaN are false, so an odd record is kept.
 constexpr float kNegligibleAlpha = 1e-8f;
 
-template <int kWide, int kHigh>
-XAD_INLINE bool negligible_in_rectangle(const Staged& s, float left, float top) {
-    const float x0 = left - s.cx, x1 = x0 + static_cast<float>(kWide - 1);
-    const float y0 = top - s.cy, y1 = y0 + static_cast<float>(kHigh - 1);
+// over the pixels from (left, top) on, kTile of them across and `high` down
+XAD_INLINE bool negligible_in_rectangle(const Staged& s, float left, float top, int high) {
+    const float x0 = left - s.cx, x1 = x0 + static_cast<float>(kTile - 1);
+    const float y0 = top - s.cy, y1 = y0 + static_cast<float>(high - 1);
     float q_min = 0.f;
     if (!(x0 <= 0.f && x1 >= 0.f && y0 <= 0.f && y1 >= 0.f)) {
         const float x_of_y = -s.b / s.a, y_of_x = -s.b / s.c;  // where q is least along a line
@@ -73,7 +75,7 @@ XAD_INLINE bool negligible_in_rectangle(const Staged& s, float left, float top) 
 }
 
 XAD_INLINE bool negligible_in_tile(const Staged& s, float tile_x, float tile_y) {
-    return negligible_in_rectangle<kTile, kTile>(s, tile_x, tile_y);
+    return negligible_in_rectangle(s, tile_x, tile_y, kTile);
 }
 
 // Entries for which the compositing loops have to make sure of two things themselves.  For all others
@@ -85,10 +87,23 @@ XAD_INLINE bool negligible_in_tile(const Staged& s, float tile_x, float tile_y) 
 // Comparisons with NaN are false, so an odd record is taken with care.
 constexpr float kFarAway = 1e18f;
 
-XAD_INLINE bool needs_care(const Staged& s) {
+XAD_INLINE bool ill_shaped(const Staged& s) {
     const float ac = s.a * s.c;
-    return !(s.alpha0 <= 0.98f && s.a >= 1e-9f && s.a <= 1e9f && s.c >= 1e-9f && s.c <= 1e9f && ac - s.b * s.b >= 1e-5f * ac &&
-             s.cx >= -1e6f && s.cx <= 1e6f && s.cy >= -5e5f && s.cy <= 5e5f);
+    return !(s.a >= 1e-9f && s.a <= 1e9f && s.c >= 1e-9f && s.c <= 1e9f && ac - s.b * s.b >= 1e-5f * ac && s.cx >= -1e6f &&
+             s.cx <= 1e6f && s.cy >= -5e5f && s.cy <= 5e5f);
+}
+XAD_INLINE bool needs_care(const Staged& s) { return !(s.alpha0 <= 0.98f) || ill_shaped(s); }
+
+// What the forward walk of one part of a tile (`high` rows from part_y on) leaves out.  The backward walk takes whole tiles
+// and leaves out what negligible_in_tile() says, and the two must not disagree about an entry that changes a pixel: one that
+// only the forward pass composited stays in the transmittance that the backward pass starts from, for every entry in front
+// of it.  For an entry of good shape they cannot: the rounding of q is at most 1e-6 (a dx^2 + c dy^2), a fifth of q, so one
+// that either test leaves out has an alpha below 1e-8^(1/1.44) = 3e-6 at every pixel in question.  Of long thin Gaussians q
+// can cancel to nothing but rounding (0.3 x 3000 pixels: one in 2000 near pairs came out up to 0.99 in one test only);
+// about those both passes ask for the tile, and get the same answer.
+XAD_INLINE bool negligible_in_part(const Staged& s, float tile_x, float tile_y, float part_y, int high) {
+    const bool whole = ill_shaped(s);
+    return negligible_in_rectangle(s, tile_x, whole ? tile_y : part_y, whole ? kTile : high);
 }
 
 }  // namespace xad_splat
