@@ -125,6 +125,14 @@ def far_away():
     return np.float32(fn())
 
 
+def sgd_launches(epochs, per_launch):
+    """Steps that the launches of an SGD call take in all; negative if they are not the steps 0 .. epochs - 1, each gathered
+    by the launch before."""
+    fn = load().xad_test_sgd_launches
+    fn.restype = ctypes.c_int64
+    return fn(ctypes.c_int(epochs), ctypes.c_int(per_launch))
+
+
 def parallel_accumulation(threads, block):
     out = np.zeros(3, np.float64)
     rc = load().xad_test_parallel_accumulation(ctypes.c_size_t(threads), ctypes.c_int(block), out.ctypes.data_as(ctypes.c_void_p))

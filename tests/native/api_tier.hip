@@ -12,6 +12,7 @@
 #include <xyz_autodiff/util/hip_managed_ptr.cuh>
 #include "tester_suite.cuh"
 #include "concept_checks.cuh"
+#include "../../xyz_autodiff_cuda_amd/csrc/linreg_launches.cuh"
 #include "../../xyz_autodiff_cuda_amd/csrc/splat_staged.cuh"
 
 using namespace xyz_autodiff;
@@ -276,6 +277,24 @@ extern "C" int xad_test_composited_alpha(int n, const float* fields, const float
 }
 
 extern "C" float xad_test_far_away(void) { return xad_splat::kFarAway; }
+
+// Host.  Follows the launches of an SGD call.  Returns the steps taken in all, or -1 - k where launch k takes other steps
+// than the ones after those before it, or other ones than were gathered for it, or more than fit.
+extern "C" std::int64_t xad_test_sgd_launches(int epochs, int per_launch) {
+    std::int64_t taken = 0, gathered_from = 0;
+    int gathered = 0;
+    const std::int64_t launches = xad_linreg::step_launches(epochs, per_launch);
+    for (std::int64_t k = -1; k < launches; ++k) {
+        const xad_linreg::StepLaunch l = xad_linreg::step_launch(k, epochs, per_launch);
+        const bool right = l.steps == gathered && (l.steps == 0 || (l.first == taken && l.first == gathered_from)) &&
+                           l.steps >= 0 && l.steps <= per_launch && l.gather >= 0 && l.gather <= per_launch;
+        if (!right) return -1 - k;
+        taken += l.steps;
+        gathered = l.gather;
+        gathered_from = l.coming;
+    }
+    return gathered == 0 ? taken : -1 - launches;
+}
 
 extern "C" int xad_test_run_case_host(int id, double* out) { return xad_test::run_case(id, out); }
 

@@ -148,3 +148,11 @@ def test_gradient_matches_reverse_mode_autodiff(oracle):
         out = oracle.linreg_gradient(x1, x2, y, params)
         np.testing.assert_allclose(out[:4], p.grad.numpy(), rtol=1e-11)
         np.testing.assert_allclose(out[4], float(loss.detach()), rtol=1e-12)
+
+
+@pytest.mark.parametrize("per_launch", [21, 64])  # steps of 8192 samples in 4 MiB, and the most
+@pytest.mark.parametrize("epochs", [1, 20, 21, 22, 63, 64, 65, 128, 129, 10_000, 2**31 - 64, 2**31 - 1])
+def test_sgd_launches_take_every_step_once(epochs, per_launch):
+    from tests import _native
+
+    assert _native.sgd_launches(epochs, min(per_launch, epochs)) == epochs

@@ -10,6 +10,7 @@
 
 #include "common.cuh"
 #include "linreg.cuh"
+#include "linreg_launches.cuh"
 #include "rng.cuh"
 
 namespace {
@@ -318,25 +319,24 @@ int queue_serial_sgd(hipStream_t s, double* gathered, int per_launch, std::size_
                      double* loss_history) {
     const double decay = std::log(lr_last / lr_first) / epochs;
     const std::size_t half = static_cast<std::size_t>(per_launch) * 3 * static_cast<std::size_t>(batch);
-    const int launches = (epochs + per_launch - 1) / per_launch;
+    const std::int64_t launches = xad_linreg::step_launches(epochs, per_launch);
     // launch k gathers for the steps of launch k + 1; the first one does nothing else
-    for (int k = -1; k < launches; ++k) {
+    for (std::int64_t k = -1; k < launches; ++k) {
+        const xad_linreg::StepLaunch l = xad_linreg::step_launch(k, epochs, per_launch);
         SerialSteps a{};
         a.x1 = x1, a.x2 = x2, a.y = y;
         a.total = total, a.key = xad_rng::stream_key(seed, 0);
         a.params = params, a.batch = batch;
-        const int first = k * per_launch;
-        if (k >= 0) {
+        a.steps = l.steps;
+        if (l.steps > 0) {
             a.samples = gathered + static_cast<std::size_t>(k & 1) * half;
-            a.steps = epochs - first < per_launch ? epochs - first : per_launch;
-            a.history = loss_history ? loss_history + first : nullptr;
-            for (int e = 0; e < a.steps; ++e) a.rates[e] = lr_first * std::exp(decay * (first + e));
+            a.history = loss_history ? loss_history + l.first : nullptr;
+            for (int e = 0; e < l.steps; ++e) a.rates[e] = lr_first * std::exp(decay * static_cast<double>(l.first + e));
         }
-        const int coming = first + per_launch, left = epochs - coming;
-        if (left > 0) {
+        if (l.gather > 0) {
             a.gathered = gathered + static_cast<std::size_t>((k + 1) & 1) * half;
-            a.first_draw = static_cast<std::uint64_t>(coming) * static_cast<std::uint64_t>(batch);
-            a.gather = static_cast<std::uint32_t>(left < per_launch ? left : per_launch) * static_cast<std::uint32_t>(batch);
+            a.first_draw = static_cast<std::uint64_t>(l.coming) * static_cast<std::uint64_t>(batch);
+            a.gather = static_cast<std::uint32_t>(l.gather) * static_cast<std::uint32_t>(batch);
         }
         const unsigned gatherers = (a.gather + kStepLanes - 1) / kStepLanes;
         const dim3 grid(1 + (gatherers < 255 ? gatherers : 255)), block(kStepLanes);
