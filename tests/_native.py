@@ -133,6 +133,11 @@ def sgd_launches(epochs, per_launch):
     return fn(ctypes.c_int(epochs), ctypes.c_int(per_launch))
 
 
+def sgd_one_block(batch, epochs):
+    """Whether one block takes the steps of an SGD call, or two launches each of them."""
+    return bool(load().xad_test_sgd_one_block(ctypes.c_int(batch), ctypes.c_int(epochs)))
+
+
 def parallel_accumulation(threads, block):
     out = np.zeros(3, np.float64)
     rc = load().xad_test_parallel_accumulation(ctypes.c_size_t(threads), ctypes.c_int(block), out.ctypes.data_as(ctypes.c_void_p))

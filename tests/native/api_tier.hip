@@ -296,6 +296,8 @@ extern "C" std::int64_t xad_test_sgd_launches(int epochs, int per_launch) {
     return gathered == 0 ? taken : -1 - launches;
 }
 
+extern "C" int xad_test_sgd_one_block(int batch, int epochs) { return xad_linreg::one_block_takes(batch, epochs) ? 1 : 0; }
+
 extern "C" int xad_test_run_case_host(int id, double* out) { return xad_test::run_case(id, out); }
 
 extern "C" int xad_test_run_case_device(int id, double* out) {

@@ -134,6 +134,7 @@ def test_sgd_trajectory_matches_oracle(gpu, oracle, batch, epochs):
 @pytest.mark.parametrize("batch,epochs", [
     (1, 130), (63, 64), (1023, 65), (1024, 3), (1025, 64),  # one sample a lane and a few more; whole launches of steps and one more
     (2048, 1), (2049, 65), (4097, 43), (8192, 22), (8193, 5),  # the largest batch one block takes, and the first it does not
+    (2049, 1), (4096, 2), (4097, 2), (4097, 3), (8192, 2), (8192, 3),  # the shortest calls it takes the steps of, and the longest it does not
 ])
 def test_sgd_where_the_ways_of_taking_steps_meet(gpu, oracle, batch, epochs):
     import torch

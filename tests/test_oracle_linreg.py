@@ -156,3 +156,12 @@ def test_sgd_launches_take_every_step_once(epochs, per_launch):
     from tests import _native
 
     assert _native.sgd_launches(epochs, min(per_launch, epochs)) == epochs
+
+
+def test_sgd_rule_where_two_launches_a_step_are_faster():
+    from tests import _native
+
+    for batch, epochs in ((2049, 1), (4096, 1), (4097, 1), (4097, 2), (8192, 1), (8192, 2), (8193, 1), (8193, 10_000), (1, 0), (8192, 0)):
+        assert not _native.sgd_one_block(batch, epochs), (batch, epochs)
+    for batch, epochs in ((1, 1), (256, 1), (2048, 1), (2049, 2), (4096, 2), (4096, 2**31 - 1), (4097, 3), (8192, 3), (8192, 10_000)):
+        assert _native.sgd_one_block(batch, epochs), (batch, epochs)

@@ -138,9 +138,8 @@ __global__ void linreg_update_kernel(double* params, double* sums, double learni
 // unit gets from beyond its XCD's L2 (about 60 GB/s).
 // Measured (us per step, calls of 200 steps, two launches a step / so): batch 256 6.1 / 0.9, 1024 7.1 / 1.2, 2048
 // 6.7 / 1.6, 4096 7.3 / 2.3, 8192 6.8 / 4.0; 16 384 would be level (7.4).  Calls of 20 steps: 9.0 / 2.2 to 9.4 / 6.6.
-constexpr int kStepLanes = 1024;
+using xad_linreg::kStepLanes;
 constexpr int kStepsPerLaunch = 64;
-constexpr int kLargestSerialBatch = 8 * kStepLanes;           // eight samples per lane: what its registers hold
 constexpr std::size_t kGatheredBytes = std::size_t(4) << 20;  // of one launch's steps, at most (two such buffers)
 
 struct SerialSteps {
@@ -390,11 +389,11 @@ extern "C" int xad_linreg_sgd_f64(size_t total, const double* x1, const double* 
     XAD_REQUIRE(total > 0 && batch > 0 && epochs >= 0, "total, batch must be positive and epochs non-negative");
     XAD_REQUIRE(lr_first > 0.0 && lr_last > 0.0, "learning rates must be positive");
     hipStream_t s = xad::as_stream(stream);
-    // One block takes all steps where it can hold a batch and there is memory for the gathered samples; otherwise two
+    // One block takes all steps where that is the faster way and there is memory for the gathered samples; otherwise two
     // launches a step.
     double* scratch_memory = nullptr;
     int per_launch = 0;
-    if (batch <= kLargestSerialBatch && epochs > 0) {
+    if (xad_linreg::one_block_takes(batch, epochs)) {
         const std::size_t step_bytes = 3 * sizeof(double) * static_cast<std::size_t>(batch);
         const std::size_t fit = kGatheredBytes / step_bytes;
         per_launch = static_cast<int>(fit < kStepsPerLaunch ? fit : kStepsPerLaunch);

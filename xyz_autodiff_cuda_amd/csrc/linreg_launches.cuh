@@ -1,9 +1,22 @@
 #pragma once
-// How the SGD steps that one block takes are dealt to launches.  In a header of its own, so that it can be checked without
-// a GPU up to the largest number of steps a call may ask for (2^31 - 1: sums of steps do not fit an int).
+// Which SGD calls one block takes the steps of, and how these are dealt to launches.  In a header of its own, so that it
+// can be checked without a GPU up to the largest number of steps a call may ask for (2^31 - 1: sums of steps do not fit an
+// int).
 #include <cstdint>
 
 namespace xad_linreg {
+
+constexpr int kStepLanes = 1024;
+constexpr int kLargestSerialBatch = 8 * kStepLanes;  // eight samples per lane: what a block's registers hold
+
+// Whether one block takes the steps, or two launches each of them.  The block's call begins with a launch that only gathers
+// and ends with one that streams its samples through one compute unit, which a call of a step or two does not make up for
+// where a batch is large.  Measured (us per call of 1 / 2 / 3 / 4 steps, two launches a step | so): batch 256 24.5 29.2 36.1
+// 72.7 | 23.0 23.6 25.0 26.2, 2048 26.4 32.1 39.9 80.7 | 26.0 27.5 28.9 30.0, 4096 26.2 30.9 37.4 63.3 | 26.9 29.0 30.8 32.9,
+// 8192 26.2 31.9 39.9 79.2 | 30.0 34.0 37.6 41.1.
+inline bool one_block_takes(int batch, int epochs) {
+    return batch <= kLargestSerialBatch && epochs > (batch <= kLargestSerialBatch / 4 ? 0 : (batch <= kLargestSerialBatch / 2 ? 1 : 2));
+}
 
 // Launch k of 0 .. step_launches() - 1 takes the steps first .. first + steps - 1 and gathers the samples of the `gather`
 // steps from `coming` on, those of launch k + 1; launch -1 does nothing but gather.
