@@ -530,6 +530,23 @@ def test_tile_lists_on_both_sides_of_the_binning_rule(gpu, oracle, G, W, H):
     ctx.close()
 
 
+def test_small_scenes_keep_no_room_for_the_lists_of_supertiles(gpu):
+    """Room for 64 Mi pairs is 256 MiB of lists where they are made by testing every tile (the copy per supertile and its
+    counts would be twice that again); the enlargement of lists that were cut short works on the same terms."""
+    import torch
+
+    from xyz_autodiff_cuda_amd import splat
+
+    G, W, H = 1000, 640, 427
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info(gpu)[0]
+    ctx = splat.SplatContext(W, H, G, pair_capacity_hint=64 << 20)
+    taken = before - torch.cuda.mem_get_info(gpu)[0]
+    ctx.close()
+    fixed = 128 * W * H + 4096 * G  # the pixels' states of the split walk and little else
+    assert (256 << 20) <= taken <= (256 << 20) + 2 * fixed, taken
+
+
 @pytest.mark.parametrize("mode", ["static", "every_step"])
 def test_steps_that_do_not_wait(gpu, oracle, mode):
     """Without a loss read-back a step only queues work; results equal those of the default mode."""

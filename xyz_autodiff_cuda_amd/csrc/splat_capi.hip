@@ -115,6 +115,8 @@ void carve_fixed(xad_splat_context* c, char* base, std::size_t* bytes) {
 void carve_paired(xad_splat_context* c, char* base, std::size_t* bytes) {
     Carver k{base};
     c->list = k.take<std::uint32_t>(c->plan.capacity);
+    *bytes = k.used;
+    if (c->bin.covering) return;  // lists made by tests need nothing else of this size
     c->bin.list_a = k.take<std::uint32_t>(c->plan.capacity);
     c->bin.matrix_a = k.take<std::uint32_t>(bin_matrix_a_words(c->plan));
     c->bin.matrix_b = k.take<std::uint32_t>(bin_matrix_b_words(c->plan));
@@ -142,8 +144,8 @@ int size_pair_buffers(xad_splat_context* c, std::uint32_t capacity) {
     c->paired = base;
     carve_paired(c, static_cast<char*>(base), &bytes);
     // the scan's state words must not look like words of a coming epoch
-    XAD_HIP_TRY(hipMemset(c->bin.scan_state, 0, bin_scan_state_words(c->plan) * sizeof(std::uint64_t)));
-    XAD_HIP_TRY(hipDeviceSynchronize());  // the fill is not on the caller's stream
+    if (c->bin.scan_state) XAD_HIP_TRY(hipMemset(c->bin.scan_state, 0, bin_scan_state_words(c->plan) * sizeof(std::uint64_t)));
+    XAD_HIP_TRY(hipDeviceSynchronize());  // the fills (this one and that of the fixed buffers) are not on the caller's stream
     return XAD_OK;
 }
 
@@ -276,7 +278,8 @@ int bin(xad_splat_context* c, const float* params, const float* depth, hipStream
             c->capacity_seen = true;
             // from now on level A is given only the room this scene needs, with a margin: fewer wavefronts at level B
             // (an overflow of that margin is reported like any other and gives level A the whole buffer back)
-            c->plan = make_bin_plan(c->G, c->tiles_x, c->tiles_y, c->plan.capacity, level_a_share(c->report->status[kStatusSuperPairs]));
+            if (!c->bin.covering)
+                c->plan = make_bin_plan(c->G, c->tiles_x, c->tiles_y, c->plan.capacity, level_a_share(c->report->status[kStatusSuperPairs]));
         }
         // what this call's own attempts left in the sticky word is settled; what earlier calls left there stays
         if (made_room && c->report->status[kStatusStickyBefore] == 0) {

@@ -42,6 +42,7 @@ struct BinPlan {
 };
 constexpr int kScanControlWords = 3;
 struct BinScratch {
+    // null where covering is not
     std::uint32_t* matrix_a = nullptr;    // bin_matrix_a_words: counts, then offsets, per (supertile, range)
     std::uint32_t* matrix_b = nullptr;    // bin_matrix_b_words: the same per (tile, range of its supertile's list)
     std::uint32_t* list_a = nullptr;      // capacity: the supertiles' lists
@@ -52,13 +53,13 @@ struct BinScratch {
     std::uint32_t* counts = nullptr;
     std::uint32_t* scan_control = nullptr;  // kScanControlWords: tickets given out, blocks finished (both zero between launches), epoch (never zero)
 };
-// The buffers are sized by a plan with capacity_a = capacity; a plan with a smaller capacity_a (once the host
-// has seen how many supertile pairs a scene produces) uses less of them and launches fewer wavefronts.
 // Whether tiles and Gaussians are few enough for the lists to be made by testing every tile against every Gaussian, 64
 // Gaussians (a chunk) a test.
 constexpr int kBinTestTiles = 2048, kBinTestChunks = 256;
 constexpr long long kBinTests = 300'000;
 bool bins_by_tests(int G, int tiles);
+// The buffers are sized by a plan with capacity_a = capacity; a plan with a smaller capacity_a (once the host
+// has seen how many supertile pairs a scene produces) uses less of them and launches fewer wavefronts.
 BinPlan make_bin_plan(int G, int tiles_x, int tiles_y, std::uint32_t capacity, std::uint32_t capacity_a);
 std::size_t bin_matrix_a_words(const BinPlan& p);
 std::size_t bin_matrix_b_words(const BinPlan& p);
