@@ -103,8 +103,9 @@ def test_depth_ranks_follow_the_depths_of_each_call(gpu, oracle):
     (15, 16, 16), (16, 18, 16), (17, 16, 24), (33, 40, 40), (63, 16, 16), (64, 33, 7), (65, 16, 16), (130, 31, 33),
 ])
 def test_compositing_at_the_edges_of_pairs_chunks_and_halves(gpu, oracle, G, W, H, logit):
-    """Lists as long as a pair, a piece of the split walk or a chunk and one more or less, pixels that stop behind either
-    entry of a pair, and, every third Gaussian, one so wide (50 000 pixels) that a stopped pixel is within its reach."""
+    """Images of few tiles, whose walks are split: lists as long as a pair, a piece of the walk or the 64 records staged at a
+    time and one more or less, pixels that stop behind either entry of a pair, and, every third Gaussian, one so wide (50 000
+    pixels) that a stopped pixel is within its reach."""
     params, depth = random_scene(G, W, H, seed=100 + G, scale_px=(6.0, 14.0))
     if logit is None:
         # two clamped layers on one pixel would leave (1 - 0.99)^2, which is below the threshold in fp32 and not in fp64
@@ -115,6 +116,56 @@ def test_compositing_at_the_edges_of_pairs_chunks_and_halves(gpu, oracle, G, W, 
     params[2:4, ::3] = np.log(5e4)
     target = np.random.default_rng(G).uniform(0, 1, (H, W, 3)).astype(np.float32)
     _check_against_oracle(oracle, _gpu_step(gpu, W, H, params, depth, target), W, H, params, depth, target)
+
+
+def _stops(params, depth, rects, width, y0, y1):
+    """For the pixels of rows y0 to y1 - 1, in fp64: the place in the depth order (from 1) of the Gaussian behind which a
+    pixel stops, or their number, and how close any transmittance comes to the threshold, relative to it."""
+    order = np.argsort(depth, kind="stable")
+    p, r = params.astype(np.float64)[:, order], rects[order]
+    y, x = (a[..., None] for a in np.mgrid[y0:y1, 0:width])
+    c, s = np.cos(p[4]), np.sin(p[4])
+    u, v = (x - p[0]) * c + (y - p[1]) * s, (y - p[1]) * c - (x - p[0]) * s
+    alpha = np.minimum(0.99, np.exp(-0.5 * ((u * np.exp(-p[2])) ** 2 + (v * np.exp(-p[3])) ** 2)) / (1 + np.exp(-p[8])))
+    covered = (x // 16 >= r[:, 0]) & (y // 16 >= r[:, 1]) & (x // 16 <= r[:, 2]) & (y // 16 <= r[:, 3])
+    T = np.cumprod(1 - np.where(covered, alpha, 0), axis=-1)
+    return np.where(T[..., -1] < 1e-4, np.argmax(T < 1e-4, axis=-1) + 1, p.shape[1]), np.abs(T / 1e-4 - 1).min()
+
+
+@pytest.mark.parametrize("where", [0.5, 0.9, None])  # how far down the list pixels stop, about; None: not at all
+@pytest.mark.parametrize("G,W,H,y0", [
+    (63, 16, 65568, 32800), (64, 16, 65568, 32800), (65, 16, 65568, 32800),  # 4098 tiles: one walk per tile, 64 entries a chunk
+    (127, 16, 65568, 32800), (128, 16, 65568, 32800), (129, 16, 65568, 32800), (200, 16, 65568, 32800),
+    (511, 33, 20, 0), (512, 33, 20, 0), (513, 33, 20, 0),  # eight segments of a chunk each, and of a chunk and a quarter
+    (1023, 33, 20, 0), (1024, 33, 20, 0), (1025, 33, 20, 0), (1100, 33, 20, 0),
+])
+def test_compositing_where_walks_have_several_chunks(gpu, oracle, G, W, H, y0, where):
+    """Lists of one tile a little shorter and longer than whole chunks, pixels that stop in different chunks and at either
+    entry of a pair, a few Gaussians that take the general path."""
+    # A pixel whose transmittance comes within fp32 rounding of the threshold may stop one entry earlier or later, which is all
+    # of a deep Gaussian's gradient: 1025 of them have such a pixel (1.2e-6 away) and the fp32 oracle lies 25 times the bound
+    # from the fp64 one.  So the first scene that keeps its distance: 1e-5 is five times the root of 1100 roundings.
+    for seed in range(300 + G, 320 + G):
+        params, depth = random_scene(G, 16, 16, seed=seed, scale_px=(6.0, 14.0))  # reach 18 pixels: in the tile's list, all of them
+        params[1] += y0
+        alpha0 = 1.0 / G if where is None else min(0.8, 9.2 / (0.65 * where * G))
+        params[8] = np.log(alpha0 / (1 - alpha0)) + 0.5 * params[8]
+        params[2:4, ::16] = np.log(5e4)
+        target = np.random.default_rng(G).uniform(0, 1, (H, W, 3)).astype(np.float32)
+        rects = oracle.splat_step(W, H, params, depth, target, np.float64, want_grads=False)["rects"]
+        stops, margin = _stops(params, depth, rects, W, max(0, y0 - 48), min(H, y0 + 64))
+        if margin > 1e-5:
+            break
+    assert margin > 1e-5
+    stops = stops[y0 - max(0, y0 - 48):][:16, :16]  # of the tile that has them all
+    if where is None:
+        assert (stops == G).all()
+    else:
+        assert (stops < G).any() and np.unique(stops[stops < G] % 2).size == 2
+        assert where == 0.9 or G in (63, 64, 65, 200) or np.unique((stops - 1) // 64).size > 1
+    got = _gpu_step(gpu, W, H, params, depth, target)
+    assert got["longest_list"] == G
+    _check_against_oracle(oracle, got, W, H, params, depth, target)
 
 
 @pytest.mark.parametrize("W,H,needles,short_px,long_px,seed", [
@@ -538,6 +589,7 @@ def test_small_scenes_keep_no_room_for_the_lists_of_supertiles(gpu):
     from xyz_autodiff_cuda_amd import splat
 
     G, W, H = 1000, 640, 427
+    splat.SplatContext(W, H, G).close()  # what the first context of a process loads is not counted
     torch.cuda.synchronize()
     before = torch.cuda.mem_get_info(gpu)[0]
     ctx = splat.SplatContext(W, H, G, pair_capacity_hint=64 << 20)
