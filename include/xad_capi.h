@@ -419,19 +419,23 @@ int xad_linreg_gradient_f64(int strategy, size_t n, size_t total,
                             const double* params, double* out, void* stream);
 /* `epochs` SGD steps, entirely on the device: step e draws `batch` rows with
  * replacement, row of draw i = random bits (seed, stream 0, e * batch + i)
- * modulo total (see xad_host_rng_bits), sums the gradients with WAVE_LDS, and
+ * modulo total (see xad_host_rng_bits), sums the gradients in fp64, and
  * updates  p -= lr(e) * sum / batch  with  lr(e) = lr_first * (lr_last /
  * lr_first)^(e / epochs)  (linear_regression_sgd.cu:137-140).  params (device, 4
  * doubles) is updated in place; loss_history (device, `epochs` doubles, or NULL)
  * receives the mean batch loss before each update.  Synchronous: returns when
- * the last step has finished. */
+ * the last step has finished.  Batches of up to 8192 samples are summed by one
+ * workgroup (calls of one or two steps of more than 2048 and 4096 excepted), for
+ * which the call allocates up to 8 MiB for samples drawn ahead and frees them
+ * again; larger ones, and any if that memory is not there, as by WAVE_LDS. */
 int xad_linreg_sgd_f64(size_t total, const double* x1, const double* x2, const double* y,
                        double* params, int batch, int epochs, double lr_first, double lr_last,
                        uint64_t seed, double* loss_history, void* stream);
 /* xad_linreg_sgd_f64 for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  No
- * counterpart in the reference.  Same arguments, same draws and same results
- * as xad_linreg_sgd_f64, with two differences:
+ * counterpart in the reference.  Same arguments, same draws and, but for the
+ * order in which a step's sums are formed (always that of WAVE_LDS here), same
+ * results as xad_linreg_sgd_f64, with two differences:
  *   - the gradient sums of a step live in a 256-byte array that is part of the
  *     library's device image (one copy per device, held until the process ends)
  *     instead of a buffer allocated and freed by the call; the call makes no

@@ -562,7 +562,7 @@ def test_tile_lists_equal_what_rectangles_and_depths_imply(gpu, oracle, G, W, H,
     (63, 40, 24), (64, 40, 24), (65, 40, 24), (511, 16, 16), (2049, 90, 50),  # every tile against every Gaussian: chunk edges
     (16384, 40, 33), (16385, 40, 33),  # the most Gaussians that are taken so, and the first number that goes by supertiles
     (300, 1024, 512), (300, 1030, 512),  # 2048 tiles, and 2080
-    (9600, 720, 704), (13000, 720, 720),  # 297 000 tests, and 411 000
+    (9600, 720, 704), (13000, 720, 720),  # 297 000 tests, and 413 100
 ])
 def test_tile_lists_on_both_sides_of_the_binning_rule(gpu, oracle, G, W, H):
     import torch

@@ -137,7 +137,8 @@ __global__ void linreg_update_kernel(double* params, double* sums, double learni
 // What bounds it: below about 1000 samples the two barriers and the sum between them, above that what one compute
 // unit gets from beyond its XCD's L2 (about 60 GB/s).
 // Measured (us per step, calls of 200 steps, two launches a step / so): batch 256 6.1 / 0.9, 1024 7.1 / 1.2, 2048
-// 6.7 / 1.6, 4096 7.3 / 2.3, 8192 6.8 / 4.0; 16 384 would be level (7.4).  Calls of 20 steps: 9.0 / 2.2 to 9.4 / 6.6.
+// 6.7 / 1.6, 4096 7.3 / 2.3, 8192 6.8 / 4.0; 16 384 would be level (7.4).  Calls of 20 steps: 9.0 / 2.2 to 9.4 / 6.6; for
+// shorter ones see one_block_takes().
 using xad_linreg::kStepLanes;
 constexpr int kStepsPerLaunch = 64;
 constexpr std::size_t kGatheredBytes = std::size_t(4) << 20;  // of one launch's steps, at most (two such buffers)

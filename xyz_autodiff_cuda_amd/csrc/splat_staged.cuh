@@ -19,7 +19,7 @@ constexpr float kHalfLog2e = 0.72134752044448170368f;  // log2(e) / 2
 struct alignas(16) Staged {
     float cx, cy, a_s, b2_s;          // centre; a' and 2b'
     float c_s, alpha0, a, b;          // c'; sigmoid(opacity); inverse covariance as stored
-    float red, green, blue, c;        // colour (a lane takes the channel of its number modulo 4); inverse covariance
+    float red, green, blue, c;        // colour; inverse covariance
 };
 static_assert(sizeof(Staged) == 48, "Staged must be three float4");
 
@@ -83,8 +83,11 @@ XAD_INLINE bool negligible_in_tile(const Staged& s, float tile_x, float tile_y) 
 //     than rounding.  (q >= (1 - |b| / sqrt(ac)) (a dx^2 + c dy^2), the rounding of its three terms is at most
 //     5e-7 (a dx^2 + c dy^2), and 1 - |b| / sqrt(ac) >= (ac - b^2) / 2ac > 5e-6);
 //   - a pixel whose x is kFarAway gets alpha = 0: there a dx^2 >= 1e-9 1e36, and neither 2 |b dx dy| <=
-//     2 sqrt(ac) 1e18 |dy| nor c dy^2 comes near it (|dy| < 1e6).
+//     2 sqrt(ac) 1e18 |dy| nor c dy^2 comes near it (|dy| < 1.1e6: images are at most 32767 tiles high).
 // Comparisons with NaN are false, so an odd record is taken with care.
+// An entry that needs care sends its pair to the general path.  Where nearly all do, opacity logits ~ N(6, 1), a step of
+// 200 000 Gaussians at 2048 x 2048 takes 635 us (forward 157, backward 400), of 10 000 at 512 x 512 111 us; loops without
+// the distinction, every pixel's compares and selects in every trip, took 668 (195, 393) and 137.
 constexpr float kFarAway = 1e18f;
 
 XAD_INLINE bool ill_shaped(const Staged& s) {
