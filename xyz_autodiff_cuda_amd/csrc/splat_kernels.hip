@@ -858,7 +858,7 @@ static unsigned padded_tile_blocks(int tiles) { return static_cast<unsigned>(((t
 // Pieces for the backward walk to be done by more wavefronts where a tile each leaves the SIMDs with few; what they cost is
 // the forward pass's states.  Forward + backward with 8 / 4 / 3 / 2 / 1 pieces (us): 10 000 Gaussians at 512 x 512 (1024
 // tiles) 31 + 48 / 30 + 45 / 28 + 45 / 28 + 48 / 25 + 64, 50 000 at 1277 x 719 (3600 tiles) 120 + 157 / 93 + 159 / 84 + 155 /
-// 80 + 157 / 65 + 177.  (So eight are 4 us more than four at 1024 tiles; they are for fewer tiles and longer lists.)
+// 80 + 157 / 65 + 177.  (The lines were drawn with the kernels before these; at 1024 tiles eight are now 4 us more than four.)
 int render_segments(int width, int height) {
     const int tiles = ((width + kTile - 1) / kTile) * ((height + kTile - 1) / kTile);
     return tiles <= 1024 ? 8 : (tiles <= 2048 ? 4 : (tiles <= 4096 ? 2 : 1));
