@@ -19,6 +19,11 @@ from tests._scenes import one_gaussian, random_scene
 pytestmark = pytest.mark.gpu
 
 
+# For tests of what a call leaves behind (list capacities, status words): 256 tiles, whose lists are made by testing every tile,
+# and 2080, which is more than are, so that these go by way of supertiles.
+BOTH_BINNINGS = [(256, 256), (1040, 512)]
+
+
 def _gpu_step(gpu, W, H, params, depth, target, forward_only=False):
     import torch
 
@@ -74,14 +79,15 @@ def test_step_matches_oracle(gpu, oracle, G, W, H, scale):
     _check_against_oracle(oracle, _gpu_step(gpu, W, H, params, depth, target), W, H, params, depth, target)
 
 
-def test_depth_ranks_follow_the_depths_of_each_call(gpu, oracle):
+@pytest.mark.parametrize("W,H", [(96, 80), (1040, 512)])
+def test_depth_ranks_follow_the_depths_of_each_call(gpu, oracle, W, H):
     """The context keeps the depth ranks of the previous call while the depths stay the same;
     a call with other depths (even one changed value) must be ordered by them."""
     import torch
 
     from xyz_autodiff_cuda_amd import splat
 
-    W, H, G = 96, 80, 400
+    G = 400
     params, depth = random_scene(G, W, H, seed=8, scale_px=(3.0, 15.0))
     params[8] += 2.0  # opaque enough for the order to matter
     reversed_depth = (1.0 - depth).astype(np.float32)
@@ -303,12 +309,13 @@ def test_host_core_step_and_gpu_step_agree(gpu, oracle):
     assert (np.abs(host["grads"].astype(np.float64) - got["grads"]) <= 2.0 * tolerance).all()
 
 
-def test_pair_buffers_grow_on_demand(gpu, oracle):
+@pytest.mark.parametrize("W,H", [(128, 128), (1040, 512)])
+def test_pair_buffers_grow_on_demand(gpu, oracle, W, H):
     import torch
 
     from xyz_autodiff_cuda_amd import splat
 
-    G, W, H = 400, 128, 128
+    G = 400
     params, depth = random_scene(G, W, H, seed=8, scale_px=(8.0, 20.0))
     target = np.zeros((H, W, 3), np.float32)
     ctx = splat.SplatContext(W, H, G, pair_capacity_hint=16)  # far too small on purpose
@@ -599,14 +606,15 @@ def test_small_scenes_keep_no_room_for_the_lists_of_supertiles(gpu):
     assert (256 << 20) <= taken <= (256 << 20) + 2 * fixed, taken
 
 
+@pytest.mark.parametrize("W,H", [(160, 112), (1040, 512)])
 @pytest.mark.parametrize("mode", ["static", "every_step"])
-def test_steps_that_do_not_wait(gpu, oracle, mode):
+def test_steps_that_do_not_wait(gpu, oracle, mode, W, H):
     """Without a loss read-back a step only queues work; results equal those of the default mode."""
     import torch
 
     from xyz_autodiff_cuda_amd import splat
 
-    G, W, H = 900, 160, 112
+    G = 900
     params, depth = random_scene(G, W, H, seed=31, scale_px=(1.0, 14.0))
     target = np.random.default_rng(4).uniform(0, 1, (H, W, 3)).astype(np.float32)
     p, t = torch.from_numpy(params).to(gpu), torch.from_numpy(target).to(gpu)
@@ -681,12 +689,13 @@ def test_a_recorded_step_can_be_replayed(gpu, oracle, G, W, H, scale):
     eager.close()
 
 
-def test_static_mode_reports_a_changed_depth(gpu, xad):
+@pytest.mark.parametrize("W,H", [(96, 96), (1040, 512)])
+def test_static_mode_reports_a_changed_depth(gpu, xad, W, H):
     import torch
 
     from xyz_autodiff_cuda_amd import splat
 
-    G, W, H = 300, 96, 96
+    G = 300
     params, depth = random_scene(G, W, H, seed=12, scale_px=(2.0, 10.0))
     p, t = torch.from_numpy(params).to(gpu), torch.zeros(H, W, 3, device=gpu)
     ctx = splat.SplatContext(W, H, G, depth_mode="static")
@@ -700,12 +709,13 @@ def test_static_mode_reports_a_changed_depth(gpu, xad):
     ctx.close()
 
 
-def test_overflow_in_a_step_that_does_not_wait_is_reported_later(gpu, oracle, xad):
+@pytest.mark.parametrize("W,H", BOTH_BINNINGS)
+def test_overflow_in_a_step_that_does_not_wait_is_reported_later(gpu, oracle, W, H, xad):
     import torch
 
     from xyz_autodiff_cuda_amd import splat
 
-    G, W, H = 600, 256, 256
+    G = 600
     small, depth = random_scene(G, W, H, seed=5, scale_px=(0.5, 1.0))
     large = small.copy()
     large[2:4] += np.log(30.0)  # the same Gaussians, thirty times wider: many times the pairs
@@ -735,14 +745,15 @@ def test_overflow_in_a_step_that_does_not_wait_is_reported_later(gpu, oracle, xa
     ctx2.close()
 
 
-def test_the_getters_report_and_settle_an_overflow_too(gpu, oracle, xad):
+@pytest.mark.parametrize("W,H", BOTH_BINNINGS)
+def test_the_getters_report_and_settle_an_overflow_too(gpu, oracle, W, H, xad):
     """xad_splat_get_stats and xad_splat_get_lists wait for the device, so they are calls that report what a
     step that did not wait has left behind, and enlarge the lists."""
     import torch
 
     from xyz_autodiff_cuda_amd import splat
 
-    G, W, H = 600, 256, 256
+    G = 600
     small, depth = random_scene(G, W, H, seed=5, scale_px=(0.5, 1.0))
     large = small.copy()
     large[2:4] += np.log(30.0)
@@ -764,14 +775,15 @@ def test_the_getters_report_and_settle_an_overflow_too(gpu, oracle, xad):
         ctx.close()
 
 
-def test_forward_only_calls_enlarge_the_lists_themselves(gpu, oracle):
+@pytest.mark.parametrize("W,H", BOTH_BINNINGS)
+def test_forward_only_calls_enlarge_the_lists_themselves(gpu, oracle, W, H):
     """In the default depth mode a forward call waits for the binning anyway: a scene that has outgrown the lists
     is binned again into larger ones before anything is composited, also when no call ever asks for a loss."""
     import torch
 
     from xyz_autodiff_cuda_amd import splat
 
-    G, W, H = 600, 256, 256
+    G = 600
     small, depth = random_scene(G, W, H, seed=5, scale_px=(0.5, 1.0))
     target = np.zeros((H, W, 3), np.float32)
     d = torch.from_numpy(depth).to(gpu)

@@ -99,14 +99,15 @@ def _grown_state(W, H, G, target):
     return state
 
 
+# the second size has more tiles than small scenes may have: other lists, and a level of them more that can overflow
+@pytest.mark.parametrize("W,H", [(256, 256), (1040, 512)])
 @pytest.mark.parametrize("iterations,loss_every", [(40, 0), (24, 6), (7, 1)])
-def test_a_run_whose_lists_outgrow_their_buffers_equals_a_run_with_ample_buffers(gpu, iterations, loss_every):
+def test_a_run_whose_lists_outgrow_their_buffers_equals_a_run_with_ample_buffers(gpu, iterations, loss_every, W, H):
     """Iterations that do not report a loss never wait for the device, so nobody sees that the tile lists of a
     scene that has grown no longer fit.  No update may use such gradients (the loop of the reference computes all
     gradients, then steps: gaussian_splatting_training.cu:127-160): the updates are withheld on the device, and the
     iterations are run again once the host has looked.  The result must be that of a run whose buffers were ample
     from the start, step numbers included."""
-    W = H = 256
     G = 4000
     target = trainer.test_pattern(W, H)
     state = _grown_state(W, H, G, target)
@@ -167,11 +168,11 @@ def test_a_run_whose_lists_outgrow_their_buffers_equals_a_run_with_ample_buffers
     ample.close()
 
 
-def test_a_withheld_update_changes_nothing(gpu, tmp_path):
+@pytest.mark.parametrize("W,H", [(256, 256), (1040, 512)])
+def test_a_withheld_update_changes_nothing(gpu, tmp_path, W, H):
     """One iteration from a known state with buffers that are too small, nobody asking for the loss: afterwards the
     state is that of one complete iteration with step number 3 (not of a step on truncated lists, not of two
     updates), and the trainer says that it ran one iteration twice."""
-    W = H = 256
     G = 4000
     target = trainer.test_pattern(W, H)
     state = _grown_state(W, H, G, target)
