@@ -27,25 +27,44 @@ struct RowRates {
     float lr_corrected[kMaxRows];
 };
 
-__global__ void __launch_bounds__(kBlock) adam_kernel(std::size_t n, int rows, float* __restrict__ p,
+// One row per blockIdx.y, kPer elements per lane.  What bounds it is HBM where rows are long, and below that the round trips
+// to memory of a lane.  So a lane asks for everything it needs, the gate included, before it looks at any of it, and rows
+// are side by side, not one after the other: 1000 columns of 9 rows 5.3 -> 2.5 us, 50 000 7.3 -> 4.6; 200 000 (50 MB) 9.0
+// as before with four elements per lane, 10.6 with one.
+template <int kPer>
+__global__ void __launch_bounds__(kBlock) adam_kernel(std::size_t n, float* __restrict__ p,
                                                       const float* __restrict__ g, float* __restrict__ m,
                                                       float* __restrict__ v, RowRates rates, float beta1, float beta2,
                                                       float eps, const std::uint32_t* __restrict__ hold_if_nonzero,
                                                       std::uint32_t* __restrict__ held_count) {
-    const std::size_t i = static_cast<std::size_t>(blockIdx.x) * kBlock + threadIdx.x;
+    const std::size_t first = static_cast<std::size_t>(blockIdx.x) * kBlock * kPer + threadIdx.x;
+    const std::size_t row = static_cast<std::size_t>(blockIdx.y) * n;
+    float grad[kPer], m_old[kPer], v_old[kPer], p_old[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const std::size_t i = first + static_cast<std::size_t>(k) * kBlock;
+        if (i < n) {
+            grad[k] = g[row + i];
+            m_old[k] = m[row + i];
+            v_old[k] = v[row + i];
+            p_old[k] = p[row + i];
+        }
+    }
     if (hold_if_nonzero != nullptr && *hold_if_nonzero != 0) {  // the same answer for every lane of the launch
-        if (i == 0 && held_count != nullptr) atomicAdd(held_count, 1u);
+        if (first == 0 && blockIdx.y == 0 && held_count != nullptr) atomicAdd(held_count, 1u);
         return;
     }
-    if (i >= n) return;
-    for (int r = 0; r < rows; ++r) {
-        const std::size_t at = static_cast<std::size_t>(r) * n + i;
-        const float grad = g[at];
-        const float m_new = beta1 * m[at] + (1.0f - beta1) * grad;
-        const float v_new = beta2 * v[at] + (1.0f - beta2) * grad * grad;
-        m[at] = m_new;
-        v[at] = v_new;
-        p[at] -= rates.lr_corrected[r] * m_new / (::sqrtf(v_new) + eps);
+    const float rate = rates.lr_corrected[blockIdx.y];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const std::size_t i = first + static_cast<std::size_t>(k) * kBlock;
+        if (i < n) {
+            const float m_new = beta1 * m_old[k] + (1.0f - beta1) * grad[k];
+            const float v_new = beta2 * v_old[k] + (1.0f - beta2) * grad[k] * grad[k];
+            m[row + i] = m_new;
+            v[row + i] = v_new;
+            p[row + i] = p_old[k] - rate * m_new / (::sqrtf(v_new) + eps);
+        }
     }
 }
 
@@ -64,8 +83,16 @@ int adam_step(const char* who, std::size_t n, int rows, float* params, const flo
     const float beta2_t = ::powf(beta2, static_cast<float>(iteration));
     RowRates rates{};
     for (int r = 0; r < rows; ++r) rates.lr_corrected[r] = row_learning_rates[r] * ::sqrtf(1.0f - beta2_t) / (1.0f - beta1_t);
-    hipLaunchKernelGGL(adam_kernel, dim3(xad::blocks_for(n, kBlock)), dim3(kBlock), 0, xad::as_stream(stream), n, rows,
-                       params, grads, m, v, rates, beta1, beta2, eps, hold_if_nonzero, held_count);
+    // four elements per lane where that leaves enough wavefronts to fill the device
+    constexpr std::size_t kFewBlocks = 512;
+    const int per = n * static_cast<std::size_t>(rows) >= kFewBlocks * 4 * kBlock ? 4 : 1;
+    const dim3 grid(xad::blocks_for(n, kBlock * static_cast<unsigned>(per)), static_cast<unsigned>(rows)), block(kBlock);
+    if (per == 4)
+        hipLaunchKernelGGL(adam_kernel<4>, grid, block, 0, xad::as_stream(stream), n, params, grads, m, v, rates, beta1, beta2, eps,
+                           hold_if_nonzero, held_count);
+    else
+        hipLaunchKernelGGL(adam_kernel<1>, grid, block, 0, xad::as_stream(stream), n, params, grads, m, v, rates, beta1, beta2, eps,
+                           hold_if_nonzero, held_count);
     XAD_HIP_TRY(hipGetLastError());
     return XAD_OK;
 }

@@ -797,19 +797,30 @@ __global__ void __launch_bounds__(kChunk) render_backward_kernel(
 // accumulated record gradients, and lets the nodes' backward rules carry them
 // to log-scale, theta and the opacity logit.  Centre and colour gradients pass
 // straight through.
+// What bounds it below some 100 000 Gaussians is the longest chain of loads.  That was the one lane that added the
+// parts of the loss up, eight at a time; a wavefront asks for all of them at once, and a lane reads its accumulator row as
+// three float4: 5.7 -> 3.8 us at 1000 Gaussians, 6.9 -> 5.6 at 200 000.
 __global__ void __launch_bounds__(256) gaussian_backward_kernel(int G, const float* __restrict__ params,
                                                                 const float* __restrict__ record_grads,
                                                                 float* __restrict__ grads, double* __restrict__ loss) {
     const int g = blockIdx.x * 256 + threadIdx.x;
-    if (g >= G) return;
-    if (g == 0) {
-        double total = 0.0;
-#pragma unroll 8
-        for (int k = 0; k < kLossParts; ++k) total += loss[kLossStride * (1 + k)];
-        loss[0] = total;
+    static_assert(kLossParts == 64, "a lane of the first wavefront for every part of the loss");
+    if (blockIdx.x == 0 && threadIdx.x < kLossParts) {
+        const double total = accumulate::wave::sum(loss[kLossStride * (1 + threadIdx.x)]);
+        if (threadIdx.x == 0) loss[0] = total;
     }
+    if (g >= G) return;
     const std::size_t n = static_cast<std::size_t>(G);
-    const float* acc = record_grads + static_cast<std::size_t>(g) * kRecordGradStride;
+    float acc[12];
+    const float4* row = reinterpret_cast<const float4*>(record_grads + static_cast<std::size_t>(g) * kRecordGradStride);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float4 quarter = row[k];
+        acc[4 * k] = quarter.x;
+        acc[4 * k + 1] = quarter.y;
+        acc[4 * k + 2] = quarter.z;
+        acc[4 * k + 3] = quarter.w;
+    }
 
     Variable<2, float> log_scale;
     log_scale[0] = params[2 * n + g];
