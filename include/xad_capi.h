@@ -424,10 +424,11 @@ int xad_linreg_gradient_f64(int strategy, size_t n, size_t total,
  * lr_first)^(e / epochs)  (linear_regression_sgd.cu:137-140).  params (device, 4
  * doubles) is updated in place; loss_history (device, `epochs` doubles, or NULL)
  * receives the mean batch loss before each update.  Synchronous: returns when
- * the last step has finished.  Batches of up to 8192 samples are summed by one
- * workgroup (calls of one or two steps of more than 2048 and 4096 excepted), for
- * which the call allocates up to 8 MiB for samples drawn ahead and frees them
- * again; larger ones, and any if that memory is not there, as by WAVE_LDS. */
+ * the last step has finished.  The steps of batches of up to 8192 samples are
+ * taken by one workgroup (calls of one or two steps of more than 2048 and 4096
+ * excepted), from samples drawn ahead or, in longer calls, from sums over them,
+ * for which the call allocates up to 8 MiB and frees them again; those of larger
+ * batches, and any if that memory is not there, as by WAVE_LDS. */
 int xad_linreg_sgd_f64(size_t total, const double* x1, const double* x2, const double* y,
                        double* params, int batch, int epochs, double lr_first, double lr_last,
                        uint64_t seed, double* loss_history, void* stream);

@@ -138,6 +138,16 @@ def sgd_one_block(batch, epochs):
     return bool(load().xad_test_sgd_one_block(ctypes.c_int(batch), ctypes.c_int(epochs)))
 
 
+def sgd_from_moments(x1, x2, y, params, centre):
+    """Gradient sums and loss of a batch from its samples' moments about `centre` (a, c), and whether the loss is resolved."""
+    out = np.zeros(5, np.float64)
+    arrays = [np.ascontiguousarray(a, dtype=np.float64) for a in (x1, x2, y, params)]
+    fn = load().xad_test_sgd_from_moments
+    resolved = fn(ctypes.c_size_t(arrays[0].size), *[a.ctypes.data_as(ctypes.c_void_p) for a in arrays], ctypes.c_double(centre[0]),
+                  ctypes.c_double(centre[1]), out.ctypes.data_as(ctypes.c_void_p))
+    return out, bool(resolved)
+
+
 def parallel_accumulation(threads, block):
     out = np.zeros(3, np.float64)
     rc = load().xad_test_parallel_accumulation(ctypes.c_size_t(threads), ctypes.c_int(block), out.ctypes.data_as(ctypes.c_void_p))

@@ -13,6 +13,7 @@
 #include "tester_suite.cuh"
 #include "concept_checks.cuh"
 #include "../../xyz_autodiff_cuda_amd/csrc/linreg_launches.cuh"
+#include "../../xyz_autodiff_cuda_amd/csrc/linreg_moments.cuh"
 #include "../../xyz_autodiff_cuda_amd/csrc/splat_staged.cuh"
 
 using namespace xyz_autodiff;
@@ -297,6 +298,27 @@ extern "C" std::int64_t xad_test_sgd_launches(int epochs, int per_launch) {
 }
 
 extern "C" int xad_test_sgd_one_block(int batch, int epochs) { return xad_linreg::one_block_takes(batch, epochs) ? 1 : 0; }
+
+extern "C" int xad_test_sgd_by_moments(int batch, int epochs) { return xad_linreg::moments_take(batch, epochs) ? 1 : 0; }
+
+// Host.  Gradient sums and loss of a batch from its samples' moments about (a0, c0); returns whether the loss is resolved.
+extern "C" int xad_test_sgd_from_moments(std::size_t n, const double* x1, const double* x2, const double* y, const double* params,
+                                         double a0, double c0, double* out) {
+    using namespace xad_linreg;
+    Twofold g[kMoments + 1] = {};
+    for (std::size_t i = 0; i < n; ++i) add_sample(g, x1[i], x2[i], y[i], a0, c0);
+    g[kMoments] = {static_cast<double>(n), 0.0};
+    const double p[4] = {params[0], params[1], params[2], params[3]};
+    const Coefficients k(p, a0, c0);
+    double gradients[4];
+    gradient(k, residual_moment(g[kF0U], g[kUU], g[kUQ], g[kUV], g[kU], k), residual_moment(g[kF0Q], g[kUQ], g[kQQ], g[kQV], g[kQ], k),
+             residual_moment(g[kF0V], g[kUV], g[kQV], g[kQ], g[kV], k), residual_moment(g[kF0], g[kU], g[kQ], g[kV], g[kMoments], k),
+             gradients);
+    for (int j = 0; j < 4; ++j) out[j] = gradients[j];
+    bool resolved = false;
+    out[4] = batch_loss(g, k, &resolved);
+    return resolved ? 1 : 0;
+}
 
 extern "C" int xad_test_run_case_host(int id, double* out) { return xad_test::run_case(id, out); }
 

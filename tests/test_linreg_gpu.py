@@ -160,3 +160,80 @@ def test_sgd_reference_hyperparameters_converge(gpu):
     assert np.all(np.isfinite(p)) and np.all(np.isfinite(hist))
     np.testing.assert_allclose(p[:3], linreg.TRUE_PARAMS[:3], atol=0.05)
     assert hist[-1] < 2e-3 * hist[0]
+
+
+def _steps_in_extended_precision(x1, x2, y, batch, epochs, lr_first, lr_last, seed):
+    real = np.longdouble
+    p, history = [real(v) for v in linreg.INITIAL_PARAMS], []
+    decay = np.log(lr_last / lr_first) / epochs
+    for e in range(epochs):
+        rows = linreg.batch_rows(seed, e, batch, x1.size)
+        u, v = p[0] - x1[rows].astype(real), p[2] - x2[rows].astype(real)
+        r = u * u + p[1] * v * v + p[3] - y[rows].astype(real)
+        history.append((r * r).sum() / batch)
+        g = [(4 * r * u).sum(), (2 * r * v * v).sum(), (4 * r * p[1] * v).sum(), (2 * r).sum()]
+        rate = real(lr_first * np.exp(decay * e))
+        p = [q - rate * (s / batch) for q, s in zip(p, g)]
+    return np.array(p), np.array(history)
+
+
+# around the sizes at which a step's samples are dealt to more lanes, parts and launches, and the shortest calls of each size
+@pytest.mark.parametrize("batch,epochs", [(1, 16), (63, 64), (255, 65), (256, 129), (257, 16), (1024, 20), (1025, 10), (2049, 7),
+                                          (4096, 64), (4097, 5), (8191, 66), (8192, 5)])
+def test_steps_from_moments_are_as_exact_as_doubles(gpu, batch, epochs):
+    """A step rounds its parameters (2^-53) and its rate's exponential (one unit in the last place of two libraries'); to the
+    loss that is a few times as much, and the iteration contracts."""
+    import torch
+
+    total, lr = 4003, (1e-4, 1e-6)
+    x1, x2, y = linreg.synthetic_data(total, seed=batch)
+    want_p, want_h = _steps_in_extended_precision(x1, x2, y, batch, epochs, *lr, seed=7)
+    params = torch.tensor(linreg.INITIAL_PARAMS, dtype=torch.float64, device=gpu)
+    hist = linreg.sgd(*_device(gpu, x1, x2, y), params, batch, epochs, *lr, seed=7, want_history=True)
+    bound = 4 * (epochs + 4) * 2.0 ** -53
+    assert (np.abs(params.cpu().numpy() - want_p).max() / np.abs(want_p).max()) <= bound
+    assert (np.abs(hist.cpu().numpy() - want_h) / want_h).max() <= 4 * bound
+
+
+def _sgd_both_ways(gpu, x1, x2, y, params, batch, epochs, lr):
+    """(parameters, losses) by the usual entry point and by the one that always sums gradients sample by sample."""
+    import torch
+
+    out = []
+    for static in (False, True):
+        p = torch.tensor(params, dtype=torch.float64, device=gpu)
+        h = torch.full((epochs,), -1.0, dtype=torch.float64, device=gpu)
+        linreg.sgd(*_device(gpu, x1, x2, y), p, batch, epochs, lr, lr, seed=4, history=h, static_scratch=static)
+        torch.cuda.synchronize()
+        out.append((p.cpu().numpy(), h.cpu().numpy()))
+    return out
+
+
+@pytest.mark.parametrize("lr", [1e-2, 1.0, 1e6])
+def test_steps_that_diverge_end_as_the_graph_says(gpu, lr):
+    x1, x2, y = linreg.synthetic_data(3000, seed=2)
+    (p, h), (want_p, want_h) = _sgd_both_ways(gpu, x1, x2, y, linreg.INITIAL_PARAMS, 700, 70, lr)
+    assert not np.all(np.isfinite(want_h))
+    np.testing.assert_array_equal(np.isnan(h), np.isnan(want_h))
+    np.testing.assert_array_equal(np.isinf(h), np.isinf(want_h))
+    np.testing.assert_array_equal(np.isnan(p), np.isnan(want_p))
+    finite = np.isfinite(want_h)
+    np.testing.assert_allclose(h[finite], want_h[finite], rtol=1e-9)
+
+
+def test_samples_that_are_not_finite_and_a_fit_without_a_residual(gpu):
+    x1, x2, y = linreg.synthetic_data(3000, seed=2)
+    for value in (np.inf, -np.inf, np.nan):
+        broken = y.copy()
+        broken[5] = value
+        (p, h), (want_p, want_h) = _sgd_both_ways(gpu, x1, x2, broken, linreg.INITIAL_PARAMS, 300, 40, 1e-4)
+        np.testing.assert_array_equal(np.isnan(h), np.isnan(want_h))
+        np.testing.assert_array_equal(np.isinf(h), np.isinf(want_h))
+        np.testing.assert_array_equal(np.isnan(p), np.isnan(want_p))
+        np.testing.assert_allclose(h[np.isfinite(want_h)], want_h[np.isfinite(want_h)], rtol=1e-9)
+    # whole numbers: residuals, losses and gradients are exactly zero, and nothing moves
+    u, v = np.round(x1), np.round(x2)
+    exact = (2.0, 3.0, -1.0, 5.0)
+    t = (exact[0] - u) ** 2 + exact[1] * (exact[2] - v) ** 2 + exact[3]
+    for p, h in _sgd_both_ways(gpu, u, v, t, exact, 300, 40, 1e-2):
+        assert np.array_equal(p, exact) and np.array_equal(h, np.zeros(40))

@@ -165,3 +165,46 @@ def test_sgd_rule_where_two_launches_a_step_are_faster():
         assert not _native.sgd_one_block(batch, epochs), (batch, epochs)
     for batch, epochs in ((1, 1), (256, 1), (2048, 1), (2049, 2), (4096, 2), (4096, 2**31 - 1), (4097, 3), (8192, 3), (8192, 10_000)):
         assert _native.sgd_one_block(batch, epochs), (batch, epochs)
+
+
+@pytest.mark.parametrize("offset", [0.0, 3.0, 1e6])
+@pytest.mark.parametrize("noise", [0.5, 1e-3, 0.0])
+@pytest.mark.parametrize("away", [3.0, 1e-3, 0.0])
+def test_gradient_and_loss_from_moments(offset, noise, away):
+    """Against exact rational arithmetic.  Two doubles a sum keep 2^-100 of what is added up (here the squares of the moments'
+    terms, up to (60)^2 n); what comes out is rounded to a double once per operation on it, four at most."""
+    from fractions import Fraction
+
+    from tests import _native
+
+    n = 300
+    x1, x2, _ = linreg.synthetic_data(n, seed=3)
+    x1, x2 = x1 + offset, x2 - offset
+    g = np.random.default_rng(5).standard_normal(n) * noise
+    true = (2.5 + offset, 1.8, -1.2 - offset, 0.7)
+    y = (x1 - true[0]) ** 2 + true[1] * (x2 - true[2]) ** 2 + true[3] + g
+    params = np.array(true) + np.array([away, 0.1 * away, -away, 0.3 * away])
+    out, resolved = _native.sgd_from_moments(x1, x2, y, params, (offset, -offset))
+    a, b, c, d = (Fraction(float(v)) for v in params)
+    want = [Fraction(0)] * 5
+    for u, v, t in zip(x1, x2, y):
+        e, f = a - Fraction(float(u)), c - Fraction(float(v))
+        r = e * e + b * f * f + d - Fraction(float(t))
+        for k, term in enumerate((4 * r * e, 2 * r * f * f, 4 * r * b * f, 2 * r, r * r)):
+            want[k] += term
+    scale = 3600.0 * 3600.0 * n
+    for k in range(5):
+        if k == 4 and not resolved:
+            assert noise == 0.0 and away == 0.0  # a fit that leaves nothing but rounding: its loss is left to the graph
+            continue
+        assert abs(float(Fraction(float(out[k])) - want[k])) <= 4 * 2.0 ** -53 * abs(float(want[k])) + 2.0 ** -98 * scale, k
+
+
+def test_rule_where_moments_of_the_samples_are_faster():
+    from tests import _native
+
+    fn = _native.load().xad_test_sgd_by_moments
+    for batch, epochs in ((1, 15), (1024, 15), (1025, 9), (2048, 9), (2049, 6), (4096, 6), (4097, 4), (8192, 4), (8193, 10_000), (1, 0)):
+        assert not fn(batch, epochs), (batch, epochs)
+    for batch, epochs in ((1, 16), (1024, 16), (1025, 10), (2048, 10), (2049, 7), (4096, 2**31 - 1), (4097, 5), (8192, 5)):
+        assert fn(batch, epochs), (batch, epochs)

@@ -11,6 +11,7 @@
 #include "common.cuh"
 #include "linreg.cuh"
 #include "linreg_launches.cuh"
+#include "linreg_moments.cuh"
 #include "rng.cuh"
 
 namespace {
@@ -135,7 +136,7 @@ __global__ void linreg_update_kernel(double* params, double* sums, double learni
 // draw and gather, into contiguous arrays, the samples of the steps that the next launch will take.  The one block
 // then streams 24 bytes per sample; it asks for the next step's samples before it adds this step's sums up.
 // What bounds it: below about 1000 samples the two barriers and the sum between them, above that what one compute
-// unit gets from beyond its XCD's L2 (about 60 GB/s).
+// unit gets from beyond its XCD's L2 (about 60 GB/s).  Longer calls take linreg_moment_steps_kernel.
 // Measured (us per step, calls of 200 steps, two launches a step / so): batch 256 6.1 / 0.9, 1024 7.1 / 1.2, 2048
 // 6.7 / 1.6, 4096 7.3 / 2.3, 8192 6.8 / 4.0; 16 384 would be level (7.4).  Calls of 20 steps: 9.0 / 2.2 to 9.4 / 6.6; for
 // shorter ones see one_block_takes().
@@ -233,6 +234,235 @@ __global__ void __launch_bounds__(kStepLanes) linreg_steps_kernel(SerialSteps a)
         __syncthreads();
     }
     if (t < 4) a.params[t] = now[t];
+}
+
+// ---------------------------------------------------------------------------
+// The steps of longer calls without a pass over samples.  The moments of a step's samples (linreg_moments.cuh) need no
+// parameters, and its gradient and loss follow from them in some two hundred operations.  So one block takes the steps, by
+// one wavefront, and the other blocks of the same launch draw and sum the samples of the steps that the next launch will
+// take.
+// What bounds it: the chain of about 160 fp64 instructions per step that one wavefront issues, 0.43 us; the losses are left
+// to as many lanes as there are steps, behind it.  Measured (us per call of 200 steps, linreg_steps_kernel / so): batch 256 175 /
+// 122, 1024 239 / 125, 2048 312 / 130, 4096 455 / 133, 8192 817 / 138; shorter calls at moments_take().
+using xad_linreg::Coefficients;
+using xad_linreg::kMoments;
+using xad_linreg::Twofold;
+constexpr int kPartLanes = 256;  // the lanes that sum one part of a step's batch ...
+constexpr int kPartPer = 4;      // ... at most so many samples each
+constexpr int kPartsPerBlock = kStepLanes / kPartLanes;
+
+struct MomentSteps {
+    const double* x1;
+    const double* x2;
+    const double* y;
+    std::uint64_t total, key;
+    double* params;
+    // the four parameters as the call found them: the moments are taken about a and c.  The first launch, which takes no steps,
+    // has them from params and keeps a copy.
+    const double* centre;
+    double* keep_centre;
+    int batch, parts, per;  // a batch is summed in `parts` parts of kPartLanes * per samples
+    // the steps of this launch: moments ([step][part][kMoments]), rates, where the mean losses go (or null)
+    const Twofold* moments;
+    int steps;
+    std::int64_t first_step;
+    double* history;
+    double rates[kStepsPerLaunch];
+    // what the other blocks sum up: the `coming` steps from first_coming on
+    Twofold* next_moments;
+    int coming;
+    std::int64_t first_coming;
+};
+
+__device__ __forceinline__ std::size_t row_of_draw(const MomentSteps& a, std::int64_t step, int i) {
+    const std::uint64_t draw = static_cast<std::uint64_t>(step) * static_cast<std::uint64_t>(a.batch) + static_cast<std::uint64_t>(i);
+    return static_cast<std::size_t>(xad_rng::bits(a.key, draw) % a.total);
+}
+
+__device__ __forceinline__ Twofold from_lane(Twofold t, int distance) {
+    return {__shfl_xor(t.hi, distance, 64), __shfl_xor(t.lo, distance, 64)};
+}
+
+// The moments of one part of a step's samples: summed per lane, then over the wavefront by a reduce-scatter (at each of four
+// steps a lane passes on half of its sums and adds the partner's copies of the others), then over the part's wavefronts.
+__device__ __forceinline__ void sum_part(const MomentSteps& a, int unit, Twofold (&waves)[kStepLanes / 64][16]) {
+    const int t = static_cast<int>(threadIdx.x) % kPartLanes, lane = t & 63;
+    const bool mine = unit < a.coming * a.parts;
+    const int step = mine ? unit / a.parts : 0, part = mine ? unit - step * a.parts : 0;
+    const double a0 = a.centre[0], c0 = a.centre[2];
+    double x1[kPartPer], x2[kPartPer], y[kPartPer];
+#pragma unroll
+    for (int u = 0; u < kPartPer; ++u) {
+        const int i = (part * a.per + u) * kPartLanes + t;
+        if (mine && u < a.per && i < a.batch) {
+            const std::size_t r = row_of_draw(a, a.first_coming + step, i);
+            x1[u] = a.x1[r];
+            x2[u] = a.x2[r];
+            y[u] = a.y[r];
+        }
+    }
+    Twofold s[16] = {};
+#pragma unroll
+    for (int u = 0; u < kPartPer; ++u)
+        if (mine && u < a.per && (part * a.per + u) * kPartLanes + t < a.batch)
+            xad_linreg::add_sample(s, x1[u], x2[u], y[u], a0, c0);
+#pragma unroll
+    for (int half = 8; half > 0; half /= 2) {
+        const bool upper = (lane & (half * 4)) != 0;
+#pragma unroll
+        for (int k = 0; k < half; ++k) {
+            const Twofold keep = upper ? s[k + half] : s[k], pass = upper ? s[k] : s[k + half];
+            s[k] = xad_linreg::plus(keep, from_lane(pass, half * 4));
+        }
+    }
+    s[0] = xad_linreg::plus(s[0], from_lane(s[0], 2));
+    s[0] = xad_linreg::plus(s[0], from_lane(s[0], 1));
+    if ((lane & 3) == 0) waves[threadIdx.x / 64][lane >> 2] = s[0];  // lane / 4: the sum that its choices above have led to
+    __syncthreads();
+    if (mine && t < kMoments) {
+        const Twofold* of = &waves[threadIdx.x / kPartLanes * (kPartLanes / 64)][t];
+        Twofold sum = of[0];
+#pragma unroll
+        for (int w = 1; w < kPartLanes / 64; ++w) sum = xad_linreg::plus(sum, of[w * 16]);
+        a.next_moments[(static_cast<std::size_t>(step) * a.parts + part) * kMoments + t] = xad_linreg::settled(sum);
+    }
+}
+
+// Gradient and loss of a step by the graph, sample by sample, for all lanes of the block: where the moments cannot tell
+// (values that are not finite, a loss below the rounding of what cancels in it).
+__device__ __forceinline__ void sums_by_graph(const MomentSteps& a, std::int64_t step, const double (&p)[4], double (&partial)[kStepLanes / 64][kWidth],
+                                           double (&sums)[kWidth]) {
+    if (p[0] != p[0] || p[1] != p[1] || p[2] != p[2] || p[3] != p[3]) {  // then so is every residual
+#pragma unroll
+        for (int k = 0; k < kWidth; ++k) sums[k] = __builtin_nan("");
+        return;
+    }
+    double mine[kWidth] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int i = static_cast<int>(threadIdx.x); i < a.batch; i += kStepLanes) {
+        const std::size_t r = row_of_draw(a, step, i);
+        Variable<1, double> pa(p[0]), pb(p[1]), pc(p[2]), pd(p[3]);
+        mine[4] += xad_linreg::run_loss_graph(pa, pb, pc, pd, a.x1[r], a.x2[r], a.y[r]);
+        mine[0] += pa.grad(0);
+        mine[1] += pb.grad(0);
+        mine[2] += pc.grad(0);
+        mine[3] += pd.grad(0);
+    }
+    __syncthreads();  // the previous call's readers are done
+#pragma unroll
+    for (int k = 0; k < kWidth; ++k) {
+        const double of_wave = accumulate::wave::sum(mine[k]);
+        if ((threadIdx.x & 63) == 0) partial[threadIdx.x / 64][k] = of_wave;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kWidth; ++k) {
+        sums[k] = 0.0;
+        for (int w = 0; w < kStepLanes / 64; ++w) sums[k] += partial[w][k];
+    }
+}
+
+__device__ __forceinline__ Twofold broadcast(Twofold t, int lane) {
+    return {accumulate::wave::read_lane(t.hi, lane), accumulate::wave::read_lane(t.lo, lane)};
+}
+
+__global__ void __launch_bounds__(kStepLanes) linreg_moment_steps_kernel(MomentSteps a) {
+    const int t = static_cast<int>(threadIdx.x);
+    if (blockIdx.x != 0) {
+        __shared__ Twofold waves[kStepLanes / 64][16];
+        sum_part(a, static_cast<int>(blockIdx.x - 1) * kPartsPerBlock + t / kPartLanes, waves);
+        return;
+    }
+    if (a.keep_centre && t < 4) a.keep_centre[t] = a.params[t];
+    if (a.steps <= 0) return;
+    __shared__ Twofold gram[kStepsPerLaunch][kMoments + 1];
+    __shared__ double rates[kStepsPerLaunch];
+    __shared__ double taken[kStepsPerLaunch + 1][4];  // the parameters that a step starts from, and behind the last one
+    __shared__ double partial[kStepLanes / 64][kWidth];
+    __shared__ int by_graph[kStepsPerLaunch];  // steps whose loss is left to the graph
+    __shared__ int reached;
+    for (int k = t; k < a.steps * (kMoments + 1); k += kStepLanes) {
+        const int step = k / (kMoments + 1), m = k - step * (kMoments + 1);
+        Twofold sum{static_cast<double>(a.batch), 0.0};
+        if (m < kMoments) {
+            const Twofold* of = a.moments + static_cast<std::size_t>(step) * a.parts * kMoments + m;
+            sum = of[0];
+            for (int p = 1; p < a.parts; ++p) sum = xad_linreg::plus(sum, of[p * kMoments]);
+            sum = xad_linreg::settled(sum);
+        }
+        gram[step][m] = sum;
+    }
+    if (t < 4) taken[0][t] = a.params[t];
+    if (t < kStepsPerLaunch) rates[t] = a.rates[t], by_graph[t] = 0;
+    const double a0 = a.centre[0], c0 = a.centre[2];
+    __syncthreads();
+    for (int step = 0; step < a.steps;) {
+        if (t < 64) {
+            // lane l < 4 has the row of u, v^2, v or 1
+            constexpr unsigned char kRows[4][5] = {{xad_linreg::kF0U, xad_linreg::kUU, xad_linreg::kUQ, xad_linreg::kUV, xad_linreg::kU},
+                                                   {xad_linreg::kF0Q, xad_linreg::kUQ, xad_linreg::kQQ, xad_linreg::kQV, xad_linreg::kQ},
+                                                   {xad_linreg::kF0V, xad_linreg::kUV, xad_linreg::kQV, xad_linreg::kQ, xad_linreg::kV},
+                                                   {xad_linreg::kF0, xad_linreg::kU, xad_linreg::kQ, xad_linreg::kV, kMoments}};
+            int at[5];
+#pragma unroll
+            for (int j = 0; j < 5; ++j) at[j] = t == 0 ? kRows[0][j] : (t == 1 ? kRows[1][j] : (t == 2 ? kRows[2][j] : kRows[3][j]));
+            double p[4] = {taken[step][0], taken[step][1], taken[step][2], taken[step][3]};
+            Twofold row[5];
+#pragma unroll
+            for (int j = 0; j < 5; ++j) row[j] = gram[step][at[j]];
+            const double batch = static_cast<double>(a.batch), share = 1.0 / batch;
+            double rate = rates[step];
+            for (int now = step; now < a.steps; ++now) {
+                const int next = now + 1 < a.steps ? now + 1 : now;
+                const Coefficients k(p, a0, c0);
+                const Twofold r = xad_linreg::residual_moment(row[0], row[1], row[2], row[3], row[4], k);
+#pragma unroll
+                for (int j = 0; j < 5; ++j) row[j] = gram[next][at[j]];
+                const double rate_next = rates[next];
+                double g[4];
+                xad_linreg::gradient(k, broadcast(r, 0), broadcast(r, 1), broadcast(r, 2), broadcast(r, 3), g);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) p[j] -= rate * xad_linreg::quotient(g[j], batch, share);
+                rate = rate_next;
+                if (t == 0) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) taken[now + 1][j] = p[j];
+                }
+            }
+            // What is not finite stays so.  The first step that such parameters came out of is for the graph to take.
+            static_assert(kStepsPerLaunch <= 64, "a lane for every step");
+            const bool lost = t >= step && t < a.steps &&
+                              !__builtin_isfinite((taken[t + 1][0] + taken[t + 1][1]) + (taken[t + 1][2] + taken[t + 1][3]));
+            const std::uint64_t any = accumulate::wave::ballot(lost);
+            if (t == 0) reached = any != 0 ? __builtin_ctzll(any) : a.steps;
+        }
+        __syncthreads();
+        step = reached;
+        if (step == a.steps) break;
+        const double p[4] = {taken[step][0], taken[step][1], taken[step][2], taken[step][3]};
+        double sums[kWidth];
+        sums_by_graph(a, a.first_step + step, p, partial, sums);
+        if (t < 4) taken[step + 1][t] = p[t] - a.rates[step] * (sums[t] / a.batch);
+        ++step;
+        __syncthreads();
+    }
+    if (a.history) {
+        if (t < a.steps) {
+            const double p[4] = {taken[t][0], taken[t][1], taken[t][2], taken[t][3]};
+            bool resolved = false;
+            const double loss = xad_linreg::batch_loss(gram[t], Coefficients(p, a0, c0), &resolved);
+            if (resolved) a.history[t] = loss / a.batch;
+            by_graph[t] = resolved ? 0 : 1;
+        }
+        __syncthreads();
+        for (int step = 0; step < a.steps; ++step) {
+            if (!by_graph[step]) continue;
+            const double p[4] = {taken[step][0], taken[step][1], taken[step][2], taken[step][3]};
+            double sums[kWidth];
+            sums_by_graph(a, a.first_step + step, p, partial, sums);
+            if (t == 0) a.history[step] = sums[4] / a.batch;
+        }
+    }
+    if (t < 4) a.params[t] = taken[a.steps][t];
 }
 
 int grid_for(std::size_t n, unsigned* blocks) {
@@ -353,6 +583,61 @@ int queue_serial_sgd(hipStream_t s, double* gathered, int per_launch, std::size_
     return XAD_OK;
 }
 
+// The same steps by linreg_moment_steps_kernel; `memory` is moment_sgd_bytes() of it.
+int parts_of(int batch, int per) { return (batch + kPartLanes * per - 1) / (kPartLanes * per); }
+
+// Samples per lane: as few as keep the parts of a launch's steps on compute units of their own, beside the one that takes
+// steps (20 steps of 1024 samples: 38 us a call with one, 43 with four).
+int samples_per_lane(int per_launch, int batch) {
+    int per = 1;
+    while (per < kPartPer && per_launch * parts_of(batch, per) > 255 * kPartsPerBlock) per *= 2;
+    return per;
+}
+
+std::size_t moment_sgd_bytes(int per_launch, int batch) {
+    // two launches' moments, and the parameters as the call found them
+    const std::size_t parts = static_cast<std::size_t>(parts_of(batch, samples_per_lane(per_launch, batch)));
+    return 2 * static_cast<std::size_t>(per_launch) * parts * kMoments * sizeof(Twofold) + 4 * sizeof(double);
+}
+
+int queue_moment_sgd(hipStream_t s, void* memory, int per_launch, std::size_t total, const double* x1, const double* x2,
+                     const double* y, double* params, int batch, int epochs, double lr_first, double lr_last, std::uint64_t seed,
+                     double* loss_history) {
+    const double decay = std::log(lr_last / lr_first) / epochs;
+    const int per = samples_per_lane(per_launch, batch), parts = parts_of(batch, per);
+    const std::size_t half = static_cast<std::size_t>(per_launch) * static_cast<std::size_t>(parts) * kMoments;
+    Twofold* const moments = static_cast<Twofold*>(memory);
+    double* const centre = reinterpret_cast<double*>(moments + 2 * half);
+    const std::int64_t launches = xad_linreg::step_launches(epochs, per_launch);
+    // launch k sums the samples of launch k + 1's steps; the first one does nothing else
+    for (std::int64_t k = -1; k < launches; ++k) {
+        const xad_linreg::StepLaunch l = xad_linreg::step_launch(k, epochs, per_launch);
+        MomentSteps a{};
+        a.x1 = x1, a.x2 = x2, a.y = y;
+        a.total = total, a.key = xad_rng::stream_key(seed, 0);
+        a.params = params;
+        a.centre = k < 0 ? params : centre;
+        a.keep_centre = k < 0 ? centre : nullptr;
+        a.batch = batch, a.parts = parts, a.per = per;
+        a.steps = l.steps;
+        if (l.steps > 0) {
+            a.moments = moments + static_cast<std::size_t>(k & 1) * half;
+            a.first_step = l.first;
+            a.history = loss_history ? loss_history + l.first : nullptr;
+            for (int e = 0; e < l.steps; ++e) a.rates[e] = lr_first * std::exp(decay * static_cast<double>(l.first + e));
+        }
+        if (l.gather > 0) {
+            a.next_moments = moments + static_cast<std::size_t>((k + 1) & 1) * half;
+            a.coming = l.gather;
+            a.first_coming = l.coming;
+        }
+        const int units = a.coming * a.parts;
+        linreg_moment_steps_kernel<<<dim3(1 + static_cast<unsigned>((units + kPartsPerBlock - 1) / kPartsPerBlock)), dim3(kStepLanes), 0, s>>>(a);
+        XAD_HIP_TRY(hipGetLastError());
+    }
+    return XAD_OK;
+}
+
 // Gradient sums of xad_linreg_sgd_f64_static: one copy of this array per device, for the life of
 // the process.  kWidth doubles are used; the size is the alignment unit.
 constexpr int kScratchDoubles = 32;
@@ -390,25 +675,34 @@ extern "C" int xad_linreg_sgd_f64(size_t total, const double* x1, const double* 
     XAD_REQUIRE(total > 0 && batch > 0 && epochs >= 0, "total, batch must be positive and epochs non-negative");
     XAD_REQUIRE(lr_first > 0.0 && lr_last > 0.0, "learning rates must be positive");
     hipStream_t s = xad::as_stream(stream);
-    // One block takes all steps where that is the faster way and there is memory for the gathered samples; otherwise two
-    // launches a step.
-    double* scratch_memory = nullptr;
+    // One block takes all steps where that is the faster way and there is memory for the gathered samples or their moments;
+    // otherwise two launches a step.
+    void* scratch_memory = nullptr;
     int per_launch = 0;
+    const bool by_moments = xad_linreg::moments_take(batch, epochs);
     if (xad_linreg::one_block_takes(batch, epochs)) {
         const std::size_t step_bytes = 3 * sizeof(double) * static_cast<std::size_t>(batch);
-        const std::size_t fit = kGatheredBytes / step_bytes;
+        const std::size_t fit = by_moments ? kStepsPerLaunch : kGatheredBytes / step_bytes;
         per_launch = static_cast<int>(fit < kStepsPerLaunch ? fit : kStepsPerLaunch);
         if (per_launch > epochs) per_launch = epochs;
-        if (hipMalloc(&scratch_memory, 2 * static_cast<std::size_t>(per_launch) * step_bytes) != hipSuccess) {
+        const std::size_t bytes = by_moments ? moment_sgd_bytes(per_launch, batch) : 2 * static_cast<std::size_t>(per_launch) * step_bytes;
+        if (hipMalloc(&scratch_memory, bytes) != hipSuccess) {
             (void)hipGetLastError();
             scratch_memory = nullptr;
         }
     }
-    const bool serial = scratch_memory != nullptr;
-    if (!serial) XAD_HIP_TRY(hipMalloc(&scratch_memory, kWidth * sizeof(double)));
-    const int status = serial ? queue_serial_sgd(s, scratch_memory, per_launch, total, x1, x2, y, params, batch, epochs, lr_first,
-                                                 lr_last, seed, loss_history)
-                              : queue_sgd(s, scratch_memory, total, x1, x2, y, params, batch, epochs, lr_first, lr_last, seed, loss_history);
+    int status = XAD_OK;
+    if (scratch_memory == nullptr) {
+        XAD_HIP_TRY(hipMalloc(&scratch_memory, kWidth * sizeof(double)));
+        status = queue_sgd(s, static_cast<double*>(scratch_memory), total, x1, x2, y, params, batch, epochs, lr_first, lr_last, seed,
+                           loss_history);
+    } else if (by_moments) {
+        status = queue_moment_sgd(s, scratch_memory, per_launch, total, x1, x2, y, params, batch, epochs, lr_first, lr_last, seed,
+                                  loss_history);
+    } else {
+        status = queue_serial_sgd(s, static_cast<double*>(scratch_memory), per_launch, total, x1, x2, y, params, batch, epochs,
+                                  lr_first, lr_last, seed, loss_history);
+    }
     const hipError_t waited = hipStreamSynchronize(s);
     const hipError_t freed = hipFree(scratch_memory);
     if (status != XAD_OK) return status;

@@ -18,6 +18,14 @@ inline bool one_block_takes(int batch, int epochs) {
     return batch <= kLargestSerialBatch && epochs > (batch <= kLargestSerialBatch / 4 ? 0 : (batch <= kLargestSerialBatch / 2 ? 1 : 2));
 }
 
+// Of the calls that one block takes, those whose steps it takes from moments of their samples.  A step is the quicker for
+// it, but a call begins and ends with more to do.  Measured (us per call of 4 / 8 / 12 / 16 steps, samples | moments): batch 256
+// 25.5 28.5 31.6 35.6 | 29.3 31.1 32.7 35.2, 1024 26.8 29.9 33.2 36.7 | 30.8 32.3 34.3 36.1, 2048 28.2 33.1 38.2 42.5 | 31.3
+// 33.9 35.8 37.2, 4096 32.1 39.9 83.6 93.1 | 34.8 36.8 38.7 40.2, 8192 39.3 89.5 103.9 117.3 | 39.2 41.2 43.0 44.8.
+inline bool moments_take(int batch, int epochs) {
+    return one_block_takes(batch, epochs) && epochs >= (batch <= 1024 ? 16 : (batch <= 2048 ? 10 : (batch <= 4096 ? 7 : 5)));
+}
+
 // Launch k of 0 .. step_launches() - 1 takes the steps first .. first + steps - 1 and gathers the samples of the `gather`
 // steps from `coming` on, those of launch k + 1; launch -1 does nothing but gather.
 struct StepLaunch {
