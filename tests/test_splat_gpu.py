@@ -19,8 +19,7 @@ from tests._scenes import one_gaussian, random_scene
 pytestmark = pytest.mark.gpu
 
 
-# For tests of what a call leaves behind (list capacities, status words): 256 tiles, whose lists are made by testing every tile,
-# and 2080, which is more than are, so that these go by way of supertiles.
+# For tests of what a call leaves behind (list capacities, status words): 256 tiles in 4 supertiles, and 2080 in 45.
 BOTH_BINNINGS = [(256, 256), (1040, 512)]
 
 
@@ -563,6 +562,31 @@ def test_tile_lists_equal_what_rectangles_and_depths_imply(gpu, oracle, G, W, H,
     ctx.forward(torch.from_numpy(params).to(gpu), torch.from_numpy(depth).to(gpu))
     _assert_lists(ctx, oracle, W, H, params, depth)
     ctx.close()
+
+
+@pytest.mark.parametrize("G,W,H,scale,within", [
+    (1024, 128, 128, (1.0, 5.0), None),      # one supertile, one block's entries exactly
+    (1025, 128, 128, (1.0, 5.0), None),      # and one more
+    (3000, 256, 256, (60.0, 90.0), None),    # rectangles over whole supertiles: more pairs than are put in order at a time
+    (40_000, 640, 400, (0.5, 1.5), 90.0),    # a cluster: more Gaussians than its supertile's own blocks take
+    (70_001, 1300, 80, (0.5, 3.0), None),    # two groups of supertiles, several slices of several ranges, a ragged end
+    (600_000, 4096, 4096, (0.3, 0.6), None), # more words than are kept at a time
+])
+def test_tile_lists_where_the_work_is_dealt_out_differently(gpu, oracle, G, W, H, scale, within):
+    import torch
+
+    from xyz_autodiff_cuda_amd import splat
+
+    params, depth = random_scene(G, W, H, seed=G, scale_px=scale)
+    if within is not None:  # all centres in a square of that side inside one supertile
+        params[0] = 16.0 + params[0] * np.float32(within / W)
+        params[1] = 16.0 + params[1] * np.float32(within / H)
+    depth[::7] = depth[0]
+    ctx = splat.SplatContext(W, H, G, depth_mode="static")
+    ctx.forward(torch.from_numpy(params).to(gpu), torch.from_numpy(depth).to(gpu))
+    _assert_lists(ctx, oracle, W, H, params, depth)
+    ctx.close()
+
 
 
 @pytest.mark.parametrize("G,W,H", [

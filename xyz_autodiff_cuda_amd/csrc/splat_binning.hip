@@ -4,28 +4,27 @@
 // The lists are a sparse transpose: Gaussian-major (a rectangle of tiles per Gaussian) to tile-major.
 // A comparison sort or a radix sort of (tile, Gaussian) pairs moves every pair several times; here a
 // pair is written once.  The Gaussians are walked in depth order, and what keeps each list in that
-// order is the walk itself, not a sort:
+// order is the walk itself, not a sort.  Two launches:
 //
-//   level A   Gaussians -> supertiles (8 x 8 tiles).  A wavefront takes a range of the depth-ordered
-//             Gaussians and 64 supertiles, one per lane.  64 Gaussians are loaded at a time, one per
-//             lane; the rectangle of each in turn is broadcast (v_readlane) and every lane tests its
-//             own supertile against it.  A first pass counts, the counts of all (supertile, range)
-//             cells are scanned in supertile-major order, and a second pass writes each Gaussian at
-//             its lane's cursor.  Ranges are visited in order inside every supertile, Gaussians in
-//             order inside every range: the list of a supertile comes out in depth order.
-//   level B   supertile -> its 64 tiles: a wavefront takes 64 entries of one supertile's list, one per
-//             lane.  The lane that loads a Gaussian forms the 64-bit mask of the tiles its rectangle
-//             covers inside the supertile (row mask x column multiplier).  Those 64 masks are a 64 x 64
-//             bit matrix, entries by tiles; it is transposed across the lanes in six exchange steps,
-//             after which lane t holds, for tile t, the mask of the entries that cover it: its
-//             population count is the tile's count, and its set bits, walked from the lowest, are the
-//             tile's Gaussians in list order.
+//   cover   A block takes a range of the depth-ordered Gaussians and a group of 64 x 64 tiles.  Every rectangle adds
+//           one to the corners of a table of differences (four LDS atomics however large it is), whose sums over rows
+//           and columns are the range's count for every tile of the group.  Besides, 64 Gaussians at a time, one per
+//           lane: the 64-bit mask of the group's supertiles (8 x 8 tiles each) that a rectangle reaches; the 64 masks
+//           are transposed across the lanes, after which lane s has a word that says which of the 64 reach supertile s.
+//   fill    A block takes a supertile and a slice of the Gaussians.  From the counts it knows where in each of its
+//           tiles' lists its entries begin.  The set bits of its words, in order, are the Gaussians it has to look at;
+//           64 at a time, one per lane: the mask of the supertile's tiles that a rectangle covers; transposed, lane t
+//           has the word that says which of the 64 cover tile t, and its set bits, in order, are written.
 //
-// Work per (Gaussian, supertile) pair is a handful of wavefront instructions; the stores of the final
-// lists are 4 bytes per pair, each pair once.  All sizes that depend on the data (pairs per
-// supertile, pairs in total) stay on the device: grids are sized by the capacity of the buffers, idle
-// wavefronts leave at once, every store is checked against the capacity, and an overflow is
-// recorded in the status words for the host to see whenever it next waits for the stream.
+// All sizes that depend on the data stay on the device, every store is checked against the capacity of the list, and an
+// overflow is recorded in the status words for the host to see whenever it next waits for the stream.
+//
+// What bounds it: latency, of a block's chain of loads, barriers and LDS accesses, 5 us a launch; with more Gaussians the
+// instructions of fill, most of them for putting pairs in order.  Measured (cover + fill, us; in parentheses as it was before:
+// two launches that tested every tile against every Gaussian in small scenes, seven by way of supertile lists in others):
+// 1000 Gaussians at 640 x 427 4.5 + 6.9 (8.6), 10 000 at 512 x 512 5.1 + 9.5 (22), 50 000 at 1277 x 719 5.5 + 13.4 (44), 100 000
+// at 1920 x 1080 7.3 + 15.4 (65), 200 000 at 2048 x 2048 9.3 + 21 (75).  With all centres within 100 pixels of the middle,
+// the whole of it between events: 15.9 (10.9), 22 (24), 43 (45), 30 (60), 40 (65).
 //
 // Replaces, for the tile-binned renderer, what the reference does not have at all: its renderer
 // visits every Gaussian at every pixel (examples/mini-gaussian-splatting/gaussian_splatting_kernel.cu:33-62).
@@ -41,169 +40,64 @@ namespace {
 
 using xyz_autodiff::accumulate::wave::ballot;
 
-__device__ __forceinline__ std::uint32_t read_lane(std::uint32_t v, int lane) {
-    return static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), lane));
-}
-
 // ---------------------------------------------------------------------------
-// Exclusive scan of n 32-bit counts, in place, in one launch (chained scan with decoupled look-back).
-// Blocks take tickets, so a block only ever waits for blocks that are already running.  The state
-// words carry the launch's epoch, so nothing has to be cleared between launches: a word of another
-// epoch simply is not there yet.  data[n] receives the total.
-// Tickets and epoch live in three control words on the device (tickets given out, blocks finished, epoch);
-// the block that finishes last puts the first two back to zero and moves the epoch on.  Nothing about
-// a launch depends on what the host knows of earlier launches, so a recorded launch can be replayed.
-enum : int { kScanTickets = 0, kScanFinished = 1, kScanEpoch = 2 };
-constexpr unsigned kScanBlock = 1024;
-constexpr unsigned kScanItems = 16;
-constexpr unsigned kScanTile = kScanBlock * kScanItems;  // few, large blocks: the chain of look-backs stays short
-
-__device__ __forceinline__ std::uint64_t scan_word(std::uint32_t epoch, std::uint32_t inclusive, std::uint32_t value) {
-    return (static_cast<std::uint64_t>((epoch << 1) | inclusive) << 32) | value;
+// The value of the lane whose number differs in bit kDistance.  Within a row of 16 lanes by DPP, which is in the
+// vector pipeline; a shuffle through LDS takes some hundred cycles, and there are chains of them here.
+template <int kControl, int kBanks>
+__device__ __forceinline__ std::uint32_t dpp(std::uint32_t old, std::uint32_t v) {
+    return static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(old), static_cast<int>(v), kControl, 0xF, kBanks, false));
+}
+template <int kDistance>
+__device__ __forceinline__ std::uint32_t from_partner(std::uint32_t v, int lane) {
+    if constexpr (kDistance == 16) {
+        // swaps the odd rows of one register with the even rows of the other
+        const auto rows = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return (lane & 16) ? rows[0] : rows[1];
+    }
+    if constexpr (kDistance == 8) return dpp<0x128, 0xF>(0, v);                       // row_ror:8
+    if constexpr (kDistance == 4) return dpp<0x114, 0xA>(dpp<0x104, 0x5>(0, v), v);   // row_shl:4 for banks 0 and 2, row_shr:4 for 1 and 3
+    if constexpr (kDistance == 2) return dpp<0x4E, 0xF>(0, v);                        // quad_perm [2,3,0,1]
+    return dpp<0xB1, 0xF>(0, v);                                                      // quad_perm [1,0,3,2]
 }
 
-__global__ void __launch_bounds__(kScanBlock) scan_kernel(std::uint32_t* __restrict__ data, std::uint32_t n,
-                                                          std::uint64_t* __restrict__ state, std::uint32_t* __restrict__ control) {
-    __shared__ std::uint32_t wave_total[kScanBlock / 64];
-    __shared__ std::uint32_t block_index, block_exclusive, launch_epoch;
-    const unsigned t = threadIdx.x;
-    if (t == 0) {
-        launch_epoch = __hip_atomic_load(control + kScanEpoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // before the ticket: it moves on only after every block has one
-        block_index = atomicAdd(control + kScanTickets, 1u);
-    }
-    __syncthreads();
-    const std::uint32_t b = block_index;
-    const std::uint32_t epoch = launch_epoch;
-    const std::uint32_t first = b * kScanTile + t * kScanItems;
-
-    std::uint32_t v[kScanItems];
-    if (first + kScanItems <= n) {
-#pragma unroll
-        for (unsigned k = 0; k < kScanItems; k += 4) {
-            const uint4 q = *reinterpret_cast<const uint4*>(data + first + k);
-            v[k] = q.x; v[k + 1] = q.y; v[k + 2] = q.z; v[k + 3] = q.w;
-        }
-    } else {
-#pragma unroll
-        for (unsigned k = 0; k < kScanItems; ++k) v[k] = first + k < n ? data[first + k] : 0u;
-    }
-    std::uint32_t mine = 0;
-#pragma unroll
-    for (unsigned k = 0; k < kScanItems; ++k) mine += v[k];
-
-    // inclusive scan of the per-thread sums: within each wavefront by shuffles, across the wavefronts through LDS
-    const unsigned lane = t & 63u, wave = t >> 6;
-    std::uint32_t inclusive_in_wave = mine;
-#pragma unroll
-    for (unsigned step = 1; step < 64; step *= 2) {
-        const std::uint32_t other = __shfl_up(inclusive_in_wave, step, 64);
-        if (lane >= step) inclusive_in_wave += other;
-    }
-    if (lane == 63) wave_total[wave] = inclusive_in_wave;
-    __syncthreads();
-    std::uint32_t before_wave = 0, aggregate = 0;
-#pragma unroll
-    for (unsigned w = 0; w < kScanBlock / 64; ++w) {
-        const std::uint32_t total = wave_total[w];
-        before_wave += w < wave ? total : 0u;
-        aggregate += total;
-    }
-    const std::uint32_t thread_exclusive = before_wave + inclusive_in_wave - mine;
-
-    // Look-back, by the block's first wavefront: 64 predecessors at a time, nearest first.  Each lane waits
-    // for its predecessor's word of this epoch (that block holds an earlier ticket, so it is running),
-    // the sums up to and including the nearest inclusive prefix are added, and if there was none among
-    // the 64 the next 64 are looked at.  Lanes that would reach before block 0 count as an inclusive zero.
-    if (t < 64) {
-        if (b > 0 && t == 0) __hip_atomic_store(state + b, scan_word(epoch, 0u, aggregate), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        std::uint32_t exclusive = 0;
-        for (std::int64_t nearest = static_cast<std::int64_t>(b) - 1; nearest >= 0; nearest -= 64) {
-            const std::int64_t mine_at = nearest - static_cast<std::int64_t>(t);
-            std::uint64_t word = scan_word(epoch, 1u, 0u);
-            if (mine_at >= 0) {
-                do {
-                    word = __hip_atomic_load(state + mine_at, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-                } while (static_cast<std::uint32_t>(word >> 33) != epoch);
-            }
-            const std::uint64_t inclusive = ballot(((word >> 32) & 1u) != 0);
-            const unsigned stop = static_cast<unsigned>(__builtin_ctzll(inclusive | (std::uint64_t(1) << 63)));
-            std::uint32_t part = t <= stop ? static_cast<std::uint32_t>(word) : 0u;
-            for (int offset = 32; offset > 0; offset >>= 1) part += __shfl_xor(part, offset, 64);
-            exclusive += part;
-            if (inclusive != 0) break;
-        }
-        if (t == 0) {
-            __hip_atomic_store(state + b, scan_word(epoch, 1u, exclusive + aggregate), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-            block_exclusive = exclusive;
-            if (static_cast<std::uint64_t>(b + 1) * kScanTile >= n) data[n] = exclusive + aggregate;  // the last block: the total
-        }
-    }
-    __syncthreads();
-
-    std::uint32_t running = block_exclusive + thread_exclusive;
-    if (first + kScanItems <= n) {
-#pragma unroll
-        for (unsigned k = 0; k < kScanItems; k += 4) {
-            uint4 q;
-            q.x = running; running += v[k];
-            q.y = running; running += v[k + 1];
-            q.z = running; running += v[k + 2];
-            q.w = running; running += v[k + 3];
-            *reinterpret_cast<uint4*>(data + first + k) = q;
-        }
-    } else {
-#pragma unroll
-        for (unsigned k = 0; k < kScanItems; ++k) {
-            if (first + k < n) data[first + k] = running;
-            running += v[k];
-        }
-    }
-    // the block that finishes last leaves the control words ready for the next launch (epoch 0 is never
-    // used: the state words start out as zero)
-    if (t == 0 && atomicAdd(control + kScanFinished, 1u) == gridDim.x - 1) {
-        const std::uint32_t next = (epoch + 1) & 0x3fffffffu;
-        control[kScanTickets] = 0;
-        control[kScanFinished] = 0;
-        control[kScanEpoch] = next == 0 ? 1u : next;
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Transpose of a 64 x 64 bit matrix held one row per lane (lo = columns 0..31, hi = columns 32..63):
 // afterwards lane t holds column t, bit j of it being bit t of lane j's row.  The usual recursive block
 // swap: at distance k, the lanes whose bit k is clear keep their columns with bit k clear and receive,
 // into their columns with bit k set, the partner's columns with bit k clear; the others the reverse.
+template <int kDistance>
+__device__ __forceinline__ void exchange_blocks(std::uint32_t& lo, std::uint32_t& hi, int lane) {
+    constexpr std::uint32_t kClear = kDistance == 16 ? 0x0000ffffu
+                                   : kDistance == 8  ? 0x00ff00ffu
+                                   : kDistance == 4  ? 0x0f0f0f0fu
+                                   : kDistance == 2  ? 0x33333333u
+                                                     : 0x55555555u;
+    const std::uint32_t other_lo = from_partner<kDistance>(lo, lane), other_hi = from_partner<kDistance>(hi, lane);
+    const bool set = (lane & kDistance) != 0;
+    // rotated, so that the partner's columns lie where they go to
+    const int by = set ? kDistance : 32 - kDistance;
+    const std::uint32_t keep = set ? ~kClear : kClear;
+    lo = (lo & keep) | (__builtin_amdgcn_alignbit(other_lo, other_lo, by) & ~keep);
+    hi = (hi & keep) | (__builtin_amdgcn_alignbit(other_hi, other_hi, by) & ~keep);
+}
 __device__ __forceinline__ void transpose_64x64(std::uint32_t& lo, std::uint32_t& hi, int lane) {
-    {
-        const std::uint32_t other_lo = __shfl_xor(lo, 32, 64), other_hi = __shfl_xor(hi, 32, 64);
-        if (lane & 32)
-            lo = other_hi;
-        else
-            hi = other_lo;
-    }
-    constexpr std::uint32_t kClear[5] = {0x0000ffffu, 0x00ff00ffu, 0x0f0f0f0fu, 0x33333333u, 0x55555555u};
-#pragma unroll
-    for (int step = 0; step < 5; ++step) {
-        const int k = 16 >> step;
-        const std::uint32_t m = kClear[step];
-        const std::uint32_t other_lo = __shfl_xor(lo, k, 64), other_hi = __shfl_xor(hi, k, 64);
-        if (lane & k) {
-            lo = ((other_lo >> k) & m) | (lo & ~m);
-            hi = ((other_hi >> k) & m) | (hi & ~m);
-        } else {
-            lo = (lo & m) | ((other_lo & m) << k);
-            hi = (hi & m) | ((other_hi & m) << k);
-        }
-    }
+    const auto halves = __builtin_amdgcn_permlane32_swap(lo, hi, false, false);  // the upper lanes' lo for the lower lanes' hi
+    lo = halves[0];
+    hi = halves[1];
+    exchange_blocks<16>(lo, hi, lane);
+    exchange_blocks<8>(lo, hi, lane);
+    exchange_blocks<4>(lo, hi, lane);
+    exchange_blocks<2>(lo, hi, lane);
+    exchange_blocks<1>(lo, hi, lane);
 }
 
-// ---------------------------------------------------------------------------
-// Both levels turn 64 rectangles into 64 lists the same way.  Lane = rectangle: the 8 x 8 cells it covers,
-// as a 64-bit mask (cell = 8 row + column).  After the transpose, lane = cell, and the mask says which of
-// the 64 rectangles cover it: its population count is the cell's count, its set bits, from the lowest, are
-// the cell's members in order.
+// The words of 64 masks, one per lane: bit j of lane t's is bit t of lane j's mask.
+__device__ __forceinline__ std::uint64_t transposed(std::uint64_t mask, int lane) {
+    std::uint32_t lo = static_cast<std::uint32_t>(mask), hi = static_cast<std::uint32_t>(mask >> 32);
+    transpose_64x64(lo, hi, lane);
+    return static_cast<std::uint64_t>(hi) << 32 | lo;
+}
 
-// Bits x0..x1 of every row y0..y1 (all within 0..7; empty if a range is).
+// Bits x0..x1 of every row y0..y1 of an 8 x 8 block of cells (all within 0..7; empty if a range is).
 __device__ __forceinline__ std::uint64_t block_mask(int x0, int x1, int y0, int y1) {
     if (x0 > x1 || y0 > y1) return 0;
     const std::uint64_t row = ((std::uint64_t(1) << (x1 - x0 + 1)) - 1) << x0;
@@ -211,60 +105,27 @@ __device__ __forceinline__ std::uint64_t block_mask(int x0, int x1, int y0, int 
     return row * rows;  // the multiplier has one bit per row: no carries
 }
 
-// Writes the members of every lane's mask (lane j's value `id` for bit j) to out[from ...], lane by lane.
-// One entry per lane and turn would scatter every store over 64 cache lines.  The entries go through LDS
-// instead: lane t puts its run at [before, before + count) there, and the runs are written out with
-// consecutive lanes on consecutive entries of a run (a window of LDS at a time).  Stores at or beyond
-// `capacity` are dropped.  Returns the lane's count.  Every lane of the wavefront must call it.
-constexpr std::uint32_t kStageEntries = 1024;
-struct RunStage {
-    std::uint32_t staged[kStageEntries];
-    std::uint32_t run_begin[65];
-    std::uint32_t run_dest[64];
-};
+__device__ __forceinline__ int at_least(int x, int lo) { return x > lo ? x : lo; }
+__device__ __forceinline__ int at_most(int x, int hi) { return x < hi ? x : hi; }
 
-__device__ __forceinline__ std::uint32_t write_runs(RunStage& lds, std::uint64_t mine, std::uint32_t id, std::uint32_t from,
-                                                    std::uint32_t* __restrict__ out, std::uint32_t capacity, int lane) {
-    const std::uint32_t count = static_cast<std::uint32_t>(__builtin_popcountll(mine));
-    std::uint32_t inclusive = count;
-#pragma unroll
-    for (int step = 1; step < 64; step *= 2) {
-        const std::uint32_t other = __shfl_up(inclusive, step, 64);
-        if (lane >= step) inclusive += other;
-    }
-    const std::uint32_t total = read_lane(inclusive, 63);
-    std::uint32_t next = inclusive - count;  // where this lane's next entry goes
-    __syncthreads();                         // the previous call's readers are done
-    lds.run_begin[lane] = next;
-    if (lane == 63) lds.run_begin[64] = total;
-    lds.run_dest[lane] = from;
-    for (std::uint32_t window = 0; window < total; window += kStageEntries) {
-        // every lane stays in the loop until the last one is done: the exchange below reads other lanes' registers
-        while (ballot(mine != 0 && next < window + kStageEntries) != 0) {
-            const bool has = mine != 0 && next < window + kStageEntries;
-            const int j = has ? __builtin_ctzll(mine) : 0;
-            const std::uint32_t member = __shfl(id, j, 64);
-            if (has) {
-                lds.staged[next - window] = member;
-                ++next;
-                mine &= mine - 1;
-            }
-        }
-        __syncthreads();
-        const std::uint32_t end = total - window < kStageEntries ? total - window : kStageEntries;
-        for (std::uint32_t e = static_cast<std::uint32_t>(lane); e < end; e += 64) {
-            const std::uint32_t at = window + e;
-            int t = 0;  // the run `at` lies in: the last one that begins at or before it (empty runs begin where the next one does)
-#pragma unroll
-            for (int step = 32; step > 0; step >>= 1)
-                if (lds.run_begin[t + step] <= at) t += step;
-            const std::uint32_t dest = lds.run_dest[t] + (at - lds.run_begin[t]);
-            if (dest < capacity) out[dest] = lds.staged[e];
-        }
-        __syncthreads();
-    }
-    return count;
+// Inclusive sums over the lanes of a row of 16, or of the wavefront, from the lowest.
+__device__ __forceinline__ std::uint32_t running_sum_of_row(std::uint32_t v) {
+    v += dpp<0x111, 0xF>(0, v);  // row_shr:1, 2, 4, 8
+    v += dpp<0x112, 0xF>(0, v);
+    v += dpp<0x114, 0xF>(0, v);
+    v += dpp<0x118, 0xF>(0, v);
+    return v;
 }
+__device__ __forceinline__ std::uint32_t running_sum(std::uint32_t v) {
+    v = running_sum_of_row(v);
+    v += static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x142, 0xA, 0xF, false));  // row_bcast:15 into rows 1 and 3
+    v += static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x143, 0xC, 0xF, false));  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+__device__ __forceinline__ std::uint32_t read_lane(std::uint32_t v, int lane) {
+    return static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), lane));
+}
+__device__ __forceinline__ std::uint32_t last_lane(std::uint32_t v) { return read_lane(v, 63); }
 
 // Supertiles are numbered group by group, a group being 8 x 8 supertiles (row-major within the group,
 // groups row-major over the image); numbers whose supertile lies beyond the image stay empty.
@@ -282,190 +143,376 @@ __device__ __forceinline__ SuperCoords super_coords(const BinPlan& p, int s) {
 }
 
 // ---------------------------------------------------------------------------
-// Level A.  One wavefront per block; block = (range of Gaussians) x (group of 8 x 8 supertiles), blocks of
-// one range adjacent so that they read the same rectangles from the same L2.  64 Gaussians at a time:
-// lane = Gaussian, mask = the group's supertiles its rectangle reaches; transposed, lane = supertile.
-// kFill = false: matrix_a[supertile * ranges_a + range] = number of Gaussians of the range that
-// touch the supertile.  kFill = true: matrix_a holds the scanned counts; the Gaussians are written.
-// rects_by_depth[i] is the rectangle of Gaussian by_depth[i]: both loads of a lane are independent and coalesced.
-template <bool kFill>
-__global__ void __launch_bounds__(64) super_kernel(BinPlan p, const std::uint32_t* __restrict__ by_depth,
-                                                   const TileRect* __restrict__ rects_by_depth,
-                                                   std::uint32_t* __restrict__ matrix_a, std::uint32_t* __restrict__ list_a) {
-    __shared__ RunStage stage;
-    const int lane = static_cast<int>(threadIdx.x);
+// rects_by_depth[i] is the rectangle of Gaussian by_depth[i].
+// kCount: counts[range][supertile][tile]; their sums per supertile, totals[supertile], and the Gaussians that reach it,
+// totals[supers + supertile] (all zero before).
+// kWords: covering[supertile][chunk - first_chunk] for the chunks (of 64 Gaussians) of the blocks' ranges, the first of
+// which is first_chunk's.
+constexpr int kGroupTiles = 64;   // tiles across a group
+
+constexpr int kCoverWaves = 16;
+constexpr int kCoverAtOnce = 64;  // chunks whose words are put together in LDS
+
+template <bool kCount, bool kWords>
+__global__ void __launch_bounds__(64 * kCoverWaves) cover_kernel(BinPlan p, int first_chunk, const TileRect* __restrict__ rects_by_depth,
+                                                                 std::uint64_t* __restrict__ covering,
+                                                                 std::uint32_t* __restrict__ counts, std::uint32_t* __restrict__ totals) {
+    __shared__ std::uint64_t words[kWords ? kCoverAtOnce : 1][65];
+    __shared__ std::uint32_t corners[kCount ? kGroupTiles + 1 : 1][kGroupTiles + 1];
+    __shared__ std::uint32_t above[kCoverWaves][kGroupTiles];
+    __shared__ std::uint32_t half[kCoverWaves][8];
+    __shared__ std::uint32_t reached[64];
+    const int t = static_cast<int>(threadIdx.x), lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int group = static_cast<int>(blockIdx.x % static_cast<unsigned>(p.groups));
-    const int range = static_cast<int>(blockIdx.x / static_cast<unsigned>(p.groups));
-    const int origin_x = (group % p.group_x) * 8, origin_y = (group / p.group_x) * 8;  // in supertiles
-    const std::size_t cell = static_cast<std::size_t>(group * 64 + lane) * p.ranges_a + range;
-    std::uint32_t cursor = kFill ? matrix_a[cell] : 0u;
-    std::uint32_t count = 0;
-
-    const int first = range * p.range_a;
-    const int last = first + p.range_a < p.G ? first + p.range_a : p.G;
-    for (int base = first; base < last; base += 64) {
-        const int i = base + lane;
-        std::uint32_t g = 0;
-        std::uint64_t mask = 0;
-        if (i < last) {
-            g = by_depth[i];
-            const TileRect rc = rects_by_depth[i];
-            if (rc.x0 <= rc.x1) {
-                const int x0 = (rc.x0 >> 3) - origin_x, x1 = (rc.x1 >> 3) - origin_x;
-                const int y0 = (rc.y0 >> 3) - origin_y, y1 = (rc.y1 >> 3) - origin_y;
-                mask = block_mask(x0 > 0 ? x0 : 0, x1 < 7 ? x1 : 7, y0 > 0 ? y0 : 0, y1 < 7 ? y1 : 7);
+    const int range = first_chunk / p.range_chunks + static_cast<int>(blockIdx.x / static_cast<unsigned>(p.groups));
+    const int origin_x = (group % p.group_x) * kGroupTiles, origin_y = (group / p.group_x) * kGroupTiles;
+    if constexpr (kCount) {
+        for (int k = t; k < (kGroupTiles + 1) * (kGroupTiles + 1); k += 64 * kCoverWaves) (&corners[0][0])[k] = 0;
+        if (t < 64) reached[t] = 0;
+        __syncthreads();
+    }
+    const int first = range * p.range_chunks, last = at_most(first + p.range_chunks, p.chunks);
+    for (int base = first; base < last; base += kCoverAtOnce) {
+        constexpr int kEach = kCoverAtOnce / kCoverWaves;
+        TileRect rects[kEach];
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) {
+            const int chunk = base + k * kCoverWaves + wave, i = chunk * 64 + lane;
+            rects[k] = TileRect{1, 1, 0, 0};  // covers nothing
+            if (chunk < last && i < p.G) rects[k] = rects_by_depth[i];
+        }
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) {
+            const int chunk = base + k * kCoverWaves + wave;
+            if (chunk >= last) break;  // the same for the wavefront
+            const int x0 = at_least(rects[k].x0 - origin_x, 0), x1 = at_most(rects[k].x1 - origin_x, kGroupTiles - 1);
+            const int y0 = at_least(rects[k].y0 - origin_y, 0), y1 = at_most(rects[k].y1 - origin_y, kGroupTiles - 1);
+            const bool reaches = x0 <= x1 && y0 <= y1;
+            if constexpr (kCount) {
+                if (reaches) {
+                    atomicAdd(&corners[y0][x0], 1u);
+                    atomicAdd(&corners[y0][x1 + 1], ~0u);
+                    atomicAdd(&corners[y1 + 1][x0], ~0u);
+                    atomicAdd(&corners[y1 + 1][x1 + 1], 1u);
+                }
+            }
+            const std::uint64_t word = transposed(reaches ? block_mask(x0 >> 3, x1 >> 3, y0 >> 3, y1 >> 3) : 0, lane);
+            if constexpr (kWords) words[chunk - base][lane] = word;
+            if constexpr (kCount)
+                if (word != 0) atomicAdd(&reached[lane], static_cast<std::uint32_t>(__builtin_popcountll(word)));
+        }
+        if constexpr (kWords) {
+            __syncthreads();
+            // a wavefront writes the words of four supertiles, consecutive lanes those of consecutive chunks
+            for (int s = wave; s < 64; s += kCoverWaves)
+                if (base + lane < last)
+                    covering[static_cast<std::size_t>(group * 64 + s) * p.slab_chunks + (base + lane - first_chunk)] = words[lane][s];
+            __syncthreads();
+        }
+    }
+    if constexpr (kCount) {
+        __syncthreads();
+        // sums down the columns, a lane a column: four rows of its own, then the wavefronts above; then along the rows
+        constexpr int kRows = kGroupTiles / kCoverWaves;
+        std::uint32_t v[kRows], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kRows; ++k) {
+            sum += corners[wave * kRows + k][lane];
+            v[k] = sum;
+        }
+        above[wave][lane] = sum;
+        __syncthreads();
+        std::uint32_t before = 0;
+        for (int w = 0; w < wave; ++w) before += above[w][lane];
+        std::uint32_t in_column = 0;
+#pragma unroll
+        for (int k = 0; k < kRows; ++k) {
+            v[k] = running_sum(v[k] + before);
+            const int row = wave * kRows + k;
+            const int super = group * 64 + (row >> 3) * 8 + (lane >> 3), tile = (row & 7) * 8 + (lane & 7);
+            counts[(static_cast<std::size_t>(range) * p.supers + super) * 64 + tile] = v[k];
+            in_column += v[k];
+        }
+        // of the eight columns of a supertile, then of its two fours of rows
+        in_column += from_partner<1>(in_column, lane);
+        in_column += from_partner<2>(in_column, lane);
+        in_column += from_partner<4>(in_column, lane);
+        static_assert(2 * kRows == 8, "two wavefronts have a supertile's rows");
+        if ((lane & 7) == 0) half[wave][lane >> 3] = in_column;
+        __syncthreads();
+        if (t < 64) {
+            const std::uint32_t sum_of_super = half[(t >> 3) * 2][t & 7] + half[(t >> 3) * 2 + 1][t & 7];
+            if (sum_of_super != 0) {
+                atomicAdd(totals + group * 64 + t, sum_of_super);
+                atomicAdd(totals + p.supers + group * 64 + t, reached[t]);
             }
         }
-        std::uint32_t lo = static_cast<std::uint32_t>(mask), hi = static_cast<std::uint32_t>(mask >> 32);
-        transpose_64x64(lo, hi, lane);  // now: which of the 64 Gaussians reach this lane's supertile
-        const std::uint64_t mine = (static_cast<std::uint64_t>(hi) << 32) | lo;
-        if constexpr (kFill) {
-            cursor += write_runs(stage, mine, g, cursor, list_a, p.capacity_a, lane);
-        } else {
-            count += static_cast<std::uint32_t>(__builtin_popcountll(mine));
-        }
-    }
-    if constexpr (!kFill) matrix_a[cell] = count;
-}
-
-// ---------------------------------------------------------------------------
-// Between the levels: how many wavefronts every supertile's list needs at level B (at least one, so
-// that every tile gets its range written), as a prefix over the supertiles, clamped to the grid that
-// will be launched.  One block.  Also records the number of (supertile, Gaussian) pairs and whether
-// they fit, and clears the tile ranges (tiles that no wavefront reaches keep an empty range).
-__global__ void __launch_bounds__(256) plan_kernel(BinPlan p, const std::uint32_t* __restrict__ offsets_a,
-                                                   std::uint32_t* __restrict__ first_wave, std::uint32_t* __restrict__ tile_ranges,
-                                                   std::uint32_t* __restrict__ status, bool clear_depth_flag) {
-    __shared__ std::uint32_t shared[256];
-    __shared__ std::uint32_t carried;
-    const unsigned t = threadIdx.x;
-    for (std::size_t k = static_cast<std::size_t>(blockIdx.x) * 256 + t; k < static_cast<std::size_t>(p.tiles_x) * p.tiles_y * 2;
-         k += static_cast<std::size_t>(gridDim.x) * 256)
-        tile_ranges[k] = 0;
-    if (blockIdx.x != 0) return;
-    if (t == 0) carried = 0;
-    __syncthreads();
-    for (int base = 0; base < p.supers; base += 256) {
-        const int s = base + static_cast<int>(t);
-        std::uint32_t waves = 0;
-        if (s < p.supers && super_coords(p, s).inside) {
-            std::uint32_t begin = offsets_a[static_cast<std::size_t>(s) * p.ranges_a];
-            std::uint32_t end = offsets_a[static_cast<std::size_t>(s + 1) * p.ranges_a];
-            begin = begin < p.capacity_a ? begin : p.capacity_a;
-            end = end < p.capacity_a ? end : p.capacity_a;
-            waves = (end - begin + kBinRangeB - 1) / kBinRangeB;
-            if (waves == 0) waves = 1;
-        }
-        shared[t] = waves;
-        __syncthreads();
-        for (unsigned step = 1; step < 256; step *= 2) {
-            const std::uint32_t other = t >= step ? shared[t - step] : 0u;
-            __syncthreads();
-            shared[t] += other;
-            __syncthreads();
-        }
-        const std::uint32_t exclusive = carried + shared[t] - waves;
-        if (s < p.supers) first_wave[s] = exclusive < p.waves_b ? exclusive : p.waves_b;
-        __syncthreads();
-        if (t == 255) carried += shared[255];
-        __syncthreads();
-    }
-    if (t == 0) {
-        first_wave[p.supers] = carried < p.waves_b ? carried : p.waves_b;
-        const std::uint32_t super_pairs = offsets_a[static_cast<std::size_t>(p.supers) * p.ranges_a];
-        status[kStatusSuperPairs] = super_pairs;
-        // this step's verdict starts here; the last kernel of the binning may still raise it
-        const bool overflow = super_pairs > p.capacity_a || carried > p.waves_b;
-        status[kStatusOverflow] = overflow ? 1u : 0u;
-        // the sticky word keeps the largest room any step would have needed (never zero for a step that overflowed)
-        if (overflow) atomicMax(status + kStatusOverflowSticky, super_pairs > 0 ? super_pairs : 1u);
-        if (clear_depth_flag) status[kStatusDepthChanged] = 0;  // the projection of this step has set it, the host has its copy
     }
 }
 
 // ---------------------------------------------------------------------------
-// Level B.  One wavefront per block: wavefront w serves entries [64 q, 64 q + 64) of the list of supertile s,
-// where first_wave[s] <= w < first_wave[s + 1] and q = w - first_wave[s]; after the transpose, lane = tile of
-// the supertile (row-major, 8 per row).  The counts of supertile s live at
-// matrix_b[64 first_wave[s] + tile * waves_of_s + q]: scanned as one flat array, that order puts every
-// tile's pieces next to each other and the tiles of a supertile one after the other, so the scanned
-// value is the position in the final list.  Wavefronts beyond the last supertile clear their 64 cells
-// and leave.
-template <bool kFill>
-__global__ void __launch_bounds__(64) tile_kernel(BinPlan p, const std::uint32_t* __restrict__ offsets_a,
-                                                  const std::uint32_t* __restrict__ first_wave,
-                                                  const std::uint32_t* __restrict__ list_a, const TileRect* __restrict__ rects,
-                                                  std::uint32_t* __restrict__ matrix_b, std::uint32_t* __restrict__ list,
-                                                  std::uint32_t* __restrict__ range_begin, std::uint32_t* __restrict__ range_end,
-                                                  std::uint32_t* __restrict__ status) {
-    __shared__ RunStage stage;
-    const int lane = static_cast<int>(threadIdx.x);
-    const std::uint32_t w = blockIdx.x;
-    const std::uint32_t used = first_wave[p.supers];
-    if (w >= used) {
-        if constexpr (!kFill) matrix_b[static_cast<std::size_t>(w) * 64 + lane] = 0;
-        return;
-    }
-    // the last supertile whose first wavefront is not after w
-    int s = 0;
-    for (int hi = p.supers; hi - s > 1;) {
-        const int mid = (s + hi) / 2;
-        if (first_wave[mid] <= w)
-            s = mid;
-        else
-            hi = mid;
-    }
-    const std::uint32_t wave0 = first_wave[s], waves = first_wave[s + 1] - wave0, q = w - wave0;
-    std::uint32_t begin = offsets_a[static_cast<std::size_t>(s) * p.ranges_a];
-    std::uint32_t end = offsets_a[static_cast<std::size_t>(s + 1) * p.ranges_a];
-    begin = begin < p.capacity_a ? begin : p.capacity_a;
-    end = end < p.capacity_a ? end : p.capacity_a;
-    const std::uint32_t i = begin + q * kBinRangeB + static_cast<std::uint32_t>(lane);
+constexpr int kFillWaves = 8;
+constexpr int kFillLanes = 64 * kFillWaves;
+constexpr int kFillGroups = 16;  // groups of 64 entries taken together
+constexpr int kFillWords = kSliceChunks / kFillLanes;  // a lane's, at most
+constexpr int kStagedPairs = 8192;
 
+struct FillLds {
+    std::uint32_t part_all[kFillWaves][64], part_before[kFillWaves][64];
+    std::uint32_t cursor[64];                 // where the tiles' next entries go
+    std::uint32_t entry[kFillGroups * 64];    // positions in the depth order, then the Gaussians there
+    std::uint32_t count_of[kFillGroups][64];  // [group of entries][tile]
+    std::uint32_t to_list[64];
+    std::uint16_t staged[kStagedPairs];
+    std::uint32_t hits_of_wave[kFillWaves], before_of_wave[kFillWaves];
+};
+
+// Calls f(bit) for the set bits of a word, from the lowest (half a word at a time: the loop is a third shorter).
+template <typename F>
+__device__ __forceinline__ void for_each_bit(std::uint64_t word, F f) {
+    for (std::uint32_t todo = static_cast<std::uint32_t>(word); todo != 0; todo &= todo - 1) f(__builtin_ctz(todo));
+    for (std::uint32_t todo = static_cast<std::uint32_t>(word >> 32); todo != 0; todo &= todo - 1) f(32 + __builtin_ctz(todo));
+}
+
+struct FillArgs {
+    BinPlan p;
+    int first_chunk;  // of the slab of words in `covering`
+    int slab_ranges;  // ranges in it
+    const std::uint32_t* by_depth;
+    const TileRect* rects_by_depth;
+    const std::uint64_t* covering;
+    const std::uint32_t* counts;
+    const std::uint32_t* totals;
+    std::uint32_t* list;
+    std::uint32_t* range_begin;
+    std::uint32_t* range_end;
+    std::uint32_t* status;
+    bool clear_depth_flag;
+};
+
+// The entries that `ranges` ranges from first_range on have in the lists of supertile s, by a block; nothing if more than
+// `most` Gaussians reach it.
+__device__ __forceinline__ void fill_lists(const FillArgs& a, int s, int first_range, int ranges, std::uint32_t most, FillLds& lds) {
+    const BinPlan& p = a.p;
+    int t = static_cast<int>(threadIdx.x);
+    asm volatile("" : "+v"(t));  // nothing that depends on the lane is to be kept in registers from item to item
+    const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const SuperCoords where = super_coords(p, s);
-    const int base_x = where.x * 8, base_y = where.y * 8;
-    std::uint32_t g = 0, mask_lo = 0, mask_hi = 0;
-    if (i < end) {
-        g = list_a[i];
-        const TileRect rc = rects[g];
-        const std::uint64_t mask = block_mask(rc.x0 - base_x > 0 ? rc.x0 - base_x : 0, rc.x1 - base_x < 7 ? rc.x1 - base_x : 7,
-                                              rc.y0 - base_y > 0 ? rc.y0 - base_y : 0, rc.y1 - base_y < 7 ? rc.y1 - base_y : 7);
-        mask_lo = static_cast<std::uint32_t>(mask);
-        mask_hi = static_cast<std::uint32_t>(mask >> 32);
+    // these ranges' words, in order: the wavefronts have equal shares, a lane a word or two of its wavefront's
+    const int words_first = first_range * p.range_chunks, words_last = at_most(words_first + ranges * p.range_chunks, p.chunks);
+    const int share = (words_last - words_first + kFillWaves - 1) / kFillWaves, my_first = words_first + wave * share;
+    std::uint64_t mine[kFillWords] = {};
+#pragma unroll
+    for (int k = 0; k < kFillWords; ++k) {
+        const int of_share = k * 64 + lane;
+        if (of_share < share && my_first + of_share < words_last)
+            mine[k] = a.covering[static_cast<std::size_t>(s) * p.slab_chunks + (my_first + of_share - a.first_chunk)];
     }
-    transpose_64x64(mask_lo, mask_hi, lane);  // now: which of the 64 entries cover this lane's tile
-    const int tx = base_x + (lane & 7), ty = base_y + (lane >> 3);
-    const bool owner = tx < p.tiles_x && ty < p.tiles_y;
-    std::uint64_t mine = owner ? (static_cast<std::uint64_t>(mask_hi) << 32) | mask_lo : 0;
-    const std::size_t cell = static_cast<std::size_t>(wave0) * 64 + static_cast<std::size_t>(lane) * waves + q;
-
-    if constexpr (!kFill) {
-        matrix_b[cell] = static_cast<std::uint32_t>(__builtin_popcountll(mine));
-    } else {
-        const std::uint32_t from = matrix_b[cell];
-        write_runs(stage, mine, g, from, list, p.capacity, lane);
-        if (q == 0 && owner) {
-            // this tile's list: from the first cell of the tile to the first cell of the next one
-            const std::size_t next_cell = static_cast<std::size_t>(wave0) * 64 + static_cast<std::size_t>(lane + 1) * waves;
-            const std::uint32_t to = matrix_b[next_cell];
-            const int tile = ty * p.tiles_x + tx;
-            range_begin[tile] = from < p.capacity ? from : p.capacity;
-            range_end[tile] = to < p.capacity ? to : p.capacity;
+    const std::uint32_t reach_it = a.totals[p.supers + s];
+    // the lists of the supertiles before this one, the counts of this one's tiles in all ranges and in those before these
+    std::uint32_t before = 0;
+    for (int k = t; k < s; k += kFillLanes) before += a.totals[k];
+    std::uint32_t all = 0, earlier = 0;
+#pragma unroll 8
+    for (int r = wave; r < p.ranges; r += kFillWaves) {
+        const std::uint32_t c = a.counts[(static_cast<std::size_t>(r) * p.supers + s) * 64 + lane];
+        all += c;
+        earlier += r < first_range ? c : 0u;
+    }
+    if (reach_it > most) return;  // (asked for with the rest, so that a block waits for memory once)
+    lds.part_all[wave][lane] = all;
+    lds.part_before[wave][lane] = earlier;
+    std::uint32_t before_word[kFillWords], found_in_wave = 0;  // entries of the words before, and of all of the wavefront's
+#pragma unroll
+    for (int k = 0; k < kFillWords; ++k) {
+        const std::uint32_t found = static_cast<std::uint32_t>(__builtin_popcountll(mine[k])), up_to = running_sum(found);
+        before_word[k] = found_in_wave + up_to - found;
+        found_in_wave += last_lane(up_to);
+    }
+    const std::uint32_t before_in_wave = last_lane(running_sum(before));
+    if (lane == 0) {
+        lds.hits_of_wave[wave] = found_in_wave;
+        lds.before_of_wave[wave] = before_in_wave;
+    }
+    __syncthreads();
+    std::uint32_t base = 0, hits = 0, place = 0;  // place: of the wavefront's first entry among the block's
+#pragma unroll
+    for (int w = 0; w < kFillWaves; ++w) {
+        const std::uint32_t of_wave = lds.hits_of_wave[w];
+        place += w < wave ? of_wave : 0u;
+        hits += of_wave;
+        base += lds.before_of_wave[w];
+    }
+    const int base_x = where.x * 8, base_y = where.y * 8;
+    if (wave == kFillWaves - 1) {  // the others look for their entries meanwhile
+        std::uint32_t tile_all = 0, tile_before = 0;
+#pragma unroll
+        for (int w = 0; w < kFillWaves; ++w) {
+            tile_all += lds.part_all[w][lane];
+            tile_before += lds.part_before[w][lane];
         }
-        if (w == 0 && lane == 0) {
-            const std::uint32_t pairs = matrix_b[static_cast<std::size_t>(p.waves_b) * 64];  // the scan's total
-            status[kStatusPairs] = pairs;
-            if (pairs > p.capacity) {
-                status[kStatusOverflow] = 1;
-                atomicMax(status + kStatusOverflowSticky, pairs);
+        const std::uint32_t behind = base + running_sum(tile_all), begin = behind - tile_all;
+        lds.cursor[lane] = begin + tile_before;
+        const int tx = base_x + (lane & 7), ty = base_y + (lane >> 3);
+        if (first_range == 0 && tx < p.tiles_x && ty < p.tiles_y) {
+            // a list that does not fit is cut short; the pair count stays exact
+            a.range_begin[ty * p.tiles_x + tx] = begin < p.capacity ? begin : p.capacity;
+            a.range_end[ty * p.tiles_x + tx] = behind < p.capacity ? behind : p.capacity;
+        }
+        if (first_range == 0 && s == p.supers - 1 && lane == 63) {
+            const bool overflow = behind > p.capacity;
+            a.status[kStatusPairs] = behind;
+            a.status[kStatusOverflow] = overflow ? 1u : 0u;
+            if (overflow) atomicMax(a.status + kStatusOverflowSticky, behind);
+            if (a.clear_depth_flag) a.status[kStatusDepthChanged] = 0;
+        }
+    }
+    for (std::uint32_t batch = 0; batch < hits; batch += kFillGroups * 64) {
+        // (place - batch wraps around where a wavefront's or a word's entries begin in an earlier batch)
+        if (share <= 16) {
+            // few words: one after the other, a lane a bit (a lane a word, below, is a loop as long as the fullest word)
+            std::uint64_t words = ballot(mine[0] != 0);
+            if (place + found_in_wave <= batch) words = 0;
+            for (; words != 0; words &= words - 1) {
+                const int l = __builtin_ctzll(words);
+                const std::uint32_t lo = read_lane(static_cast<std::uint32_t>(mine[0]), l), hi = read_lane(static_cast<std::uint32_t>(mine[0] >> 32), l);
+                const std::uint32_t at = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, place - batch + read_lane(before_word[0], l)));
+                if (((static_cast<std::uint64_t>(hi) << 32 | lo) >> lane & 1) != 0 && at < kFillGroups * 64u)
+                    lds.entry[at] = static_cast<std::uint32_t>((my_first + l) * 64 + lane);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < kFillWords; ++k) {
+                std::uint32_t at = place + before_word[k] - batch;
+                if (at < kFillGroups * 64u || at + 64 < 64u)
+                    for_each_bit(mine[k], [&](int bit) {
+                        if (at < kFillGroups * 64u) lds.entry[at] = static_cast<std::uint32_t>((my_first + k * 64 + lane) * 64 + bit);
+                        ++at;
+                    });
             }
         }
+        __syncthreads();
+        const int here = static_cast<int>(hits - batch < kFillGroups * 64u ? hits - batch : kFillGroups * 64u);
+        // groups of fewer than 64 entries where all wavefronts have one then
+        const int span = here > 32 * kFillWaves ? 64 : (here > 16 * kFillWaves ? 32 : (here > 8 * kFillWaves ? 16 : 8));
+        constexpr int kEach = kFillGroups / kFillWaves;
+        TileRect rects[kEach];
+        std::uint32_t id[kEach];
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) {
+            const int e = (k * kFillWaves + wave) * span + lane;
+            rects[k] = TileRect{1, 1, 0, 0};
+            id[k] = 0;
+            if (lane < span && e < here) {
+                const std::uint32_t i = lds.entry[e];
+                rects[k] = a.rects_by_depth[i];
+                id[k] = a.by_depth[i];
+            }
+        }
+        std::uint64_t word[kEach];  // of a group that this wavefront has: the entries that cover tile `lane`
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) {
+            const int group = k * kFillWaves + wave;
+            word[k] = 0;
+            if (group * span < here) {  // the same for the wavefront
+                const std::uint64_t mask = block_mask(at_least(rects[k].x0 - base_x, 0), at_most(rects[k].x1 - base_x, 7),
+                                                      at_least(rects[k].y0 - base_y, 0), at_most(rects[k].y1 - base_y, 7));
+                int here_lane = lane;
+                asm volatile("" : "+v"(here_lane));
+                word[k] = transposed(mask, here_lane);
+                if (lane < span) lds.entry[group * span + lane] = id[k];
+            }
+            lds.count_of[group][lane] = static_cast<std::uint32_t>(__builtin_popcountll(word[k]));
+        }
+        __syncthreads();
+        // The pairs of the batch, tile after tile: numbered, put in that order into LDS as (tile, entry), and written from there with
+        // consecutive lanes on consecutive places of a list.  (A store by the lanes that hold the words touches 64 lines.)
+        std::uint32_t of_tile = 0, number[kEach] = {};
+#pragma unroll 8
+        for (int group = 0; group < kFillGroups; ++group) {
+            const std::uint32_t count = lds.count_of[group][lane];
+#pragma unroll
+            for (int k = 0; k < kEach; ++k) number[k] += group < k * kFillWaves + wave ? count : 0u;
+            of_tile += count;
+        }
+        const std::uint32_t behind_tile = running_sum(of_tile), pairs = last_lane(behind_tile);
+        if (wave == 0) {
+            const std::uint32_t from = lds.cursor[lane];
+            lds.to_list[lane] = from - (behind_tile - of_tile);  // (wraps around: a place is this plus the pair's number)
+            lds.cursor[lane] = from + of_tile;
+        }
+        for (std::uint32_t window = 0; window < pairs; window += kStagedPairs) {
+#pragma unroll
+            for (int k = 0; k < kEach; ++k) {
+                std::uint32_t at = number[k] + (behind_tile - of_tile) - window;
+                const int tag = (lane << 10) + (k * kFillWaves + wave) * span;
+                for_each_bit(word[k], [&](int bit) {
+                    if (at < kStagedPairs) lds.staged[at] = static_cast<std::uint16_t>(tag + bit);
+                    ++at;
+                });
+            }
+            __syncthreads();
+            const std::uint32_t end = pairs - window < kStagedPairs ? pairs - window : kStagedPairs;
+#pragma unroll 4
+            for (std::uint32_t e = static_cast<std::uint32_t>(t); e < end; e += kFillLanes) {
+                const std::uint32_t pair = lds.staged[e], to = lds.to_list[pair >> 10] + (window + e);
+                if (to < p.capacity) a.list[to] = lds.entry[pair & 1023u];
+            }
+            __syncthreads();
+        }
+        if (pairs == 0) __syncthreads();  // the counts have been read
+        static_assert(kFillGroups * 64 == 1 << 10, "ten bits for an entry");
     }
 }
+
+// Block = (slice of slice_ranges ranges) x supertile.  Supertiles that very many Gaussians reach (more than kHeavy for each of
+// their blocks: a cluster) are left to `helpers` blocks more, which deal their ranges out among them.
+constexpr std::uint32_t kHeavy = 4096;
+__global__ void __launch_bounds__(kFillLanes, 8) fill_kernel(FillArgs a, int helpers) {
+    __shared__ FillLds lds;
+    const BinPlan& p = a.p;
+    const std::uint32_t* const reached = a.totals + p.supers;
+    const std::uint32_t heavy = helpers > 0 ? kHeavy * static_cast<std::uint32_t>(p.slices) : ~0u;
+    const int first_of_slab = a.first_chunk / p.range_chunks;
+    const int own_blocks = static_cast<int>(gridDim.x) - helpers, block = static_cast<int>(blockIdx.x);
+    const bool helps = block >= own_blocks;
+    // every helper counts the same items (heavy supertile, range) and takes each helpers-th
+    int base = 0, next = block - own_blocks;  // the supertiles looked at; the block's next item, counted from the first of these
+    for (;;) {
+        int s, from, ranges;
+        if (helps) {
+            std::uint64_t those = 0;
+            for (; base < p.supers; base += 64) {
+                those = ballot(reached[base + (threadIdx.x & 63)] > heavy);
+                const int items = __builtin_popcountll(those) * a.slab_ranges;
+                if (next < items) break;
+                next -= items;
+            }
+            if (base >= p.supers) return;
+            for (int k = next / a.slab_ranges; k > 0; --k) those &= those - 1;
+            s = base + __builtin_ctzll(those);
+            from = next % a.slab_ranges;
+            ranges = 1;
+            next += helpers;
+        } else {
+            s = block % p.supers;
+            from = block / p.supers * p.slice_ranges;
+            ranges = at_most(p.slice_ranges, a.slab_ranges - from);
+            const bool reports = s == p.supers - 1 && first_of_slab + from == 0;
+            if (!super_coords(p, s).inside && !reports) return;
+        }
+        fill_lists(a, s, first_of_slab + from, ranges, helps ? ~0u : heavy, lds);
+        if (!helps) return;
+        __syncthreads();  // what this item left in LDS has been read
+    }
+}
+
+constexpr int kFillHelpers = 256;  // a block per compute unit
+constexpr std::size_t kSlabBytes = std::size_t(64) << 20;  // of words kept between cover and fill, if a slice needs no more
 
 }  // namespace
 
-BinPlan make_bin_plan(int G, int tiles_x, int tiles_y, std::uint32_t capacity, std::uint32_t capacity_a) {
+BinPlan make_bin_plan(int G, int tiles_x, int tiles_y, std::uint32_t capacity) {
     BinPlan p{};
     p.G = G;
     p.tiles_x = tiles_x;
@@ -475,185 +522,64 @@ BinPlan make_bin_plan(int G, int tiles_x, int tiles_y, std::uint32_t capacity, s
     p.group_x = (p.super_x + 7) / 8;
     p.groups = p.group_x * ((p.super_y + 7) / 8);
     p.supers = p.groups * 64;  // numbered group by group; those beyond the image stay empty
-    // about 8192 wavefronts at level A (short ones: a wavefront's chunks of 64 Gaussians are a chain of memory
-    // latencies), and never less than 64 Gaussians per wavefront
-    const long long per_wave = (static_cast<long long>(G) * p.groups + 8191) / 8192;
-    p.range_a = static_cast<int>(((per_wave > 64 ? per_wave : 64) + 63) / 64 * 64);
-    p.ranges_a = (G + p.range_a - 1) / p.range_a;
     p.capacity = capacity;
-    p.capacity_a = capacity_a < capacity ? capacity_a : capacity;
-    p.waves_b = static_cast<std::uint32_t>((static_cast<std::uint64_t>(p.capacity_a) + kBinRangeB - 1) / kBinRangeB) +
-                static_cast<std::uint32_t>(p.supers);
+    p.chunks = (G + 63) / 64;
+    // cover: a chunk per wavefront at least, up to 64 ranges (every one adds to the same totals, one after the other), and none
+    // beyond what a fill block takes
+    const int wanted_range = ((p.chunks + 63) / 64 + kCoverWaves - 1) / kCoverWaves * kCoverWaves;
+    p.range_chunks = wanted_range < kSliceChunks ? wanted_range : kSliceChunks;
+    p.ranges = (p.chunks + p.range_chunks - 1) / p.range_chunks;
+    // fill: slices of 256 Gaussians per supertile of the image, so that a block has a batch of entries or so where they lie evenly,
+    // and no more words than its lanes hold, so that a cluster in one supertile is not one block's work
+    const long long wanted = 4ll * p.super_x * p.super_y;
+    const int most = static_cast<int>(wanted < kSliceChunks ? wanted : kSliceChunks);
+    p.slice_ranges = most / p.range_chunks > 1 ? most / p.range_chunks : 1;
+    p.slice_chunks = p.slice_ranges * p.range_chunks;
+    p.slices = (p.chunks + p.slice_chunks - 1) / p.slice_chunks;
+    const std::size_t slice_bytes = static_cast<std::size_t>(p.supers) * p.slice_chunks * sizeof(std::uint64_t);
+    const std::size_t fit = kSlabBytes / slice_bytes;
+    p.slab_slices = static_cast<int>(fit < 1 ? 1 : (fit < static_cast<std::size_t>(p.slices) ? fit : p.slices));
+    p.slab_chunks = p.slab_slices * p.slice_chunks;
     return p;
 }
 
-std::size_t bin_matrix_a_words(const BinPlan& p) { return static_cast<std::size_t>(p.supers) * p.ranges_a + 1; }
-std::size_t bin_matrix_b_words(const BinPlan& p) { return static_cast<std::size_t>(p.waves_b) * 64 + 1; }
-std::size_t bin_scan_state_words(const BinPlan& p) {
-    const std::size_t longest = bin_matrix_a_words(p) > bin_matrix_b_words(p) ? bin_matrix_a_words(p) : bin_matrix_b_words(p);
-    return (longest + kScanTile - 1) / kScanTile + 1;
-}
+std::size_t bin_covering_words(const BinPlan& p) { return static_cast<std::size_t>(p.supers) * p.slab_chunks; }
+std::size_t bin_counts_words(const BinPlan& p) { return static_cast<std::size_t>(p.supers) * 64 * p.ranges; }
 
-namespace {
-
-int launch_scan(hipStream_t s, std::uint32_t* data, std::size_t n, const BinScratch& scratch) {
-    XAD_REQUIRE(n > 0 && n < (std::size_t(1) << 32) - 2 * kScanTile, "splat binning: %zu counts do not fit the 32-bit scan", n);
-    const unsigned blocks = static_cast<unsigned>((n + kScanTile - 1) / kScanTile);
-    hipLaunchKernelGGL(scan_kernel, dim3(blocks), dim3(kScanBlock), 0, s, data, static_cast<std::uint32_t>(n), scratch.scan_state,
-                       scratch.scan_control);
+int launch_cover(hipStream_t s, const BinPlan& p, const TileRect* rects_by_depth, const BinScratch& scratch) {
+    XAD_REQUIRE(p.G > 0 && p.supers > 0 && p.ranges > 0, "splat binning: empty plan");
+    const dim3 grid(static_cast<unsigned>(p.groups) * static_cast<unsigned>(p.ranges)), block(64 * kCoverWaves);
+    if (p.slab_slices >= p.slices)
+        hipLaunchKernelGGL((cover_kernel<true, true>), grid, block, 0, s, p, 0, rects_by_depth, scratch.covering, scratch.counts,
+                           scratch.totals);
+    else
+        hipLaunchKernelGGL((cover_kernel<true, false>), grid, block, 0, s, p, 0, rects_by_depth, scratch.covering, scratch.counts,
+                           scratch.totals);
     XAD_HIP_TRY(hipGetLastError());
     return XAD_OK;
 }
 
-}  // namespace
-
-// ---------------------------------------------------------------------------
-// Small scenes in two launches.  The two levels above take seven, 3 to 10 us each however little there is to do.  Here a
-// block tests one tile against all Gaussians, 64 rectangles to a wavefront at a time and in depth order, and leaves
-// one bit per Gaussian and their count; a second launch adds up the counts of the tiles before its own, and the set
-// bits, in order, are the list.  (In one launch, with room for the lists taken from a counter: 28 us with 1080 tiles
-// and next to no Gaussians, for the atomics on one address.)
-// What bounds it: the tests, tiles x Gaussians of them, and the latency of a wavefront's chain of loads.
-// The rule (bins_by_tests) is where the two ways cross.  A forward call, us, two levels / so: 1000 Gaussians at
-// 640 x 427 43.6 / 21.4, 2000 at 720 x 700 45.5 / 25.5, 10 000 at 512 x 512 69.8 / 53.6, 12 000 at 640 x 640 (301 000
-// tests) 68.3 / 58.2, 16 384 at 512 x 288 99.9 / 90.1, 16 000 at 128 x 128 119 / 102; but 20 000 at 512 x 512
-// (321 000) 91.0 / 89.3, 20 000 at 768 x 768 (721 000) 75.8 / 88.0, 60 000 at 256 x 256, where a wavefront's chain of
-// chunks is long, 108 / 148, and 10 000 at 1024 x 1024 (4096 tiles) 61.9 / 67.6.
-constexpr int kTestWaves = 4;
-
-__device__ __forceinline__ std::uint32_t sum_over_block(std::uint32_t v, std::uint32_t (&per_wave)[kTestWaves]) {
-    for (int step = 32; step > 0; step /= 2) v += __shfl_xor(v, step, 64);
-    if ((threadIdx.x & 63) == 0) per_wave[threadIdx.x >> 6] = v;
-    __syncthreads();
-    std::uint32_t total = 0;
-#pragma unroll
-    for (int w = 0; w < kTestWaves; ++w) total += per_wave[w];
-    return total;
-}
-
-__global__ void __launch_bounds__(64 * kTestWaves) test_tiles_kernel(BinPlan p, const TileRect* __restrict__ rects_by_depth,
-                                                                     std::uint64_t* __restrict__ covering,
-                                                                     std::uint32_t* __restrict__ counts) {
-    __shared__ std::uint32_t per_wave[kTestWaves];
-    const int wave = static_cast<int>(threadIdx.x) >> 6, lane = static_cast<int>(threadIdx.x) & 63;
-    const int tile = static_cast<int>(blockIdx.x), tx = tile % p.tiles_x, ty = tile / p.tiles_x;
-    const int chunks = (p.G + 63) / 64;
-    std::uint64_t* mine = covering + static_cast<std::size_t>(tile) * chunks;
-    constexpr int kAhead = 8;  // loads in flight
-    std::uint32_t count = 0;   // of this lane's Gaussians
-    for (int c0 = wave * kAhead; c0 < chunks; c0 += kTestWaves * kAhead) {
-        TileRect r[kAhead];
-#pragma unroll
-        for (int k = 0; k < kAhead; ++k) {
-            const int i = (c0 + k) * 64 + lane;
-            r[k] = TileRect{1, 1, 0, 0};  // covers nothing
-            if (i < p.G) r[k] = rects_by_depth[i];
+int launch_fill(hipStream_t s, const BinPlan& p, const std::uint32_t* by_depth, const TileRect* rects_by_depth, const BinScratch& scratch,
+                std::uint32_t* list, std::uint32_t* range_begin, std::uint32_t* range_end, std::uint32_t* status, bool clear_depth_flag) {
+    XAD_REQUIRE(p.capacity > 0, "splat binning: no room for lists");
+    const bool one_slab = p.slab_slices >= p.slices;
+    const unsigned groups = static_cast<unsigned>(p.groups), supers = static_cast<unsigned>(p.supers);
+    for (int slice = 0; slice < p.slices; slice += p.slab_slices) {
+        const int slices = p.slices - slice < p.slab_slices ? p.slices - slice : p.slab_slices, first_chunk = slice * p.slice_chunks;
+        const int left = p.ranges - slice * p.slice_ranges, ranges = left < slices * p.slice_ranges ? left : slices * p.slice_ranges;
+        if (!one_slab) {
+            hipLaunchKernelGGL((cover_kernel<false, true>), dim3(groups * static_cast<unsigned>(ranges)), dim3(64 * kCoverWaves), 0, s, p,
+                               first_chunk, rects_by_depth, scratch.covering, scratch.counts, scratch.totals);
+            XAD_HIP_TRY(hipGetLastError());
         }
-        std::uint64_t answer = 0;
-#pragma unroll
-        for (int k = 0; k < kAhead; ++k) {
-            const bool covers = tx >= r[k].x0 && tx <= r[k].x1 && ty >= r[k].y0 && ty <= r[k].y1;
-            const std::uint64_t mask = ballot(covers);
-            count += covers ? 1u : 0u;
-            if (lane == k) answer = mask;
-        }
-        if (lane < kAhead && c0 + lane < chunks) mine[c0 + lane] = answer;
-    }
-    const std::uint32_t total = sum_over_block(count, per_wave);
-    if (threadIdx.x == 0) counts[tile] = total;
-}
-
-__global__ void __launch_bounds__(64 * kTestWaves) write_lists_kernel(
-    BinPlan p, const std::uint32_t* __restrict__ by_depth, const std::uint64_t* __restrict__ covering,
-    const std::uint32_t* __restrict__ counts, std::uint32_t* __restrict__ list, std::uint32_t* __restrict__ range_begin,
-    std::uint32_t* __restrict__ range_end, std::uint32_t* __restrict__ status, bool clear_depth_flag) {
-    __shared__ std::uint32_t per_wave[kTestWaves];
-    __shared__ std::uint32_t found[kTestWaves];
-    const int wave = static_cast<int>(threadIdx.x) >> 6, lane = static_cast<int>(threadIdx.x) & 63;
-    const int tile = static_cast<int>(blockIdx.x);
-    const int chunks = (p.G + 63) / 64, share = (chunks + kTestWaves - 1) / kTestWaves;
-    const int begin = wave * share, end = begin + share < chunks ? begin + share : chunks;
-    const std::uint64_t* mine = covering + static_cast<std::size_t>(tile) * chunks;
-
-    std::uint32_t before = 0, here = 0;
-    for (int t = static_cast<int>(threadIdx.x); t < tile; t += 64 * kTestWaves) before += counts[t];
-    for (int c = begin + lane; c < end; c += 64) here += static_cast<std::uint32_t>(__builtin_popcountll(mine[c]));
-    for (int step = 32; step > 0; step /= 2) here += __shfl_xor(here, step, 64);
-    if (lane == 0) found[wave] = here;
-    const std::uint32_t first = sum_over_block(before, per_wave);
-    std::uint32_t at = first;
-    for (int w = 0; w < wave; ++w) at += found[w];
-
-    for (int c = begin; c < end; c += 64) {
-        const std::uint64_t answers = c + lane < end ? mine[c + lane] : 0;
-        for (std::uint64_t todo = ballot(answers != 0); todo != 0; todo &= todo - 1) {
-            const int k = __builtin_ctzll(todo);
-            const std::uint64_t mask =
-                static_cast<std::uint64_t>(static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(answers >> 32), k))) << 32 |
-                static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(answers), k));
-            if ((mask >> lane) & 1) {
-                const std::uint32_t to = at + static_cast<std::uint32_t>(__builtin_popcountll(mask & ((std::uint64_t(1) << lane) - 1)));
-                if (to < p.capacity) list[to] = by_depth[(c + k) * 64 + lane];
-            }
-            at += static_cast<std::uint32_t>(__builtin_popcountll(mask));
-        }
-    }
-    if (threadIdx.x == 0) {
-        // a list that does not fit is cut short; the pair count stays exact
-        const std::uint32_t behind = first + counts[tile];
-        range_begin[tile] = first < p.capacity ? first : p.capacity;
-        range_end[tile] = behind < p.capacity ? behind : p.capacity;
-        if (blockIdx.x == gridDim.x - 1) {
-            const bool overflow = behind > p.capacity;
-            status[kStatusPairs] = behind;
-            status[kStatusSuperPairs] = 0;
-            status[kStatusOverflow] = overflow ? 1u : 0u;
-            if (overflow) atomicMax(status + kStatusOverflowSticky, behind);
-            if (clear_depth_flag) status[kStatusDepthChanged] = 0;
-        }
-    }
-}
-
-bool bins_by_tests(int G, int tiles) {
-    const long long chunks = (static_cast<long long>(G) + 63) / 64;
-    return tiles <= kBinTestTiles && chunks <= kBinTestChunks && chunks * tiles <= kBinTests;
-}
-
-int launch_binning(hipStream_t s, const BinPlan& p, const std::uint32_t* by_depth, const TileRect* rects_by_depth,
-                   const TileRect* rects, BinScratch& scratch,
-                   std::uint32_t* list, std::uint32_t* range_begin, std::uint32_t* range_end, std::uint32_t* status,
-                   bool clear_depth_flag) {
-    XAD_REQUIRE(p.G > 0 && p.supers > 0 && p.ranges_a > 0 && p.capacity > 0, "splat binning: empty plan");
-    XAD_REQUIRE(range_end == range_begin + static_cast<std::size_t>(p.tiles_x) * p.tiles_y,
-                "splat binning: the two halves of the tile ranges must be adjacent");
-    if (scratch.covering) {
-        const dim3 grid(static_cast<unsigned>(p.tiles_x) * static_cast<unsigned>(p.tiles_y)), block(64 * kTestWaves);
-        hipLaunchKernelGGL(test_tiles_kernel, grid, block, 0, s, p, rects_by_depth, scratch.covering, scratch.counts);
+        // (none where no supertile can be that heavy)
+        const int helpers = static_cast<std::uint32_t>(p.G) > kHeavy * static_cast<std::uint32_t>(p.slices) ? kFillHelpers : 0;
+        const FillArgs args{p, first_chunk, ranges, by_depth, rects_by_depth, scratch.covering, scratch.counts, scratch.totals, list,
+                            range_begin, range_end, status, clear_depth_flag};
+        hipLaunchKernelGGL(fill_kernel, dim3(static_cast<unsigned>(helpers) + supers * static_cast<unsigned>(slices)), dim3(kFillLanes), 0, s,
+                           args, helpers);
         XAD_HIP_TRY(hipGetLastError());
-        hipLaunchKernelGGL(write_lists_kernel, grid, block, 0, s, p, by_depth, scratch.covering, scratch.counts, list, range_begin,
-                           range_end, status, clear_depth_flag);
-        XAD_HIP_TRY(hipGetLastError());
-        return XAD_OK;
     }
-    const unsigned waves_a = static_cast<unsigned>(p.ranges_a) * static_cast<unsigned>(p.groups);
-    hipLaunchKernelGGL(super_kernel<false>, dim3(waves_a), dim3(64), 0, s, p, by_depth, rects_by_depth, scratch.matrix_a,
-                       scratch.list_a);
-    XAD_HIP_TRY(hipGetLastError());
-    if (int st = launch_scan(s, scratch.matrix_a, bin_matrix_a_words(p) - 1, scratch)) return st;
-    const unsigned plan_blocks = static_cast<unsigned>((static_cast<std::size_t>(p.tiles_x) * p.tiles_y * 2 + 4095) / 4096);
-    hipLaunchKernelGGL(plan_kernel, dim3(plan_blocks < 1 ? 1 : (plan_blocks > 512 ? 512 : plan_blocks)), dim3(256), 0, s, p,
-                       scratch.matrix_a, scratch.first_wave, range_begin, status, clear_depth_flag);
-    XAD_HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(super_kernel<true>, dim3(waves_a), dim3(64), 0, s, p, by_depth, rects_by_depth, scratch.matrix_a,
-                       scratch.list_a);
-    XAD_HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(tile_kernel<false>, dim3(p.waves_b), dim3(64), 0, s, p, scratch.matrix_a, scratch.first_wave, scratch.list_a,
-                       rects, scratch.matrix_b, list, range_begin, range_end, status);
-    XAD_HIP_TRY(hipGetLastError());
-    if (int st = launch_scan(s, scratch.matrix_b, bin_matrix_b_words(p) - 1, scratch)) return st;
-    hipLaunchKernelGGL(tile_kernel<true>, dim3(p.waves_b), dim3(64), 0, s, p, scratch.matrix_a, scratch.first_wave, scratch.list_a,
-                       rects, scratch.matrix_b, list, range_begin, range_end, status);
-    XAD_HIP_TRY(hipGetLastError());
     return XAD_OK;
 }
 

@@ -36,8 +36,7 @@ struct xad_splat_context {
     // one allocation for everything whose size is fixed by (G, image): `fixed` is its base
     void* fixed = nullptr;
     Record* records = nullptr;
-    TileRect* rects = nullptr;
-    TileRect* rects_by_depth = nullptr;  // the same rectangles in depth order
+    TileRect* rects_by_depth = nullptr;  // in depth order
     std::uint32_t* rank = nullptr;       // G: position of every Gaussian in the depth order
     std::uint32_t *depth_keys = nullptr, *depth_keys_sorted = nullptr;  // G each
     std::uint32_t *identity = nullptr, *by_depth = nullptr;             // G each; by_depth = Gaussians in (depth, index) order
@@ -54,9 +53,7 @@ struct xad_splat_context {
     void* depth_sort_temp = nullptr;
     std::size_t depth_sort_bytes = 0;
 
-    // one allocation for everything sized by the pair capacity: `paired` is its base
-    void* paired = nullptr;
-    std::uint32_t* list = nullptr;  // the tiles' lists
+    std::uint32_t* list = nullptr;  // the tiles' lists: plan.capacity entries, an allocation of its own
     BinPlan plan{};
     BinScratch bin;
 
@@ -86,7 +83,6 @@ void carve_fixed(xad_splat_context* c, char* base, std::size_t* bytes) {
     Carver k{base};
     const std::size_t G = static_cast<std::size_t>(c->G), pixels = static_cast<std::size_t>(c->width) * c->height;
     c->records = k.take<Record>(G);
-    c->rects = k.take<TileRect>(G);
     c->rects_by_depth = k.take<TileRect>(G);
     c->rank = k.take<std::uint32_t>(G);
     c->depth_keys = k.take<std::uint32_t>(G);
@@ -98,54 +94,33 @@ void carve_fixed(xad_splat_context* c, char* base, std::size_t* bytes) {
     c->range_end = c->range_begin ? c->range_begin + c->tiles : nullptr;
     c->final_T = k.take<float>(pixels);
     c->n_contrib = k.take<std::uint32_t>(pixels);
-    c->tile_order = k.take<std::uint32_t>(static_cast<std::size_t>((c->tiles + 7) / 8) * 8);
+    if (orders_tiles(c->G)) c->tile_order = k.take<std::uint32_t>(static_cast<std::size_t>((c->tiles + 7) / 8) * 8);
     c->segment_state = c->segments > 1 ? k.take<float4>(pixels * static_cast<std::size_t>(c->segments)) : nullptr;
     c->record_grads = k.take<float>(G * kRecordGradStride);
     c->loss = k.take<double>(kLossWords);
     c->status = k.take<std::uint32_t>(kStatusWords);
-    if (bins_by_tests(c->G, c->tiles)) {
-        c->bin.covering = k.take<std::uint64_t>((G + 63) / 64 * static_cast<std::size_t>(c->tiles));
-        c->bin.counts = k.take<std::uint32_t>(static_cast<std::size_t>(c->tiles));
-    }
-    c->bin.scan_control = k.take<std::uint32_t>(kScanControlWords);
+    c->bin.covering = k.take<std::uint64_t>(bin_covering_words(c->plan));
+    c->bin.counts = k.take<std::uint32_t>(bin_counts_words(c->plan));
+    c->bin.totals = k.take<std::uint32_t>(2 * static_cast<std::size_t>(c->plan.supers));
     c->depth_sort_temp = k.take<char>(c->depth_sort_bytes ? c->depth_sort_bytes : 16);
-    *bytes = k.used;
-}
-
-void carve_paired(xad_splat_context* c, char* base, std::size_t* bytes) {
-    Carver k{base};
-    c->list = k.take<std::uint32_t>(c->plan.capacity);
-    *bytes = k.used;
-    if (c->bin.covering) return;  // lists made by tests need nothing else of this size
-    c->bin.list_a = k.take<std::uint32_t>(c->plan.capacity);
-    c->bin.matrix_a = k.take<std::uint32_t>(bin_matrix_a_words(c->plan));
-    c->bin.matrix_b = k.take<std::uint32_t>(bin_matrix_b_words(c->plan));
-    c->bin.first_wave = k.take<std::uint32_t>(static_cast<std::size_t>(c->plan.supers) + 1);
-    c->bin.scan_state = k.take<std::uint64_t>(bin_scan_state_words(c->plan));
     *bytes = k.used;
 }
 
 // (Re)allocates the buffers sized by the pair capacity.  Waits for the device first: a step may still be using them.
 int size_pair_buffers(xad_splat_context* c, std::uint32_t capacity) {
-    if (c->paired) {
+    if (c->list) {
         XAD_HIP_TRY(hipDeviceSynchronize());
-        (void)hipFree(c->paired);
-        c->paired = nullptr;
+        (void)hipFree(c->list);
+        c->list = nullptr;
     }
     c->capacity_seen = false;
-    c->plan = make_bin_plan(c->G, c->tiles_x, c->tiles_y, capacity, capacity);  // the buffers are sized for this one
-    std::size_t bytes = 0;
-    carve_paired(c, nullptr, &bytes);
+    c->plan.capacity = 0;
     void* base = nullptr;
-    if (hipMalloc(&base, bytes) != hipSuccess) {
-        c->plan.capacity = 0;  // the next call tries again
+    const std::size_t bytes = static_cast<std::size_t>(capacity) * sizeof(std::uint32_t);
+    if (hipMalloc(&base, bytes) != hipSuccess)  // the next call tries again
         return xad::fail(XAD_ERR_HIP, "splat: hipMalloc of %zu bytes for %u pairs failed", bytes, capacity);
-    }
-    c->paired = base;
-    carve_paired(c, static_cast<char*>(base), &bytes);
-    // the scan's state words must not look like words of a coming epoch
-    if (c->bin.scan_state) XAD_HIP_TRY(hipMemset(c->bin.scan_state, 0, bin_scan_state_words(c->plan) * sizeof(std::uint64_t)));
-    XAD_HIP_TRY(hipDeviceSynchronize());  // the fills (this one and that of the fixed buffers) are not on the caller's stream
+    c->list = static_cast<std::uint32_t*>(base);
+    c->plan.capacity = capacity;
     return XAD_OK;
 }
 
@@ -153,7 +128,8 @@ void mark(xad_splat_context* c, int index, hipStream_t s) {
     if (c->profile) (void)hipEventRecord(c->marks[index], s);
 }
 
-// Projection, after ordering the Gaussians by (depth, index) when asked to; the order is then kept until a depth changes.
+// Projection, after ordering the Gaussians by (depth, index) when asked to (the order is then kept until a depth changes), and
+// the first part of the binning.
 int project_gaussians(xad_splat_context* c, const float* params, const float* depth, hipStream_t s, bool first_of_step,
                       bool ordering) {
     if (ordering) {
@@ -165,15 +141,16 @@ int project_gaussians(xad_splat_context* c, const float* params, const float* de
     }
     mark(c, 1, s);
     if (int st = launch_project(s, c->G, params, depth, c->ordered_depth, c->rank, c->status, c->width, c->height, c->records,
-                                c->rects, c->rects_by_depth, c->record_grads, c->loss, first_of_step))
+                                c->rects_by_depth, c->record_grads, c->loss, c->bin.totals, 2 * c->plan.supers, first_of_step))
         return st;
     mark(c, 2, s);
-    return XAD_OK;
+    return launch_cover(s, c->plan, c->rects_by_depth, c->bin);
 }
 
+// The second part of the binning.
 int bin_lists(xad_splat_context* c, hipStream_t s, bool clear_depth_flag) {
-    return launch_binning(s, c->plan, c->by_depth, c->rects_by_depth, c->rects, c->bin, c->list, c->range_begin, c->range_end,
-                          c->status, clear_depth_flag);
+    return launch_fill(s, c->plan, c->by_depth, c->rects_by_depth, c->bin, c->list, c->range_begin, c->range_end, c->status,
+                       clear_depth_flag);
 }
 
 // Queues a copy of the status words (and the loss) to the host and waits for it.
@@ -207,27 +184,9 @@ std::uint32_t grown(std::uint32_t pairs) {
     return static_cast<std::uint32_t>(want < 0xfffffff0ull ? want : 0xfffffff0ull);
 }
 
-// Level A's share of the buffers once a scene's supertile pairs are known: twice that many (the wavefronts
-// launched at level B follow it, so it is not simply everything).
-std::uint32_t level_a_share(std::uint32_t super_pairs) {
-    const std::uint64_t want = 2ull * super_pairs + 1024;
-    return static_cast<std::uint32_t>(want < 0xfffffff0ull ? want : 0xfffffff0ull);
-}
-
-// A step needed room for `seen` pairs (tile or supertile level, whichever is larger) and did not have it.
-// If the buffers themselves are large enough, only level A's share of them was too small: it gets the whole
-// buffer back, nothing is allocated.  Otherwise the buffers are replaced by larger ones.
+// A step needed room for `seen` pairs and did not have it.
 int make_room(xad_splat_context* c, std::uint32_t seen) {
-    if (seen <= c->plan.capacity && c->plan.capacity_a < c->plan.capacity) {
-        c->plan = make_bin_plan(c->G, c->tiles_x, c->tiles_y, c->plan.capacity, c->plan.capacity);
-        c->capacity_seen = false;
-        return XAD_OK;
-    }
     return size_pair_buffers(c, grown(seen > c->plan.capacity ? seen : c->plan.capacity + 1));
-}
-
-std::uint32_t pairs_needed(const HostReport* r) {
-    return r->status[kStatusPairs] > r->status[kStatusSuperPairs] ? r->status[kStatusPairs] : r->status[kStatusSuperPairs];
 }
 
 // Project and bin; leaves the tiles' lists in the context.  Where the host has to look:
@@ -263,24 +222,17 @@ int bin(xad_splat_context* c, const float* params, const float* depth, hipStream
             if (int st = bin_lists(c, s, true)) return st;
             if (int st = fetch_report(c, s)) return st;
         }
-        // The tile-level pair count is exact even when it exceeds the capacity, unless the supertile lists
-        // were cut short as well (then it is a lower bound and the next attempt's count is exact).
+        // (the pair count is exact also when it exceeds the capacity)
         bool made_room = false;
         for (int attempt = 0; c->report->status[kStatusOverflow] != 0; ++attempt) {
-            const std::uint32_t seen = pairs_needed(c->report);
+            const std::uint32_t seen = c->report->status[kStatusPairs];
             XAD_REQUIRE(attempt < 4 && seen < 0xfffffff0u, "splat: the pair lists overflow at %u pairs", seen);
             if (int st = make_room(c, seen)) return st;
-            if (int st = bin_lists(c, s, false)) return st;
+            if (int st = bin_lists(c, s, false)) return st;  // (what the first part left does not depend on the room)
             if (int st = fetch_report(c, s)) return st;
             made_room = true;
         }
-        if (!c->capacity_seen) {
-            c->capacity_seen = true;
-            // from now on level A is given only the room this scene needs, with a margin: fewer wavefronts at level B
-            // (an overflow of that margin is reported like any other and gives level A the whole buffer back)
-            if (!c->bin.covering)
-                c->plan = make_bin_plan(c->G, c->tiles_x, c->tiles_y, c->plan.capacity, level_a_share(c->report->status[kStatusSuperPairs]));
-        }
+        c->capacity_seen = true;
         // what this call's own attempts left in the sticky word is settled; what earlier calls left there stays
         if (made_room && c->report->status[kStatusStickyBefore] == 0) {
             if (int st = clear_status(c, s, kStatusOverflowSticky, 1)) return st;
@@ -346,6 +298,7 @@ extern "C" int xad_splat_create(int width, int height, int num_gaussians, std::s
     c->tiles_y = tiles_y;
     c->tiles = tiles_x * tiles_y;
     c->segments = render_segments(width, height);
+    c->plan = make_bin_plan(num_gaussians, tiles_x, tiles_y, 0);
     c->depth_sort_bytes = depth_sort_temp_bytes(num_gaussians);
     int st = XAD_OK;
     std::size_t bytes = 0;
@@ -353,11 +306,9 @@ extern "C" int xad_splat_create(int width, int height, int num_gaussians, std::s
     if (hipMalloc(&c->fixed, bytes) != hipSuccess) st = xad::fail(XAD_ERR_HIP, "%s: hipMalloc of %zu bytes failed", who, bytes);
     if (st == XAD_OK) {
         carve_fixed(c, static_cast<char*>(c->fixed), &bytes);
-        // status words, the scan's control words and the tile ranges start from zero; the scan's epoch from one
-        if (hipMemset(c->fixed, 0, bytes) != hipSuccess) st = xad::fail(XAD_ERR_HIP, "%s: hipMemset failed", who);
-        const std::uint32_t control[kScanControlWords] = {0u, 0u, 1u};
-        if (st == XAD_OK && hipMemcpy(c->bin.scan_control, control, sizeof(control), hipMemcpyHostToDevice) != hipSuccess)
-            st = xad::fail(XAD_ERR_HIP, "%s: hipMemcpy failed", who);
+        // status words and the tile ranges start from zero
+        if (hipMemset(c->fixed, 0, bytes) != hipSuccess || hipDeviceSynchronize() != hipSuccess)  // (not on the caller's stream)
+            st = xad::fail(XAD_ERR_HIP, "%s: hipMemset failed", who);
     }
     if (st == XAD_OK && hipHostMalloc(reinterpret_cast<void**>(&c->report), sizeof(HostReport)) != hipSuccess)
         st = xad::fail(XAD_ERR_HIP, "%s: pinned allocation failed", who);
@@ -380,7 +331,7 @@ extern "C" int xad_splat_create(int width, int height, int num_gaussians, std::s
 
 extern "C" void xad_splat_destroy(xad_splat_context* c) {
     if (!c) return;
-    if (c->paired) (void)hipFree(c->paired);
+    if (c->list) (void)hipFree(c->list);
     if (c->fixed) (void)hipFree(c->fixed);
     if (c->report) (void)hipHostFree(c->report);
     for (auto& e : c->marks)
@@ -444,7 +395,7 @@ extern "C" int xad_splat_step(xad_splat_context* c, const float* params, const f
             // this very step did not fit (the scene grew): enlarge the lists and do it again.  Whether steps
             // before it overflowed too is in the word the step saved when it began.
             earlier_steps_overflowed = c->report->status[kStatusStickyBefore] != 0;
-            if (int st = make_room(c, pairs_needed(c->report))) return st;
+            if (int st = make_room(c, c->report->status[kStatusPairs])) return st;
             if (int st = clear_status(c, s, kStatusOverflowSticky, 1)) return st;
             c->report->status[kStatusOverflowSticky] = 0;
             continue;

@@ -34,15 +34,16 @@ __global__ void __launch_bounds__(256) project_kernel(int G, const float* __rest
                                                       const float* __restrict__ ordered_depth,
                                                       const std::uint32_t* __restrict__ rank,
                                                       std::uint32_t* __restrict__ status, int width, int height,
-                                                      Record* __restrict__ records, TileRect* __restrict__ rects,
-                                                      TileRect* __restrict__ rects_by_depth,
+                                                      Record* __restrict__ records, TileRect* __restrict__ rects_by_depth,
                                                       float* __restrict__ record_grads, double* __restrict__ loss,
+                                                      std::uint32_t* __restrict__ bin_totals, int total_words,
                                                       bool first_of_step) {
     const int g = blockIdx.x * 256 + threadIdx.x;
     // what the steps before this one left in the sticky overflow word (this step's own binning may add to it)
     if (first_of_step && g == 0) status[kStatusStickyBefore] = status[kStatusOverflowSticky];
-    // what the compositing backward adds into starts from zero: the parts of the loss, this Gaussian's accumulator row
+    // what later launches add into starts from zero: the parts of the loss, the binning's sums, this Gaussian's accumulator row
     if (blockIdx.x == 0 && threadIdx.x < kLossParts) loss[kLossStride * (1 + threadIdx.x)] = 0.0;
+    for (int k = g; k < total_words; k += static_cast<int>(gridDim.x) * 256) bin_totals[k] = 0;
     if (g >= G) return;
     {
         float4* row = reinterpret_cast<float4*>(record_grads + static_cast<std::size_t>(g) * kRecordGradStride);
@@ -95,7 +96,6 @@ __global__ void __launch_bounds__(256) project_kernel(int G, const float* __rest
             rc.y1 = static_cast<std::int16_t>(hi_y > static_cast<float>(tiles_y - 1) ? tiles_y - 1 : static_cast<int>(hi_y));
         }
     }
-    rects[g] = rc;
     rects_by_depth[rank[g]] = rc;  // the binning walks the Gaussians in depth order
 }
 
@@ -152,10 +152,12 @@ __global__ void __launch_bounds__(1024) tile_order_kernel(int tiles, const std::
     for (int k = band_last - band_first + t; k < per; k += 1024) order[band_first + k] = ~0u;  // the last band may be short
 }
 
-// Tile of a block: block b belongs to XCD b % 8 and is that XCD's (b / 8)-th block.
+// Tile of a block: block b belongs to XCD b % 8 and is that XCD's (b / 8)-th block, which takes the (b / 8)-th tile of the
+// XCD's band, or of its order if there is one.
 __device__ __forceinline__ int ordered_tile_of_block(int block, int tiles, const std::uint32_t* __restrict__ order) {
-    const int per = (tiles + 7) / 8;
-    const std::uint32_t tile = order[(block % 8) * per + block / 8];
+    const int per = (tiles + 7) / 8, at = (block % 8) * per + block / 8;
+    if (order == nullptr) return block / 8 < per && at < tiles ? at : tiles;
+    const std::uint32_t tile = order[at];
     return tile == ~0u ? tiles : static_cast<int>(tile);
 }
 
@@ -856,10 +858,11 @@ __global__ void __launch_bounds__(256) gaussian_backward_kernel(int G, const flo
 // launchers (declared in splat_launch.cuh)
 
 int launch_project(hipStream_t s, int G, const float* params, const float* depth, const float* ordered_depth,
-                   const std::uint32_t* rank, std::uint32_t* status, int width, int height, Record* records, TileRect* rects,
-                   TileRect* rects_by_depth, float* record_grads, double* loss, bool first_of_step) {
+                   const std::uint32_t* rank, std::uint32_t* status, int width, int height, Record* records,
+                   TileRect* rects_by_depth, float* record_grads, double* loss, std::uint32_t* bin_totals, int total_words,
+                   bool first_of_step) {
     hipLaunchKernelGGL(project_kernel, dim3(xad::blocks_for(G, 256)), dim3(256), 0, s, G, params, depth, ordered_depth, rank,
-                       status, width, height, records, rects, rects_by_depth, record_grads, loss, first_of_step);
+                       status, width, height, records, rects_by_depth, record_grads, loss, bin_totals, total_words, first_of_step);
     XAD_HIP_TRY(hipGetLastError());
     return XAD_OK;
 }
@@ -881,8 +884,10 @@ int launch_render_forward(hipStream_t s, int width, int height, const std::uint3
                           std::uint32_t* tile_order) {
     const int tiles_x = (width + kTile - 1) / kTile, tiles = tiles_x * ((height + kTile - 1) / kTile);
     // the order both compositing kernels of this step take the tiles in
-    hipLaunchKernelGGL(tile_order_kernel, dim3(8), dim3(1024), 0, s, tiles, range_begin, range_end, tile_order);
-    XAD_HIP_TRY(hipGetLastError());
+    if (tile_order) {
+        hipLaunchKernelGGL(tile_order_kernel, dim3(8), dim3(1024), 0, s, tiles, range_begin, range_end, tile_order);
+        XAD_HIP_TRY(hipGetLastError());
+    }
     XAD_REQUIRE(segments >= 1 && segments <= kMaxSegments && (segments == 1 || segment_state), "splat: a split walk needs its per-segment state");
     const dim3 grid(padded_tile_blocks(tiles) * kForwardParts), block(kChunk);
     if (segments > 1)
