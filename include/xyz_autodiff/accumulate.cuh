@@ -112,6 +112,17 @@ __device__ __forceinline__ V sum(V v) {
     return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
 }
 
+// Largest v of all 64 lanes, not less than 0, returned to every lane.
+__device__ __forceinline__ int most(int v) {
+    auto step = [](int x, int moved) { return x > moved ? x : moved; };
+    v = step(v, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true));
+    v = step(v, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true));
+    v = step(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, true));
+    v = step(v, __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, true));
+    const int rows = step(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16));
+    return step(rows, step(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
 }  // namespace wave
 
 template <typename T, int Width, Strategy S = Strategy::LdsAtomics, int PeelRounds = 8, int MinGroup = 4,
@@ -143,9 +154,10 @@ public:
     // instruction that share such a slot no longer share an address (each sharing lane costs an LDS
     // atomic about 3 cycles); flush() adds the copies up.  The copies take (replicas - 1) *
     // (hot_rows | 1) rows of the capacity, after the rows of the slots themselves (rows_for()).
-    // Clears the table; ends with a block barrier.
+    // Clears the table; ends with a block barrier.  `cleared`: neither, because the block has set the table's memory to zero
+    // (and its tags, if there are any, to kEmpty) itself and passed a barrier since.
     __device__ BlockAccumulator(void* lds, int capacity, T* global, int num_slots, int row_stride = Width,
-                                int replicas = 1, bool claim_rows = true, int hot_rows = -1)
+                                int replicas = 1, bool claim_rows = true, int hot_rows = -1, bool cleared = false)
         : table_(static_cast<TableT*>(lds)),
           tags_(reinterpret_cast<int*>(static_cast<TableT*>(lds) + static_cast<std::size_t>(capacity) * Width)),
           global_(global),
@@ -162,7 +174,7 @@ public:
         copies_base_ = main_rows_ | 1;
         const int copy = static_cast<int>(wave::lane_id() & static_cast<unsigned>(replicas - 1));
         my_copy_ = copy == 0 ? 0 : copies_base_ + (copy - 1) * hot_stride_;
-        clear();
+        if (!cleared) clear();
     }
 
     // Slots that own a row of a table of `capacity` rows that is not tagged: all of them if they fit, else the
@@ -232,8 +244,8 @@ public:
     }
 
     // Writes the table out (one global atomic per non-zero element) and clears
-    // it, so the object can take another round of add().
-    __device__ void flush() {
+    // it, so the object can take another round of add(); `last`: leaves it as it is.
+    __device__ void flush(bool last = false) {
         if constexpr (S == Strategy::GlobalAtomics) return;
         if constexpr (Spill) {
             if (spill_ != nullptr && staged_ != 0) write_out_staged();
@@ -251,6 +263,7 @@ public:
             const T v = static_cast<T>(sum);
             if (slot != kEmpty && v != T(0)) detail::atomic_add(global_ + static_cast<std::size_t>(slot) * row_stride_ + element, v);
         }
+        if (last) return;
         __syncthreads();
         clear();
     }

@@ -158,3 +158,16 @@ def test_lds_fp64_atomics_are_the_fast_ones(gpu, xad):
     cycles = instruments.lds_atomic_cycles()
     assert cycles["f64"]["64_distinct"] * 4 < cycles["f32"]["64_distinct"]
     assert cycles["f64"]["one_address"] > cycles["f64"]["64_distinct"]
+
+
+# Slots dealt to the blocks of a stretch: the fewest and the most slots that are (two hands, and 32 full ones) and one more, a
+# last hand that is short or empty, the fewest problems that fill every compute unit and one more or less, a ragged end.
+@pytest.mark.parametrize("n,num_slots", [(262_144, 3073), (262_143, 3073), (262_145, 24_577), (300_001, 98_304), (300_001, 98_305),
+                                         (1_000_003, 10_000), (700_001, 65_540), (2_000_003, 3500)])
+def test_auto_where_slots_are_dealt_out(gpu, oracle, n, num_slots):
+    inputs = chain_inputs(n, seed=num_slots % 97)
+    rng = np.random.default_rng(n + num_slots)
+    slot = rng.integers(0, num_slots, n).astype(np.int32)
+    slot[::41] = rng.choice([-1, -2**31, num_slots, 2**31 - 1], size=slot[::41].size)
+    sums, mass, kmass = _reference(oracle, inputs, slot, num_slots)
+    _assert_close(_run(gpu, inputs, slot, num_slots, "auto", prefill=-1.5) + 1.5, (sums, mass + 1.5, kmass), 1e-4)

@@ -50,6 +50,11 @@ struct AccumulateArgs {
     // The layout by slot index is made for laws whose low slots are the hot ones; under any other law the
     // hot slots would go through the spill path, one same-address atomic after the other.
     int fallback_rows;
+    // With deal_shift > 0: under such a law the slots are dealt out instead, to 2^deal_shift blocks for every stretch of the
+    // inputs, deal_rows consecutive ones to each (see accumulate_dealt()); its queues lie queue_offset bytes into the LDS.
+    int deal_shift;
+    int deal_rows;
+    unsigned queue_offset;
 };
 
 // Which part a block serves, the rows of its table and where they live in the global array.
@@ -66,40 +71,14 @@ struct Part {
     }
 };
 
-template <Strategy S, int Peel, typename TableT, bool Spill = false>
-__global__ void __launch_bounds__(kBlock) accumulate_kernel(AccumulateArgs a) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];
+template <Strategy S, int Peel, typename TableT, bool Spill>
+__device__ __forceinline__ void accumulate_stretch(const AccumulateArgs& a, float* lds, bool cleared = false) {
     const Part part(a);
     const std::size_t begin = static_cast<std::size_t>(blockIdx.x >> a.part_shift) * a.per_block;
     const std::size_t end = begin + a.per_block < a.n ? begin + a.per_block : a.n;
     using Acc = BlockAccumulator<float, kWidth, S, Peel, 4, TableT, Spill>;
-    if (a.fallback_rows > 0) {  // the same for every block
-        // the block's first slots as a sample of the law: who would find a row of its own?
-        const std::size_t i = begin + threadIdx.x;
-        const int sample = i < end ? part.row_of(a.slot[i], a) : -1;
-        const int owners = Acc::main_rows_for(a.capacity, part.rows, a.replicas, a.hot_rows);
-        // counted in the first two words of the table's memory, which the accumulator clears afterwards
-        int* count = reinterpret_cast<int*>(lds);
-        if (threadIdx.x < 2) count[threadIdx.x] = 0;
-        __syncthreads();
-        const int seen_here = __builtin_popcountll(xyz_autodiff::accumulate::wave::ballot(sample >= 0));
-        const int served_here = __builtin_popcountll(xyz_autodiff::accumulate::wave::ballot(sample >= 0 && sample < owners));
-        if (xyz_autodiff::accumulate::wave::lane_id() == 0) {
-            atomicAdd(count + 0, seen_here);
-            atomicAdd(count + 1, served_here);
-        }
-        __syncthreads();
-        const int seen = count[0], served = count[1];
-        __syncthreads();
-        if (2 * served < seen) {
-            a.capacity = a.fallback_rows;
-            a.replicas = 1;
-            a.claim_rows = 1;
-            a.hot_rows = -1;
-        }
-    }
     Acc acc(lds, a.capacity, a.grads + part.index * kWidth, part.rows, part.parts * kWidth, a.replicas, a.claim_rows != 0,
-            a.hot_rows);
+            a.hot_rows, cleared);
     if constexpr (Spill) acc.use_spill_staging(reinterpret_cast<char*>(lds) + a.spill_offset);
 
     // The inputs of the next trip are requested before the arithmetic of this one, so that a lane has
@@ -137,7 +116,188 @@ __global__ void __launch_bounds__(kBlock) accumulate_kernel(AccumulateArgs a) {
         acc.add(slot, g);
         current = next;
     }
-    acc.flush();
+    acc.flush(true);
+}
+
+template <Strategy S, int Peel, typename TableT, bool Spill = false>
+__global__ void __launch_bounds__(kBlock) accumulate_kernel(AccumulateArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    accumulate_stretch<S, Peel, TableT, Spill>(a, lds);
+}
+
+// More slots than a table holds, under a law that does not favour the low ones.  A block that walks a stretch of the inputs
+// by itself has rows for some of the slots it meets; the rest goes out one global atomic request a contribution (20 G/s).
+// Instead 2^deal_shift blocks walk the same stretch, each for consecutive slots that its table holds all of: every block
+// reads the slots, queues the problems that are its own, and evaluates 64 of them whenever a wavefront has that many.  What
+// goes out is the table, whole rows side by side.  The blocks of a stretch run on one XCD (blocks are handed to the eight
+// XCDs in turn), whose L2 then reads the inputs once.  (The table's memory is zero when this is called.)
+// What bounds it: with few problems the requests of the tables and the latency of a short walk, with many the lines of the
+// inputs that every block of a stretch reads.  Measured (us, uniform slots, before / so): 1 M problems into 4096 / 10 000 /
+// 40 000 / 90 000 slots 43 62 63 62 / 20 24 37 51, 4 M into 10 000 229 / 51, 16 M into 10 000 / 40 000 / 90 000 880 930 930 / 171
+// 386 635.  10 000 slots dealt to 4 / 8 / 16 / 32 hands: 28 24 29 43 (1 M), 173 243 380 600 (16 M).
+constexpr int kQueue = 128;  // problems a wavefront can have waiting: fewer than 64, and 64 more
+__device__ __forceinline__ void accumulate_dealt(const AccumulateArgs& a, float* lds) {
+    using Acc = BlockAccumulator<float, kWidth, Strategy::LdsAtomics, 0, 4, double>;
+    namespace wave = xyz_autodiff::accumulate::wave;
+    const int turn = static_cast<int>(blockIdx.x) / 8;
+    const int first_slot = (turn & ((1 << a.deal_shift) - 1)) * a.deal_rows;
+    const int rows = a.num_slots - first_slot < a.deal_rows ? a.num_slots - first_slot : a.deal_rows;
+    const std::size_t stretches = gridDim.x >> a.deal_shift;
+    const std::size_t per = ((a.n + stretches - 1) / stretches + 63) / 64 * 64;
+    const std::size_t begin = (static_cast<std::size_t>(turn >> a.deal_shift) * 8 + blockIdx.x % 8) * per;
+    if (rows <= 0 || begin >= a.n) return;  // the same for the block
+    const std::size_t end = begin + per < a.n ? begin + per : a.n;
+    Acc acc(lds, a.deal_rows, a.grads + static_cast<std::size_t>(first_slot) * kWidth, rows, kWidth, 1, false, -1, true);
+
+    const unsigned lane = wave::lane_id();
+    const unsigned wavefront = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    // (problem within the stretch, row)
+    uint2* const queue = reinterpret_cast<uint2*>(reinterpret_cast<char*>(lds) + a.queue_offset) + wavefront * kQueue;
+    unsigned waiting = 0;  // the same for the wavefront
+    struct Problems {
+        int row;  // -1 for none
+        float x[6];
+    };
+    auto take = [&](unsigned count) {  // the last `count` of the queue
+        Problems p{-1, {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}};
+        waiting -= count;
+        __builtin_amdgcn_wave_barrier();
+        if (lane < count) {
+            const uint2 entry = queue[waiting + lane];
+            p.row = static_cast<int>(entry.y);
+#pragma unroll
+            for (int k = 0; k < 6; ++k) p.x[k] = a.in[k][begin + entry.x];
+        }
+        __builtin_amdgcn_wave_barrier();
+        return p;
+    };
+    auto add = [&](const Problems& p) {
+        float g[kWidth] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (p.row >= 0) {
+            const auto r = xad_chain::forward_backward<float>(p.x[0], p.x[1], p.x[2], p.x[3], p.x[4], p.x[5]);
+            g[0] = r.d_sx;
+            g[1] = r.d_sy;
+            g[2] = r.d_theta;
+            g[3] = r.d_o;
+            g[4] = r.d_px;
+            g[5] = r.d_py;
+        }
+        acc.add(p.row, g);
+    };
+    // the inputs of 64 problems are on their way while the 64 before are evaluated
+    Problems coming{-1, {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}};
+    constexpr int kAhead = 4;  // loads of slots in flight
+    for (std::size_t base = begin; base < end; base += kAhead * kBlock) {
+        int slot[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const std::size_t i = base + static_cast<std::size_t>(u) * kBlock + threadIdx.x;
+            slot[u] = i < end ? a.slot[i] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const unsigned row = static_cast<unsigned>(slot[u]) - static_cast<unsigned>(first_slot);
+            const bool own = slot[u] >= 0 && row < static_cast<unsigned>(rows);
+            const std::uint64_t owners = wave::ballot(own);
+            if (own) {
+                const unsigned before = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(owners >> 32),
+                                                                  __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(owners), 0u));
+                queue[waiting + before] = uint2{static_cast<unsigned>(base - begin) + u * kBlock + threadIdx.x, row};
+            }
+            waiting += static_cast<unsigned>(__builtin_popcountll(owners));
+            if (waiting >= 64) {
+                const Problems next = take(64);
+                add(coming);
+                coming = next;
+            }
+        }
+    }
+    add(coming);
+    if (waiting != 0) add(take(waiting));
+    acc.flush(true);
+}
+
+// Strategy AUTO for more slots than a table holds.  Two samples of slots say which layout: 256 from all over, the same for
+// every block (what the blocks do together they have to agree on), and the block's first 1024.
+//   dealt    if by this estimate (picoseconds, from the measurements at accumulate_dealt()) it is the faster;
+//   by index the first slots own the rows: made for laws whose low slots are the hot ones;
+//   claimed  if fewer than half of the block's sample would find a row by index.
+struct DealEstimate {  // what the estimate needs of the launch
+    float by_index_rows;   // requests for the tables by index
+    float dealt_rows;      // for the dealt ones
+    float scan;            // reading every slot 2^deal_shift times
+    float evaluate;        // evaluating all problems, evenly dealt
+    float miss;            // of all problems, if each went out by itself
+    float per_row;         // hands a slot is worth
+};
+constexpr int kMostHands = 32;
+constexpr unsigned kCommonSample = 256;
+
+template <bool kDeals>
+__global__ void __launch_bounds__(kBlock) accumulate_many_slots_kernel(AccumulateArgs a, DealEstimate cost) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    using Acc = BlockAccumulator<float, kWidth, Strategy::LdsAtomics, 0, 4, double, true>;
+    namespace wave = xyz_autodiff::accumulate::wave;
+    constexpr unsigned kWaves = kBlock / 64, kSampleWaves = kCommonSample / 64;
+    const Part part(a);
+    const unsigned lane = wave::lane_id(), wavefront = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const std::size_t begin = static_cast<std::size_t>(blockIdx.x) * a.per_block;
+    const std::size_t end = begin + a.per_block < a.n ? begin + a.per_block : a.n;
+    const std::size_t own = begin + threadIdx.x;
+    const bool looks = kDeals && wavefront < kSampleWaves;
+    const int sample = own < end ? part.row_of(a.slot[own], a) : -1;
+    // (sixteen neighbours at sixteen places: a wavefront reads four lines)
+    const int common = looks ? part.row_of(a.slot[a.n / 16 * (threadIdx.x / 16) + threadIdx.x % 16], a) : -1;
+    const int owners = Acc::main_rows_for(a.capacity, part.rows, a.replicas, a.hot_rows);
+    // meanwhile: no table is larger than the one by index
+    for (int k = static_cast<int>(threadIdx.x); k < a.capacity * kWidth / 2; k += kBlock) reinterpret_cast<double2*>(lds)[k] = double2{0.0, 0.0};
+    // counted behind it, where rows will be staged
+    int4* const of_wave = reinterpret_cast<int4*>(reinterpret_cast<char*>(lds) + a.spill_offset);
+    int* const hands = reinterpret_cast<int*>(of_wave + kWaves);  // [wavefront][kMostHands]
+    auto count = [](bool yes) { return __builtin_popcountll(wave::ballot(yes)); };
+    const int4 here{count(sample >= 0), count(sample >= 0 && sample < owners), count(common >= 0), count(common >= 0 && common < owners)};
+    if (lane == 0) of_wave[wavefront] = here;
+    if (looks) {
+        // (a row of counters to a wavefront: its LDS accesses are in order)
+        int* const mine = hands + wavefront * kMostHands;
+        if (lane < kMostHands) mine[lane] = 0;
+        __builtin_amdgcn_wave_barrier();
+        if (common >= 0) atomicAdd(mine + static_cast<int>(static_cast<float>(common) * cost.per_row), 1);  // (an estimate)
+    }
+    __syncthreads();
+    int4 all{0, 0, 0, 0};  // seen and served, of both samples
+#pragma unroll
+    for (unsigned w = 0; w < kWaves; ++w) {
+        const int4 one = of_wave[w];
+        all.x += one.x, all.y += one.y, all.z += one.z, all.w += one.w;
+    }
+    bool deal = false;
+    if constexpr (kDeals) {
+        int in_hands = 0;  // lane k: hand k; the fullest is what the others wait for
+#pragma unroll
+        for (unsigned w = 0; w < kSampleWaves; ++w) in_hands += hands[w * kMostHands + (lane & (kMostHands - 1))];
+        const int most = wave::most(in_hands);
+        const float by_index = cost.by_index_rows + cost.miss * static_cast<float>(all.z - all.w) * (1.f / kCommonSample);
+        const float dealt = cost.dealt_rows + cost.scan + cost.evaluate * static_cast<float>((most << a.deal_shift) - all.z) * (1.f / kCommonSample);
+        deal = dealt < by_index;
+    }
+    __syncthreads();
+    if constexpr (kDeals) {
+        if (deal) {
+            accumulate_dealt(a, lds);
+            return;
+        }
+    }
+    if (2 * all.y < all.x) {
+        a.capacity = a.fallback_rows;
+        a.replicas = 1;
+        a.claim_rows = 1;
+        a.hot_rows = -1;
+        int* const tags = reinterpret_cast<int*>(reinterpret_cast<double*>(lds) + a.capacity * kWidth);
+        for (int k = static_cast<int>(threadIdx.x); k < a.capacity; k += kBlock) tags[k] = Acc::kEmpty;
+        __syncthreads();
+    }
+    accumulate_stretch<Strategy::LdsAtomics, 0, double, true>(a, lds, true);
 }
 
 // Same work with the accumulator used through drop-in leaves: the graph is
@@ -178,7 +338,7 @@ __global__ void __launch_bounds__(kBlock) accumulate_leaf_kernel(AccumulateArgs 
             w.run();
         }
     }
-    acc.flush();
+    acc.flush(true);
 }
 
 __global__ void __launch_bounds__(256) zipf_kernel(int* dst, std::size_t n, std::uint64_t key, const double* cdf,
@@ -202,14 +362,42 @@ __global__ void __launch_bounds__(256) zipf_kernel(int* dst, std::size_t n, std:
 int device_compute_units(int* out) {
     int dev = 0;
     XAD_HIP_TRY(hipGetDevice(&dev));
-    hipDeviceProp_t prop;
-    XAD_HIP_TRY(hipGetDeviceProperties(&prop, dev));
-    *out = prop.multiProcessorCount;
+    XAD_HIP_TRY(hipDeviceGetAttribute(out, hipDeviceAttributeMultiprocessorCount, dev));
     return XAD_OK;
 }
 
-template <typename Kernel>
-int launch(Kernel kernel, AccumulateArgs a, std::size_t lds_bytes, int blocks_per_cu, void* stream) {
+// In how many hands to deal the slots where the device finds it the faster way, if at all: from as many as it takes for a
+// table to hold a hand, twice as many while that saves more requests than reading the slots once more costs.
+constexpr std::size_t kQueueBytes = kBlock / 64 * kQueue * sizeof(uint2);
+DealEstimate deal_slots(AccumulateArgs* a, int cus, std::size_t* lds_bytes) {
+    constexpr std::size_t kRowBytes = kWidth * sizeof(double);
+    constexpr float kRequest = 50.f, kReadSlot = 270.f, kEvaluate = 1700.f;  // picoseconds: of the device, of a compute unit (twice)
+    constexpr float kRequestsPerRow = kWidth * 4.f / 64.f;                   // rows side by side: 64 bytes a request
+    const float n = static_cast<float>(a->n), blocks = static_cast<float>(cus);
+    const float rows = static_cast<float>(a->num_slots);
+    DealEstimate e{blocks * static_cast<float>(a->capacity) * kRequestsPerRow * kRequest, 0.f, 0.f, n / blocks * kEvaluate, n * kRequest, 0.f};
+    if (a->n < static_cast<std::size_t>(cus) * kBlock) return e;  // fewer blocks than there are compute units
+    for (int shift = 1; (1 << shift) <= kMostHands && cus % (8 << shift) == 0; ++shift) {
+        const int hand = (((a->num_slots + (1 << shift) - 1) >> shift) + 7) / 8 * 8;  // (whole 64 bytes of the output)
+        const std::size_t bytes = static_cast<std::size_t>(hand) * kRowBytes + kQueueBytes;
+        if (bytes > kMaxLdsBytes) continue;
+        const float dealt_rows = blocks / static_cast<float>(1 << shift) * rows * kRequestsPerRow * kRequest;
+        const float scan = n * static_cast<float>(1 << shift) / blocks * kReadSlot;
+        if (a->deal_shift > 0 && dealt_rows + scan >= e.dealt_rows + e.scan) break;
+        a->deal_shift = shift;
+        a->deal_rows = hand;
+        a->queue_offset = static_cast<unsigned>(static_cast<std::size_t>(hand) * kRowBytes);
+        e.dealt_rows = dealt_rows;
+        e.scan = scan;
+        e.per_row = 1.f / static_cast<float>(hand);
+    }
+    const std::size_t needed = a->deal_shift > 0 ? a->queue_offset + kQueueBytes : 0;
+    if (needed > *lds_bytes) *lds_bytes = needed;
+    return e;
+}
+
+template <typename Kernel, typename... More>
+int launch(Kernel kernel, AccumulateArgs a, std::size_t lds_bytes, int blocks_per_cu, void* stream, More... more) {
     int cus = 0;
     if (int st = device_compute_units(&cus)) return st;
     if (lds_bytes > 64 * 1024)
@@ -220,9 +408,10 @@ int launch(Kernel kernel, AccumulateArgs a, std::size_t lds_bytes, int blocks_pe
     std::size_t blocks = std::min<std::size_t>(chunks, resident);  // per part
     const std::size_t chunks_per_block = (chunks + blocks - 1) / blocks;
     a.per_block = chunks_per_block * kBlock;
-    blocks = (a.n + a.per_block - 1) / a.per_block;
+    // (dealt slots need every block there is; by index the last ones may then have nothing to walk)
+    if (a.deal_shift == 0) blocks = (a.n + a.per_block - 1) / a.per_block;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks << a.part_shift)), dim3(kBlock), lds_bytes,
-                       xad::as_stream(stream), a);
+                       xad::as_stream(stream), a, more...);
     XAD_HIP_TRY(hipGetLastError());
     return XAD_OK;
 }
@@ -235,7 +424,7 @@ extern "C" int xad_accumulate_chain_gradients_f32(int strategy, std::size_t n, c
                                                   void* stream) {
     const char* who = "xad_accumulate_chain_gradients_f32";
     if (n == 0) return XAD_OK;
-    AccumulateArgs a{{sx, sy, theta, o, px, py}, slot, grads, n, 0, num_slots, 0, 0, 0, 1, 1, -1, 0};
+    AccumulateArgs a{{sx, sy, theta, o, px, py}, slot, grads, n, 0, num_slots, 0, 0, 0, 1, 1, -1, 0, 0, 0, 0};
     for (int k = 0; k < 6; ++k) XAD_REQUIRE(a.in[k], "%s: input array %d is null", who, k);
     XAD_REQUIRE(slot && grads, "%s: slot or grads is null", who);
     XAD_REQUIRE(num_slots > 0, "%s: num_slots must be positive, got %d", who, num_slots);
@@ -261,7 +450,12 @@ extern "C" int xad_accumulate_chain_gradients_f32(int strategy, std::size_t n, c
             a.hot_rows = 32;
             a.fallback_rows = 2048;  // with their tags the most fp64 rows in a power of two that fit
             a.spill_offset = static_cast<unsigned>(static_cast<std::size_t>(rows) * kRowBytes);
-            return launch(accumulate_kernel<Strategy::LdsAtomics, 0, double, true>, a, a.spill_offset + kSpillBytes, 1, stream);
+            std::size_t lds = a.spill_offset + kSpillBytes;
+            int cus = 0;
+            if (int st = device_compute_units(&cus)) return st;
+            const DealEstimate cost = deal_slots(&a, cus, &lds);
+            return a.deal_shift > 0 ? launch(accumulate_many_slots_kernel<true>, a, lds, 1, stream, cost)
+                                    : launch(accumulate_many_slots_kernel<false>, a, lds, 1, stream, cost);
         }
         if (num_slots > kHotRows) {
             // one fp64 table for every slot, the hot rows in as many copies as the LDS of a CU still holds
