@@ -194,3 +194,52 @@ def test_more_than_two_to_the_32_problems(gpu, oracle):
         assert float(ident) < 1e-6, (lo, float(ident))
     del ins, outs
     torch.cuda.empty_cache()
+
+
+def test_a_call_goes_to_the_stream_that_is_current_or_given(gpu):
+    """What a call queues is ordered behind the work of its own stream: a spin of some milliseconds, then the inputs."""
+    import torch
+
+    from xyz_autodiff_cuda_amd import _lib, chain
+
+    other = torch.cuda.Stream(gpu)
+    assert _lib.stream_handle(gpu) == torch.cuda.current_stream(gpu).cuda_stream
+    assert _lib.stream_handle(torch.device("cuda")) == torch.cuda.current_stream().cuda_stream  # no index
+    assert _lib.stream_handle(gpu, other) == other.cuda_stream
+    with torch.cuda.stream(other):
+        assert _lib.stream_handle(gpu) == other.cuda_stream
+    values = [torch.from_numpy(a).to(gpu) for a in chain_inputs(5000, seed=1)]
+    want = [o.clone() for o in chain.forward_backward(values)]
+    torch.cuda.synchronize()
+    for how in ("current", "given"):
+        inputs = [torch.zeros_like(v) for v in values]
+        outputs = [torch.zeros_like(w) for w in want]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            torch.cuda._sleep(5_000_000)
+            for i, v in zip(inputs, values):
+                i.copy_(v)
+            if how == "current":
+                chain.forward_backward(inputs, outputs)
+        if how == "given":
+            chain.forward_backward(inputs, outputs, stream=other)
+        other.synchronize()
+        assert all(torch.equal(o, w) for o, w in zip(outputs, want)), how
+
+
+def test_refused_arrays(gpu):
+    import torch
+
+    from xyz_autodiff_cuda_amd import chain
+
+    good = [torch.zeros(64, device=gpu) for _ in range(6)]
+    for bad, error in ((torch.zeros(64), TypeError), (np.zeros(64, np.float32), TypeError), (torch.zeros(64, device=gpu).double(), ValueError),
+                       (torch.zeros(65, device=gpu), ValueError), (torch.zeros(128, device=gpu)[::2], ValueError)):
+        with pytest.raises(error, match="py must be"):
+            chain.forward_backward(good[:5] + [bad])
+        with pytest.raises(error, match="d_py must be"):
+            chain.forward_backward(good, [torch.zeros(64, device=gpu) for _ in range(6)] + [bad])
+    with pytest.raises(ValueError, match="expected 6"):
+        chain.forward_backward(good[:5])
+    with pytest.raises(ValueError, match="expected 7"):
+        chain.forward_backward(good, good)

@@ -118,6 +118,28 @@ def load():
     return lib
 
 
+def stream_handle(device, stream=None):
+    """The hipStream_t of `stream`, or of the device's current stream."""
+    import torch
+
+    if stream is not None:
+        return stream.cuda_stream
+    index = device.index
+    # (2 us less than making a torch.cuda.Stream to ask it for its handle; the same per-thread current stream)
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None) if index is not None else None
+    return raw(index) if raw is not None else torch.cuda.current_stream(device).cuda_stream
+
+
+def call_on(device, fn, *args):
+    """fn(*args) with `device` current."""
+    import torch
+
+    if device.index is not None and device.index == torch.cuda.current_device():
+        return fn(*args)  # nothing to switch to and back from: 1 us less
+    with torch.cuda.device(device):
+        return fn(*args)
+
+
 def check(status, what):
     if status != XAD_OK:
         msg = load().xad_last_error().decode("utf-8", "replace")

@@ -48,11 +48,8 @@ def accumulate_chain_gradients(inputs, slot, grads, strategy=DEFAULT, stream=Non
         raise ValueError("slot must be a contiguous int32 CUDA tensor")
     if not (grads.is_cuda and grads.dtype == torch.float32 and grads.is_contiguous() and grads.dim() == 2 and grads.shape[1] == WIDTH):
         raise ValueError("grads must be a contiguous float32 CUDA tensor of shape (num_slots, 6)")
-    s = stream if stream is not None else torch.cuda.current_stream(slot.device)
-    with torch.cuda.device(slot.device):
-        st = lib.xad_accumulate_chain_gradients_f32(
-            int(strategy), n, *[t.data_ptr() for t in inputs], slot.data_ptr(), grads.data_ptr(), grads.shape[0], s.cuda_stream
-        )
+    st = _lib.call_on(slot.device, lib.xad_accumulate_chain_gradients_f32, int(strategy), n, *[t.data_ptr() for t in inputs],
+                      slot.data_ptr(), grads.data_ptr(), grads.shape[0], _lib.stream_handle(slot.device, stream))
     _lib.check(st, "xad_accumulate_chain_gradients_f32")
     return grads
 

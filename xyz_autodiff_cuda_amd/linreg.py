@@ -48,11 +48,9 @@ def batch_gradient(x1, x2, y, params, rows=None, strategy=WAVE_LDS, out=None, st
     if out is None:
         out = torch.empty(5, dtype=torch.float64, device=x1.device)
     n = rows.numel() if rows is not None else x1.numel()
-    s = stream if stream is not None else torch.cuda.current_stream(x1.device)
-    with torch.cuda.device(x1.device):
-        st = lib.xad_linreg_gradient_f64(int(strategy), n, x1.numel(), x1.data_ptr(), x2.data_ptr(), y.data_ptr(),
-                                         rows.data_ptr() if rows is not None else None, params.data_ptr(),
-                                         out.data_ptr(), s.cuda_stream)
+    st = _lib.call_on(x1.device, lib.xad_linreg_gradient_f64, int(strategy), n, x1.numel(), x1.data_ptr(), x2.data_ptr(),
+                      y.data_ptr(), rows.data_ptr() if rows is not None else None, params.data_ptr(), out.data_ptr(),
+                      _lib.stream_handle(x1.device, stream))
     _lib.check(st, "xad_linreg_gradient_f64")
     return out
 
@@ -77,12 +75,10 @@ def sgd(x1, x2, y, params, batch, epochs, lr_first=1e-4, lr_last=1e-6, seed=0, w
             raise ValueError("history must be a contiguous float64 CUDA tensor of at least `epochs` elements")
     elif want_history:
         history = torch.empty(epochs, dtype=torch.float64, device=x1.device)
-    s = stream if stream is not None else torch.cuda.current_stream(x1.device)
     name = "xad_linreg_sgd_f64_static" if static_scratch else "xad_linreg_sgd_f64"
-    with torch.cuda.device(x1.device):
-        st = getattr(lib, name)(x1.numel(), x1.data_ptr(), x2.data_ptr(), y.data_ptr(), params.data_ptr(),
-                                int(batch), int(epochs), float(lr_first), float(lr_last), int(seed),
-                                history.data_ptr() if history is not None else None, s.cuda_stream)
+    st = _lib.call_on(x1.device, getattr(lib, name), x1.numel(), x1.data_ptr(), x2.data_ptr(), y.data_ptr(), params.data_ptr(),
+                      int(batch), int(epochs), float(lr_first), float(lr_last), int(seed),
+                      history.data_ptr() if history is not None else None, _lib.stream_handle(x1.device, stream))
     _lib.check(st, name)
     return history
 

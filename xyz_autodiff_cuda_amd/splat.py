@@ -55,9 +55,7 @@ class SplatContext:
             pass
 
     def _stream(self, stream):
-        import torch
-
-        return (stream if stream is not None else torch.cuda.current_stream(self.device)).cuda_stream
+        return _lib.stream_handle(self.device, stream)
 
     def set_depth_mode(self, mode):
         _lib.check(self._lib.xad_splat_set_depth_mode(self._handle, DEPTH_MODES[mode] if isinstance(mode, str) else int(mode)),
@@ -94,8 +92,8 @@ class SplatContext:
         if image is None:
             image = torch.empty(self.height, self.width, 3, dtype=torch.float32, device=self.device)
         _check_tensor(image, (self.height, self.width, 3), "image")
-        with torch.cuda.device(self.device):
-            st = self._lib.xad_splat_forward(self._handle, params.data_ptr(), depth.data_ptr(), image.data_ptr(), self._stream(stream))
+        st = _lib.call_on(self.device, self._lib.xad_splat_forward, self._handle, params.data_ptr(), depth.data_ptr(), image.data_ptr(),
+                          self._stream(stream))
         _lib.check(st, "xad_splat_forward")
         return image
 
@@ -114,9 +112,8 @@ class SplatContext:
         _check_tensor(image, (self.height, self.width, 3), "image")
         _check_tensor(grads, (9, G), "grads")
         loss = ctypes.c_double(0.0)
-        with torch.cuda.device(self.device):
-            st = self._lib.xad_splat_step(self._handle, params.data_ptr(), depth.data_ptr(), target.data_ptr(), image.data_ptr(),
-                                          grads.data_ptr(), ctypes.byref(loss) if want_loss else None, self._stream(stream))
+        st = _lib.call_on(self.device, self._lib.xad_splat_step, self._handle, params.data_ptr(), depth.data_ptr(), target.data_ptr(),
+                          image.data_ptr(), grads.data_ptr(), ctypes.byref(loss) if want_loss else None, self._stream(stream))
         if st == _lib.XAD_ERR_INCOMPLETE:
             # this step's outputs are complete; an earlier step that did not wait lacked pairs (lists since enlarged)
             warnings.warn(self._lib.xad_last_error().decode("utf-8", "replace"), RuntimeWarning)
@@ -192,16 +189,14 @@ def adam_step(params, grads, m, v, learning_rates, iteration, beta1=0.9, beta2=0
     if len(learning_rates) != rows:
         raise ValueError("need one learning rate per row")
     lrs = (ctypes.c_float * rows)(*[float(x) for x in learning_rates])
-    s = (stream if stream is not None else torch.cuda.current_stream(params.device)).cuda_stream
-    with torch.cuda.device(params.device):
-        if hold_if_nonzero is None:
-            st = _lib.load().xad_adam_step_f32(n, rows, params.data_ptr(), grads.data_ptr(), m.data_ptr(), v.data_ptr(), lrs,
-                                               beta1, beta2, eps, int(iteration), s)
-        else:
-            gate = hold_if_nonzero.data_ptr() if hasattr(hold_if_nonzero, "data_ptr") else int(hold_if_nonzero)
-            st = _lib.load().xad_adam_step_gated_f32(n, rows, params.data_ptr(), grads.data_ptr(), m.data_ptr(), v.data_ptr(), lrs,
-                                                     beta1, beta2, eps, int(iteration), gate,
-                                                     held_count.data_ptr() if held_count is not None else None, s)
+    s = _lib.stream_handle(params.device, stream)
+    pointers = (params.data_ptr(), grads.data_ptr(), m.data_ptr(), v.data_ptr())
+    if hold_if_nonzero is None:
+        st = _lib.call_on(params.device, _lib.load().xad_adam_step_f32, n, rows, *pointers, lrs, beta1, beta2, eps, int(iteration), s)
+    else:
+        gate = hold_if_nonzero.data_ptr() if hasattr(hold_if_nonzero, "data_ptr") else int(hold_if_nonzero)
+        st = _lib.call_on(params.device, _lib.load().xad_adam_step_gated_f32, n, rows, *pointers, lrs, beta1, beta2, eps,
+                          int(iteration), gate, held_count.data_ptr() if held_count is not None else None, s)
     _lib.check(st, "xad_adam_step_f32")
 
 
