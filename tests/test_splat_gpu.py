@@ -241,6 +241,21 @@ def test_forward_only_equals_step_image(gpu, oracle):
     assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("G,W,H", [
+    (3000, 480, 512),   # 960 tiles: the backward walk in eight pieces
+    (3000, 496, 496),   # 961: in four
+    (19220, 496, 496),  # the same, as many Gaussians as that takes
+    (19221, 496, 496),  # one more: in eight
+])
+def test_pieces_of_the_walk_on_both_sides_of_their_rule(gpu, oracle, G, W, H):
+    params, depth = random_scene(G, W, H, seed=11, scale_px=(1.0, 4.0))
+    target = np.random.default_rng(11).uniform(0, 1, (H, W, 3)).astype(np.float32)
+    got = _gpu_step(gpu, W, H, params, depth, target)
+    _check_against_oracle(oracle, got, W, H, params, depth, target)
+    alone = _gpu_step(gpu, W, H, params, depth, target, forward_only=True)["image"]  # which keeps nothing for a backward walk
+    assert np.array_equal(alone, got["image"])
+
+
 def test_clamp_cutoff_and_depth_ties(gpu, oracle):
     W = H = 16
     layers = [one_gaussian(8, 8, np.log(1000.0), np.log(1000.0), 0.0, (1.0, 0.0, 0.0), 12.0) for _ in range(5)]

@@ -297,7 +297,7 @@ extern "C" int xad_splat_create(int width, int height, int num_gaussians, std::s
     c->tiles_x = tiles_x;
     c->tiles_y = tiles_y;
     c->tiles = tiles_x * tiles_y;
-    c->segments = render_segments(width, height);
+    c->segments = render_segments(width, height, num_gaussians);
     c->plan = make_bin_plan(num_gaussians, tiles_x, tiles_y, 0);
     c->depth_sort_bytes = depth_sort_temp_bytes(num_gaussians);
     int st = XAD_OK;
@@ -361,8 +361,10 @@ extern "C" int xad_splat_forward(xad_splat_context* c, const float* params, cons
     XAD_REQUIRE(c && params && depth && image, "%s: null argument", who);
     hipStream_t s = xad::as_stream(stream);
     if (int st = bin(c, params, depth, s)) return st;
+    // No states for a backward walk that does not follow.  A call with them / without: 10 000 Gaussians at 512 x 512 47.1 / 45.7 us, at
+    // 700 x 700 43.0 / 41.6, 20 000 at 1000 x 500 60.2 / 58.3.
     if (int st = launch_render_forward(s, c->width, c->height, c->range_begin, c->range_end, c->list, c->records, image,
-                                       c->final_T, c->n_contrib, c->segments, c->segment_state, c->tile_order))
+                                       c->final_T, c->n_contrib, c->segments, nullptr, c->tile_order))
         return st;
     mark(c, 4, s);
     collect_times(c, 4);

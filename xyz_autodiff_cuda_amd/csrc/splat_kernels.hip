@@ -399,7 +399,7 @@ __global__ void __launch_bounds__(kChunk) render_forward_kernel(
             // colours (a difference of running totals would cancel).
             for (int k = segment - 1; k >= 0; --k) {
                 const float4 own = finished[(k * kPx + p) * kChunk + lane];
-                if (inside)
+                if (inside && segment_state)  // (the pieces' sums are added up in one order whether a backward walk follows or not)
                     segment_state[k * static_cast<std::size_t>(width) * height + at] = float4{own.x, sum[0], sum[1], sum[2]};
                 sum[0] += own.y;
                 sum[1] += own.z;
@@ -870,12 +870,14 @@ int launch_project(hipStream_t s, int G, const float* params, const float* depth
 static unsigned padded_tile_blocks(int tiles) { return static_cast<unsigned>(((tiles + 7) / 8) * 8); }
 
 // Pieces for the backward walk to be done by more wavefronts where a tile each leaves the SIMDs with few; what they cost is
-// the forward pass's states.  Forward + backward with 8 / 4 / 3 / 2 / 1 pieces (us): 10 000 Gaussians at 512 x 512 (1024
-// tiles) 31 + 48 / 30 + 45 / 28 + 45 / 28 + 48 / 25 + 64, 50 000 at 1277 x 719 (3600 tiles) 120 + 157 / 93 + 159 / 84 + 155 /
-// 80 + 157 / 65 + 177.  (The lines were drawn with the kernels before these; at 1024 tiles eight are now 4 us more than four.)
-int render_segments(int width, int height) {
+// the forward pass's states.  A step with 8 / 4 / 2 / 1 pieces (us): 2500 Gaussians at 256 x 256 (256 tiles) 64 / 66 / 79 / 97, 12 000 at
+// 480 x 360 (690) 116 / 121 / 133, 12 000 at 640 x 340 (880) 114 / 118 / 119, at 512 x 512 (1024) 10 000 97 / 93 / 94 / 108, 20 000
+// 146 / 144 / 152 and 30 000, whose lists are long, 171 / 175 / 191 / 226, 10 000 at 700 x 700 (1936) 104 / 94 / 91 / 88 and 30 000
+// 228 / 216 / 229; forward + backward of 50 000 at 1277 x 719 (3600) 277 / 252 / 237 / 242.
+int render_segments(int width, int height, int G) {
     const int tiles = ((width + kTile - 1) / kTile) * ((height + kTile - 1) / kTile);
-    return tiles <= 1024 ? 8 : (tiles <= 2048 ? 4 : (tiles <= 4096 ? 2 : 1));
+    if (tiles <= 960 || (tiles <= 1024 && G > 20 * tiles)) return 8;
+    return tiles <= 2048 ? 4 : (tiles <= 4096 ? 2 : 1);
 }
 
 int launch_render_forward(hipStream_t s, int width, int height, const std::uint32_t* range_begin,
@@ -888,7 +890,7 @@ int launch_render_forward(hipStream_t s, int width, int height, const std::uint3
         hipLaunchKernelGGL(tile_order_kernel, dim3(8), dim3(1024), 0, s, tiles, range_begin, range_end, tile_order);
         XAD_HIP_TRY(hipGetLastError());
     }
-    XAD_REQUIRE(segments >= 1 && segments <= kMaxSegments && (segments == 1 || segment_state), "splat: a split walk needs its per-segment state");
+    XAD_REQUIRE(segments >= 1 && segments <= kMaxSegments, "splat: a split walk takes up to %d segments", kMaxSegments);
     const dim3 grid(padded_tile_blocks(tiles) * kForwardParts), block(kChunk);
     if (segments > 1)
         hipLaunchKernelGGL(render_forward_kernel<true>, grid, block, (segments - 1) * kForwardPixels * kChunk * sizeof(float4), s,

@@ -72,8 +72,9 @@ inline bool orders_tiles(int G) { return G > 4096; }
 // tile_order: null if they do not, else 8 * ceil(tiles / 8) words, written by launch_render_forward (the order, longest list first within
 // each XCD's band of tiles, in which the blocks of both kernels take the tiles) and read by launch_render_backward.
 // Pieces a tile's list is cut into for the backward walk (1, 2, 4 or 8: more for images with few tiles);
-// segment_state holds that many float4 per pixel when it is more than one: [segment][row][column].
-int render_segments(int width, int height);
+// segment_state holds that many float4 per pixel when it is more than one: [segment][row][column] (null in the forward pass:
+// no backward walk follows).
+int render_segments(int width, int height, int G);
 // Also adds the parts of the loss up into loss[0].
 int launch_gaussian_backward(hipStream_t s, int G, const float* params, const float* record_grads, float* grads, double* loss);
 
