@@ -627,6 +627,15 @@ def test_tile_lists_on_both_sides_of_the_binning_rule(gpu, oracle, G, W, H):
     ctx.close()
 
 
+@pytest.mark.parametrize("G,W,H", [
+    (3072, 1024, 512), (3073, 1024, 512),  # 2048 tiles: the most Gaussians whose tiles are tested one by one, and one more
+    (6144, 512, 512), (6145, 512, 512),    # 1024 tiles
+    (6145, 40, 24),
+])
+def test_tile_lists_where_testing_every_tile_ends(gpu, oracle, G, W, H):
+    test_tile_lists_on_both_sides_of_the_binning_rule(gpu, oracle, G, W, H)
+
+
 def test_small_scenes_keep_no_room_for_the_lists_of_supertiles(gpu):
     """Room for 64 Mi pairs is 256 MiB of lists where they are made by testing every tile (the copy per supertile and its
     counts would be twice that again); the enlargement of lists that were cut short works on the same terms."""

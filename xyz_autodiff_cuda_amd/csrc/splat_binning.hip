@@ -16,15 +16,16 @@
 //           64 at a time, one per lane: the mask of the supertile's tiles that a rectangle covers; transposed, lane t
 //           has the word that says which of the 64 cover tile t, and its set bits, in order, are written.
 //
+// Few Gaussians on few tiles are tested one by one instead, also in two launches (test_tiles_kernel, write_lists_kernel).
+//
 // All sizes that depend on the data stay on the device, every store is checked against the capacity of the list, and an
 // overflow is recorded in the status words for the host to see whenever it next waits for the stream.
 //
 // What bounds it: latency, of a block's chain of loads, barriers and LDS accesses, 5 us a launch; with more Gaussians the
-// instructions of fill, most of them for putting pairs in order.  Measured (cover + fill, us; in parentheses as it was before:
-// two launches that tested every tile against every Gaussian in small scenes, seven by way of supertile lists in others):
-// 1000 Gaussians at 640 x 427 4.5 + 6.9 (8.6), 10 000 at 512 x 512 5.1 + 9.5 (22), 50 000 at 1277 x 719 5.5 + 13.4 (44), 100 000
+// instructions of fill, most of them for putting pairs in order.  Measured (cover + fill, us; in parentheses as it was before,
+// seven launches by way of supertile lists): 10 000 Gaussians at 512 x 512 5.1 + 9.5 (22), 50 000 at 1277 x 719 5.5 + 13.4 (44), 100 000
 // at 1920 x 1080 7.3 + 15.4 (65), 200 000 at 2048 x 2048 9.3 + 21 (75).  With all centres within 100 pixels of the middle,
-// the whole of it between events: 15.9 (10.9), 22 (24), 43 (45), 30 (60), 40 (65).
+// the whole of it between events: 22 (24), 43 (45), 30 (60), 40 (65).
 //
 // Replaces, for the tile-binned renderer, what the reference does not have at all: its renderer
 // visits every Gaussian at every pixel (examples/mini-gaussian-splatting/gaussian_splatting_kernel.cu:33-62).
@@ -507,6 +508,112 @@ __global__ void __launch_bounds__(kFillLanes, 8) fill_kernel(FillArgs a, int hel
     }
 }
 
+// ---------------------------------------------------------------------------
+// Few Gaussians.  A block tests one tile against all of them, 64 rectangles to a wavefront at a time and in depth order, and
+// leaves one bit per Gaussian and their count; the second launch adds up the counts of the tiles before its own, and the set
+// bits, in order, are the list.  (In one launch, with room for the lists taken from a counter: 28 us with 1080 tiles and
+// next to no Gaussians, for the atomics on one address.)
+// What bounds it: the latency of a wavefront's chain of loads, and behind it the number of tests.
+// The rule is where the two ways cross.  Both launches between events, us, cover and fill / so: 1000 Gaussians at 640 x 427 (1080
+// tiles) 13.7 / 10.6, 4096 there 16.4 / 14.4, 6000 17.4 / 17.7; 5500 at 512 x 512 15.9 / 15.5; 2000 at 1000 x 500 (2016) 14.4 / 13.4,
+// 4096 there 15.6 / 16.8; 500 at 1000 x 1000 (3969) 13.3 / 15.8, 1500 there 13.6 / 18.2; 4096 at 256 x 256 15.1 / 12.2, 8000 there
+// 17.7 / 17.6, 16 000 21.2 / 26.5.  With all centres within 100 pixels of the middle 1000 at 640 x 427 15.8 / 10.4, 4096 32.7 / 14.3.
+// A training iteration of 1000 at 640 x 427 38.9 / 35.1.
+constexpr int kTestWaves = 4;
+constexpr int kMostTestTiles = 2048, kMostTestChunks = 96, kMostTests = 96 * 1024;  // tiles, chunks of 64 Gaussians, tiles x chunks
+
+__device__ __forceinline__ std::uint32_t sum_over_block(std::uint32_t v, std::uint32_t (&per_wave)[kTestWaves]) {
+    const std::uint32_t of_wave = last_lane(running_sum(v));
+    if ((threadIdx.x & 63) == 0) per_wave[threadIdx.x >> 6] = of_wave;
+    __syncthreads();
+    std::uint32_t total = 0;
+#pragma unroll
+    for (int w = 0; w < kTestWaves; ++w) total += per_wave[w];
+    return total;
+}
+
+__global__ void __launch_bounds__(64 * kTestWaves) test_tiles_kernel(BinPlan p, const TileRect* __restrict__ rects_by_depth,
+                                                                     std::uint64_t* __restrict__ covering,
+                                                                     std::uint32_t* __restrict__ counts) {
+    __shared__ std::uint32_t per_wave[kTestWaves];
+    const int wave = static_cast<int>(threadIdx.x) >> 6, lane = static_cast<int>(threadIdx.x) & 63;
+    const int tile = static_cast<int>(blockIdx.x), tx = tile % p.tiles_x, ty = tile / p.tiles_x;
+    const int chunks = (p.G + 63) / 64;
+    std::uint64_t* mine = covering + static_cast<std::size_t>(tile) * chunks;
+    constexpr int kAhead = 8;  // loads in flight
+    std::uint32_t count = 0;   // of this lane's Gaussians
+    for (int c0 = wave * kAhead; c0 < chunks; c0 += kTestWaves * kAhead) {
+        TileRect r[kAhead];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            const int i = (c0 + k) * 64 + lane;
+            r[k] = TileRect{1, 1, 0, 0};  // covers nothing
+            if (i < p.G) r[k] = rects_by_depth[i];
+        }
+        std::uint64_t answer = 0;
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            const bool covers = tx >= r[k].x0 && tx <= r[k].x1 && ty >= r[k].y0 && ty <= r[k].y1;
+            const std::uint64_t mask = ballot(covers);
+            count += covers ? 1u : 0u;
+            if (lane == k) answer = mask;
+        }
+        if (lane < kAhead && c0 + lane < chunks) mine[c0 + lane] = answer;
+    }
+    const std::uint32_t total = sum_over_block(count, per_wave);
+    if (threadIdx.x == 0) counts[tile] = total;
+}
+
+__global__ void __launch_bounds__(64 * kTestWaves) write_lists_kernel(
+    BinPlan p, const std::uint32_t* __restrict__ by_depth, const std::uint64_t* __restrict__ covering,
+    const std::uint32_t* __restrict__ counts, std::uint32_t* __restrict__ list, std::uint32_t* __restrict__ range_begin,
+    std::uint32_t* __restrict__ range_end, std::uint32_t* __restrict__ status, bool clear_depth_flag) {
+    __shared__ std::uint32_t per_wave[kTestWaves];
+    __shared__ std::uint32_t found[kTestWaves];
+    const int wave = static_cast<int>(threadIdx.x) >> 6, lane = static_cast<int>(threadIdx.x) & 63;
+    const int tile = static_cast<int>(blockIdx.x);
+    const int chunks = (p.G + 63) / 64, share = (chunks + kTestWaves - 1) / kTestWaves;
+    const int begin = wave * share, end = begin + share < chunks ? begin + share : chunks;
+    const std::uint64_t* mine = covering + static_cast<std::size_t>(tile) * chunks;
+
+    std::uint32_t before = 0, here = 0;
+    for (int t = static_cast<int>(threadIdx.x); t < tile; t += 64 * kTestWaves) before += counts[t];
+    for (int c = begin + lane; c < end; c += 64) here += static_cast<std::uint32_t>(__builtin_popcountll(mine[c]));
+    here = last_lane(running_sum(here));
+    if (lane == 0) found[wave] = here;
+    const std::uint32_t first = sum_over_block(before, per_wave);
+    std::uint32_t at = first;
+    for (int w = 0; w < wave; ++w) at += found[w];
+
+    for (int c = begin; c < end; c += 64) {
+        const std::uint64_t answers = c + lane < end ? mine[c + lane] : 0;
+        for (std::uint64_t todo = ballot(answers != 0); todo != 0; todo &= todo - 1) {
+            const int k = __builtin_ctzll(todo);
+            const std::uint64_t mask =
+                static_cast<std::uint64_t>(static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(answers >> 32), k))) << 32 |
+                static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(answers), k));
+            if ((mask >> lane) & 1) {
+                const std::uint32_t to = at + static_cast<std::uint32_t>(__builtin_popcountll(mask & ((std::uint64_t(1) << lane) - 1)));
+                if (to < p.capacity) list[to] = by_depth[(c + k) * 64 + lane];
+            }
+            at += static_cast<std::uint32_t>(__builtin_popcountll(mask));
+        }
+    }
+    if (threadIdx.x == 0) {
+        // a list that does not fit is cut short; the pair count stays exact
+        const std::uint32_t behind = first + counts[tile];
+        range_begin[tile] = first < p.capacity ? first : p.capacity;
+        range_end[tile] = behind < p.capacity ? behind : p.capacity;
+        if (blockIdx.x == gridDim.x - 1) {
+            const bool overflow = behind > p.capacity;
+            status[kStatusPairs] = behind;
+            status[kStatusOverflow] = overflow ? 1u : 0u;
+            if (overflow) atomicMax(status + kStatusOverflowSticky, behind);
+            if (clear_depth_flag) status[kStatusDepthChanged] = 0;
+        }
+    }
+}
+
 constexpr int kFillHelpers = 256;  // a block per compute unit
 constexpr std::size_t kSlabBytes = std::size_t(64) << 20;  // of words kept between cover and fill, if a slice needs no more
 
@@ -524,6 +631,7 @@ BinPlan make_bin_plan(int G, int tiles_x, int tiles_y, std::uint32_t capacity) {
     p.supers = p.groups * 64;  // numbered group by group; those beyond the image stay empty
     p.capacity = capacity;
     p.chunks = (G + 63) / 64;
+    p.tests_tiles = tiles_x * tiles_y <= kMostTestTiles && p.chunks <= kMostTestChunks && p.chunks * tiles_x * tiles_y <= kMostTests;
     // cover: a chunk per wavefront at least, up to 64 ranges (every one adds to the same totals, one after the other), and none
     // beyond what a fill block takes
     const int wanted_range = ((p.chunks + 63) / 64 + kCoverWaves - 1) / kCoverWaves * kCoverWaves;
@@ -543,11 +651,23 @@ BinPlan make_bin_plan(int G, int tiles_x, int tiles_y, std::uint32_t capacity) {
     return p;
 }
 
-std::size_t bin_covering_words(const BinPlan& p) { return static_cast<std::size_t>(p.supers) * p.slab_chunks; }
-std::size_t bin_counts_words(const BinPlan& p) { return static_cast<std::size_t>(p.supers) * 64 * p.ranges; }
+std::size_t bin_covering_words(const BinPlan& p) {
+    if (p.tests_tiles) return static_cast<std::size_t>(p.tiles_x) * p.tiles_y * p.chunks;
+    return static_cast<std::size_t>(p.supers) * p.slab_chunks;
+}
+std::size_t bin_counts_words(const BinPlan& p) {
+    if (p.tests_tiles) return static_cast<std::size_t>(p.tiles_x) * p.tiles_y;
+    return static_cast<std::size_t>(p.supers) * 64 * p.ranges;
+}
 
 int launch_cover(hipStream_t s, const BinPlan& p, const TileRect* rects_by_depth, const BinScratch& scratch) {
     XAD_REQUIRE(p.G > 0 && p.supers > 0 && p.ranges > 0, "splat binning: empty plan");
+    if (p.tests_tiles) {
+        hipLaunchKernelGGL(test_tiles_kernel, dim3(static_cast<unsigned>(p.tiles_x * p.tiles_y)), dim3(64 * kTestWaves), 0, s, p,
+                           rects_by_depth, scratch.covering, scratch.counts);
+        XAD_HIP_TRY(hipGetLastError());
+        return XAD_OK;
+    }
     const dim3 grid(static_cast<unsigned>(p.groups) * static_cast<unsigned>(p.ranges)), block(64 * kCoverWaves);
     if (p.slab_slices >= p.slices)
         hipLaunchKernelGGL((cover_kernel<true, true>), grid, block, 0, s, p, 0, rects_by_depth, scratch.covering, scratch.counts,
@@ -562,6 +682,12 @@ int launch_cover(hipStream_t s, const BinPlan& p, const TileRect* rects_by_depth
 int launch_fill(hipStream_t s, const BinPlan& p, const std::uint32_t* by_depth, const TileRect* rects_by_depth, const BinScratch& scratch,
                 std::uint32_t* list, std::uint32_t* range_begin, std::uint32_t* range_end, std::uint32_t* status, bool clear_depth_flag) {
     XAD_REQUIRE(p.capacity > 0, "splat binning: no room for lists");
+    if (p.tests_tiles) {
+        hipLaunchKernelGGL(write_lists_kernel, dim3(static_cast<unsigned>(p.tiles_x * p.tiles_y)), dim3(64 * kTestWaves), 0, s, p,
+                           by_depth, scratch.covering, scratch.counts, list, range_begin, range_end, status, clear_depth_flag);
+        XAD_HIP_TRY(hipGetLastError());
+        return XAD_OK;
+    }
     const bool one_slab = p.slab_slices >= p.slices;
     const unsigned groups = static_cast<unsigned>(p.groups), supers = static_cast<unsigned>(p.supers);
     for (int slice = 0; slice < p.slices; slice += p.slab_slices) {

@@ -38,13 +38,15 @@ struct BinPlan {
     int supers;              // supertile numbers: 64 per group, whether inside the image or not
     std::uint32_t capacity;  // (tile, Gaussian) pairs the lists can hold
     int chunks;                     // of 64 Gaussians
+    bool tests_tiles;               // few Gaussians: every tile is tested against all of them; what follows is not used then
     int range_chunks, ranges;       // that a block of the first launch takes, and how many such ranges
     int slice_ranges, slice_chunks, slices;  // ranges and chunks that a block of the second launch takes, and how many such slices
     int slab_slices, slab_chunks;   // slices and chunks whose words are kept between the launches
 };
 struct BinScratch {
-    std::uint64_t* covering = nullptr;  // bin_covering_words: per (supertile, chunk of the slab), a bit per Gaussian that reaches it
-    std::uint32_t* counts = nullptr;    // bin_counts_words: pairs per (range, supertile, tile)
+    // bin_covering_words: per (supertile, chunk of the slab), a bit per Gaussian that reaches it; per (tile, chunk) if tiles are tested
+    std::uint64_t* covering = nullptr;
+    std::uint32_t* counts = nullptr;    // bin_counts_words: pairs per (range, supertile, tile), or per tile
     std::uint32_t* totals = nullptr;    // 2 x supers: pairs per supertile, Gaussians that reach it
 };
 BinPlan make_bin_plan(int G, int tiles_x, int tiles_y, std::uint32_t capacity);
