@@ -42,11 +42,40 @@ def _check(gpu, depth):
     np.testing.assert_array_equal(rank, inverse)
 
 
-# (up to 4096 keys one block sorts alone, with 2 or 4 keys per lane; above, tiles of 4096 keys)
+# (up to 12 288 keys every key is compared with all; up to 262 144 bins between samples; above, tiles of 4096 keys)
 @pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 511, 512, 513, 1024, 1025, 2047, 2048, 2049, 4096, 4097, 8192, 8193, 10_000, 12_287,
                                12_288, 12_289, 16_384, 200_000, 1_000_003])
 def test_uniform_depths(gpu, n):
     _check(gpu, np.random.default_rng(n).uniform(0.0, 1.0, n))
+
+
+@pytest.mark.parametrize("n", [12_289, 12_544, 12_545, 100_000, 262_143, 262_144, 262_145])
+def test_where_keys_are_sorted_by_samples(gpu, n):
+    r = np.random.default_rng(n)
+    _check(gpu, r.uniform(0.0, 1.0, n))
+    _check(gpu, r.integers(0, 3, n).astype(np.float32))     # a tie of many bins
+    d = r.uniform(0.0, 1.0, n).astype(np.float32)
+    d[n // 5:] = d[0]
+    _check(gpu, d)
+
+
+def test_a_bin_of_nearly_all_keys(gpu):
+    """Depths made so that no sample falls among most of them: the bins' sizes decide the time, not the order."""
+    n = 13_000
+    samples = (n + 255) // 256 * 8
+    s = np.arange(samples, dtype=np.uint64)
+    low, high = s * np.uint64(n) // np.uint64(samples), (s + np.uint64(1)) * np.uint64(n) // np.uint64(samples)
+    mask = np.uint64(0xFFFFFFFF)
+    h = s * np.uint64(0x9E3779B1) & mask
+    h ^= h >> np.uint64(15)
+    h = h * np.uint64(0x85EBCA77) & mask
+    h ^= h >> np.uint64(13)
+    sampled = low + (h * (high - low) >> np.uint64(32))
+    r = np.random.default_rng(7)
+    d = r.uniform(0.4, 0.6, n).astype(np.float32)
+    d[r.integers(0, n, n // 3)] = 0.5
+    d[sampled.astype(np.int64)] = r.integers(0, 2, samples).astype(np.float32)
+    _check(gpu, d)
 
 
 @pytest.mark.parametrize("n", [5, 2048, 9000, 50_000, 300_001])

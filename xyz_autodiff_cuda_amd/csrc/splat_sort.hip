@@ -1,7 +1,17 @@
-// The depth order of the Gaussians: a stable least-significant-digit radix sort of (depth bits, index),
-// written for this size of problem (10^4 to 10^6 keys of 32 bits), where the time is launches and
-// round trips to memory, not bandwidth.  Five launches in all (one, by one block, up to 4096 keys: see
-// sort_small_kernel), no library primitive, no host read-back:
+// The depth order of the Gaussians: a stable sort of (depth bits, index), written for this size of problem (10^2 to 10^6 keys of
+// 32 bits), where the time is launches and round trips to memory, not bandwidth.  No library primitive, no host read-back.
+//
+//   up to 12 288 keys    the place of a key is the number of keys before it: compared with all of them, one launch
+//                        (rank_directly_kernel)
+//   up to 262 144 keys   bins between splitters from a sorted sample, and the place within the bin likewise: four launches
+//                        (SampleSort)
+//   more                 a least-significant-digit radix sort of five launches
+//
+// Measured on MI355X, the whole sort, as the difference between a splatting step that orders and one that does not, us (in
+// parentheses by radix passes: of one block up to 4096 keys, of tiles above): 1000 keys 2 (4), 4096 5.5 (19), 8192 12 (45), 10 000
+// 16 (47), 12 288 18 (48), 20 000 22 (44), 50 000 26 (60), 100 000 33 (71), 200 000 45 (64), 262 144 58 (71); 400 000 85 in either.
+//
+// The radix sort:
 //
 //   prepare   one lane per Gaussian: the order-preserving bits of its depth, a copy of the depth (what
 //             the order was computed from), and the counts of the three lower 8-bit digits (a histogram
@@ -30,20 +40,19 @@
 // Sizes: a pass is a chain of round trips to memory (ticket, keys, look-back) whatever the size of a
 // tile; the look-back is as long as there are tiles; and the rounds of a wavefront are serial.  So the
 // tiles are large (4096 keys: 49 of them at 2 x 10^5 keys, three looks of 16 words) and wide rather than
-// deep (sixteen wavefronts of four rounds).  Measured on MI355X, the whole sort at 2 x 10^5 keys, as the
-// difference between a splatting step that orders and one that does not: 256 lanes x 8 rounds with a
+// deep (sixteen wavefronts of four rounds).  Measured, the whole sort at 2 x 10^5 keys: 256 lanes x 8 rounds with a
 // look-back of one word at a time 0.32 ms; the same, sixteen words at a time 0.10 ms; 1024 lanes x 16
 // rounds 0.20 ms (one compute unit does the work of four); 1024 x 8 0.107; 512 x 8 0.070; 1024 x 4 with
 // looks of 8, 16, 24, 32 words 0.071, 0.059-0.064, 0.068, 0.076 ms (more words per look is more code and
 // more registers: with 64 and a wait loop per word a pass spent 20 us fetching instructions); tiles
 // taken by block index instead of by ticket 0.078 (blocks do not start in index order, so more of
-// them wait).  At 10^4 keys (three tiles) 0.05 ms: five launches of about 10 us.  The five steps in one
+// them wait).  The five steps in one
 // launch, with a barrier across the (resident) blocks and agent-scope fences between them: 0.23 ms at
-// 2 x 10^5 keys, 0.085 at 10^4 -- the release and acquire of plain data across the XCDs' L2 caches
+// 2 x 10^5 keys -- the release and acquire of plain data across the XCDs' L2 caches
 // (write back, invalidate) cost far more than the launch boundaries they replace.
 //
-// Equal depths keep index order (every pass is stable and the first one takes the keys in index
-// order).  Order of the keys: the total order of the bit patterns in sign-magnitude reading, with
+// Equal depths keep index order (every radix pass is stable and the first one takes the keys in index
+// order; comparisons take the index as well).  Order of the keys: the total order of the bit patterns in sign-magnitude reading, with
 // -0.0 and +0.0 taken as the same depth; a NaN sorts by its bits, before everything when its sign bit
 // is set and after everything when it is not.
 //
@@ -310,125 +319,250 @@ __global__ void __launch_bounds__(kSortBlock) sort_pass_kernel(int G, int pass, 
     }
 }
 
-// The whole sort in one block, for scenes of up to kSmallSortKeys Gaussians: no tickets, no look-back, no
-// histograms in memory, one launch instead of five (which cost about 10 us each whatever the size).  Every
-// lane keeps kRounds keys in registers; a pass ranks them as above, scans the 256 digit counts of the block,
-// writes every key and value to its place in `keys` / `values` (global scratch: the block's own stores, read
-// back by the same block after a barrier) and takes its next keys from there; the last pass writes the order
-// and its inverse instead.  Measured (kernel time): 14.6 us with two keys per lane, 26.5 with four, 51 with
-// eight, 74 with twelve, against 52 us for the five launches up to 12 288 keys: a round of ranking costs 1.5 us
-// per pass wherever it runs, and the tiles of the five launches run theirs side by side on different compute
-// units.  So one block sorts alone up to four keys per lane.
-constexpr unsigned kSmallSortMaxRounds = 4;
-constexpr unsigned kSmallSortKeys = kSortBlock * kSmallSortMaxRounds;  // 4096
+// ---------------------------------------------------------------------------
+// Up to kDirectKeys keys: the place of a key is the number of keys before it, counted by comparing it with all of them, in one
+// launch.  A block has 64 keys, one per lane, and all keys in LDS, a sixteenth of them for every wavefront: two instructions a
+// comparison and a quarter of a broadcast read.  Equal keys are taken in index order: those of lower index count if they are not
+// above, those of higher index if they are below, and only in the block's own 64 does it matter which is which.
+// kSamples: the keys are samples of the depths (sample_index), of which every kPerSplitter-th in order becomes a splitter.
+// What bounds it: the comparisons, 14 cycles of a SIMD for 64 of them where 8 are two instructions (the mask that a comparison leaves
+// has to be waited for).  Measured: 19 us for 10 000 keys.  By ballots, a key against 64 at a time and counts on the scalar unit:
+// 24.  Above 12 288 keys the sample sort is faster: 15 360 keys 23.3 so, 21.0 with it.
+constexpr unsigned kDirectKeys = 12288;
+constexpr unsigned kPerSplitter = 8;
+constexpr unsigned kBinKeys = 256;  // on average
+constexpr unsigned kMostBins = 1024;
+constexpr unsigned kSampleSortKeys = kMostBins * kBinKeys;
 
-template <unsigned kRounds>
-__global__ void __launch_bounds__(kSortBlock) sort_small_kernel(int G, const float* __restrict__ depth, std::uint32_t* keys,
-                                                                std::uint32_t* values, std::uint32_t* __restrict__ by_depth,
-                                                                std::uint32_t* __restrict__ rank,
-                                                                float* __restrict__ ordered_depth) {
-    __shared__ std::uint32_t count[kSortWaves][kDigits];
-    __shared__ std::uint32_t digit_base[kDigits];
-    __shared__ std::uint32_t wave_sum[kDigits / 64];
-    const unsigned t = threadIdx.x, lane = t & 63u, w = t >> 6;
-    const unsigned chunk = w * 64u * kRounds;  // a wavefront's keys are contiguous; in round i lane l holds key i * 64 + l of them
-    const unsigned n = static_cast<unsigned>(G);
-    const std::uint64_t below = (std::uint64_t(1) << lane) - 1;
-    std::uint32_t key[kRounds], value[kRounds], place[kRounds];
+// One index in each of `samples` equal stretches of [0, G), at a place that a hash of the stretch's number says (a fixed stride
+// would be at the mercy of depths with the same period).
+__device__ __forceinline__ std::uint32_t sample_index(std::uint32_t s, std::uint32_t samples, std::uint32_t G) {
+    const std::uint32_t lo = static_cast<std::uint32_t>(static_cast<std::uint64_t>(s) * G / samples);
+    const std::uint32_t hi = static_cast<std::uint32_t>(static_cast<std::uint64_t>(s + 1) * G / samples);
+    std::uint32_t h = s * 0x9E3779B1u;
+    h ^= h >> 15;
+    h *= 0x85EBCA77u;
+    h ^= h >> 13;
+    return lo + static_cast<std::uint32_t>(static_cast<std::uint64_t>(h) * (hi - lo) >> 32);
+}
+
+__device__ __forceinline__ std::uint64_t with_index(std::uint32_t key, std::uint32_t index) {
+    return static_cast<std::uint64_t>(key) << 32 | index;
+}
+
+template <bool kSamples>
+__global__ void __launch_bounds__(kSortBlock) rank_directly_kernel(std::uint32_t n, std::uint32_t G, const float* __restrict__ depth,
+                                                                   std::uint32_t* __restrict__ by_depth,
+                                                                   std::uint32_t* __restrict__ rank,
+                                                                   float* __restrict__ ordered_depth,
+                                                                   std::uint64_t* __restrict__ splitters,
+                                                                   std::uint32_t* __restrict__ totals, std::uint32_t bins) {
+    extern __shared__ uint4 four_keys[];  // all keys, rounded up to a multiple of 4 per wavefront
+    __shared__ std::uint32_t counted[kSortWaves][64];
+    std::uint32_t* keys = reinterpret_cast<std::uint32_t*>(four_keys);
+    const std::uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    const std::uint32_t share = (n + 4 * kSortWaves - 1) / (4 * kSortWaves) * 4;  // of a wavefront
+    constexpr int kAhead = 8;  // loads in flight
+    for (std::uint32_t j0 = t; j0 < share * kSortWaves; j0 += kAhead * kSortBlock) {
+        float d[kAhead];
 #pragma unroll
-    for (unsigned i = 0; i < kRounds; ++i) {
-        const unsigned at = chunk + i * 64 + lane;
-        key[i] = 0u;
-        value[i] = at;
-        if (at < n) {
-            const float d = depth[at];
-            key[i] = depth_key(d);
-            ordered_depth[at] = d;
+        for (int k = 0; k < kAhead; ++k) {
+            const std::uint32_t j = j0 + k * kSortBlock;
+            d[k] = j < n ? depth[kSamples ? sample_index(j, n, G) : j] : 0.0f;
+        }
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            const std::uint32_t j = j0 + k * kSortBlock;
+            if (j < share * kSortWaves) keys[j] = j < n ? depth_key(d[k]) : ~0u;  // (those beyond the end are never below)
         }
     }
-#pragma unroll 1
-    for (unsigned pass = 0; pass < static_cast<unsigned>(kPasses); ++pass) {
-        const unsigned shift = 8u * pass;
+    if constexpr (kSamples)
+        for (std::uint32_t j = blockIdx.x * kSortBlock + t; j < bins; j += gridDim.x * kSortBlock) totals[j] = 0;
+    __syncthreads();
+    const std::uint32_t i0 = blockIdx.x * 64u, i = i0 + lane;
+    const std::uint32_t key = i < n ? keys[i] : 0u;
+    const std::uint32_t begin = w * share, end = begin + share;
+    const std::uint32_t own = end < i0 ? end : (begin > i0 ? begin : i0);                    // where the block's own keys begin
+    const std::uint32_t behind = end < i0 + 64 ? end : (begin > i0 + 64 ? begin : i0 + 64);  // and end, if within the share
+    std::uint32_t count = 0;
+#pragma unroll 4
+    for (std::uint32_t j = begin; j < own; j += 4) {
+        const uint4 k = four_keys[j / 4];
+        count += k.x <= key;
+        count += k.y <= key;
+        count += k.z <= key;
+        count += k.w <= key;
+    }
+    for (std::uint32_t j = own; j < behind; ++j) count += keys[j] < key || (keys[j] == key && j < i);
+#pragma unroll 4
+    for (std::uint32_t j = behind; j < end; j += 4) {
+        const uint4 k = four_keys[j / 4];
+        count += k.x < key;
+        count += k.y < key;
+        count += k.z < key;
+        count += k.w < key;
+    }
+    counted[w][lane] = count;
+    __syncthreads();
+    if (w != 0 || i >= n) return;
+    std::uint32_t at = 0;
 #pragma unroll
-        for (unsigned k = 0; k < kSortWaves * kDigits / kSortBlock; ++k) (&count[0][0])[k * kSortBlock + t] = 0;
-        __syncthreads();
-#pragma unroll
-        for (unsigned i = 0; i < kRounds; ++i) {
-            const bool valid = chunk + i * 64 + lane < n;
-            const std::uint32_t digit = (key[i] >> shift) & 255u;
-            std::uint64_t same = ballot(valid);
-#pragma unroll
-            for (unsigned bit = 0; bit < 8; ++bit) {
-                const std::uint64_t set = ballot(((digit >> bit) & 1u) != 0);
-                same &= ((digit >> bit) & 1u) ? set : ~set;
-            }
-            volatile std::uint32_t* counter = &count[w][digit];
-            const std::uint32_t before = *counter;
-            place[i] = before + static_cast<std::uint32_t>(__builtin_popcountll(same & below));
-            if (valid && (same & below) == 0) *counter = before + static_cast<std::uint32_t>(__builtin_popcountll(same));
+    for (unsigned k = 0; k < kSortWaves; ++k) at += counted[k][lane];
+    if constexpr (kSamples) {
+        if (at % kPerSplitter == 0 && at != 0) splitters[at / kPerSplitter - 1] = with_index(key, sample_index(i, n, G));
+    } else {
+        by_depth[at] = i;
+        rank[i] = at;
+        ordered_depth[i] = depth[i];
+    }
+}
+
+// Up to kSampleSortKeys keys: bins between splitters taken from a sorted sample, then the place of every key within its bin by
+// comparing it with all of that bin.  Key and index together are compared, so no two are equal, and many equal depths fall into
+// many bins.  A bin is as large as the sample leaves it (some hundred keys; all of them only if the depths were made with the hash in
+// hand, and then it is slow, not wrong).  Four launches, none of which waits for another block: the samples (rank_directly_kernel),
+// the bin of every key and the room that a block's keys take in each, the keys to their bins, and the places within the bins.
+// What bounds it: latency; launches of 12 + 5 + 5 + 13 us at 100 000 keys, 19 + 7 + 6 + 15 at 200 000.  Four samples to a splitter
+// instead of eight: 10 and 13 us for the first launch, but bins of more than 1000 keys now and then, 35 us instead of 23 where one
+// was met.
+struct SampleSort {
+    std::uint32_t G, bins, tile;  // tile: keys of a block in the two launches in the middle
+    std::uint64_t* splitters;     // bins - 1
+    std::uint32_t* totals;        // bins: keys in each
+    std::uint32_t* base;          // (block, bin): where the block's keys begin in the bin
+};
+
+__global__ void __launch_bounds__(kSortBlock) find_bins_kernel(SampleSort a, const float* __restrict__ depth,
+                                                               std::uint32_t* __restrict__ found, float* __restrict__ ordered_depth) {
+    __shared__ std::uint64_t splitters[kMostBins];
+    __shared__ std::uint32_t count[kMostBins];
+    const std::uint32_t t = threadIdx.x;
+    if (t < a.bins) {
+        splitters[t] = t + 1 < a.bins ? a.splitters[t] : ~std::uint64_t(0);
+        count[t] = 0;
+    }
+    __syncthreads();
+    const std::uint32_t begin = blockIdx.x * a.tile, end = begin + a.tile < a.G ? begin + a.tile : a.G;
+    for (std::uint32_t i = begin + t; i < end; i += kSortBlock) {
+        const float d = depth[i];
+        const std::uint64_t key = with_index(depth_key(d), i);
+        std::uint32_t bin = 0;  // the number of splitters that are not above the key
+        for (std::uint32_t n = a.bins - 1; n > 0;) {
+            const std::uint32_t half = (n + 1) / 2;
+            const bool above = splitters[bin + half - 1] > key;
+            bin += above ? 0 : half;
+            n = above ? half - 1 : n - half;
         }
-        __syncthreads();
-        // lane d of the block (the first 256): digit d.  Offsets of the wavefronts, then of the digits.
-        std::uint32_t inclusive = 0, total = 0;
-        if (t < kDigits) {
+        found[i] = bin << 16 | atomicAdd(&count[bin], 1u);
+        ordered_depth[i] = d;
+    }
+    __syncthreads();
+    if (t < a.bins && count[t] != 0) a.base[blockIdx.x * a.bins + t] = atomicAdd(a.totals + t, count[t]);
+}
+
+__global__ void __launch_bounds__(kSortBlock) fill_bins_kernel(SampleSort a, const float* __restrict__ depth,
+                                                               const std::uint32_t* __restrict__ found,
+                                                               std::uint32_t* __restrict__ keys, std::uint32_t* __restrict__ indices) {
+    __shared__ std::uint32_t at[kMostBins];
+    __shared__ std::uint32_t of_wave[kSortWaves];
+    const std::uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    const std::uint32_t total = t < a.bins ? a.totals[t] : 0;
+    const std::uint32_t base = t < a.bins ? a.base[blockIdx.x * a.bins + t] : 0;  // (unset and unused where the block has no key)
+    std::uint32_t sum = total;
 #pragma unroll
-            for (unsigned k = 0; k < kSortWaves; ++k) {
-                const std::uint32_t c = count[k][t];
-                count[k][t] = total;
-                total += c;
-            }
-            inclusive = total;
+    for (unsigned step = 1; step < 64; step *= 2) {
+        const std::uint32_t other = __shfl_up(sum, step, 64);
+        if (lane >= step) sum += other;
+    }
+    if (lane == 63) of_wave[w] = sum;
+    __syncthreads();
+    sum -= total;
 #pragma unroll
-            for (unsigned step = 1; step < 64; step *= 2) {
-                const std::uint32_t other = __shfl_up(inclusive, step, 64);
-                if (lane >= step) inclusive += other;
-            }
-            if (lane == 63) wave_sum[w] = inclusive;
-        }
-        __syncthreads();
-        if (t < kDigits) {
-            std::uint32_t smaller_digits = inclusive - total;
+    for (unsigned k = 0; k < kSortWaves; ++k) sum += k < w ? of_wave[k] : 0u;
+    at[t] = sum + base;
+    __syncthreads();
+    const std::uint32_t begin = blockIdx.x * a.tile, end = begin + a.tile < a.G ? begin + a.tile : a.G;
+    for (std::uint32_t i = begin + t; i < end; i += kSortBlock) {
+        const std::uint32_t f = found[i];
+        const std::uint32_t to = at[f >> 16] + (f & 0xffffu);
+        keys[to] = depth_key(depth[i]);
+        indices[to] = i;
+    }
+}
+
+constexpr std::uint32_t kBinParts = 4;     // that the comparisons of 64 keys are dealt out in
+constexpr std::uint32_t kBinTile = 1024;   // keys of the bin in LDS
+
+__global__ void __launch_bounds__(kSortBlock) rank_in_bins_kernel(SampleSort a, const std::uint32_t* __restrict__ keys,
+                                                                  const std::uint32_t* __restrict__ indices,
+                                                                  std::uint32_t* __restrict__ by_depth,
+                                                                  std::uint32_t* __restrict__ rank) {
+    __shared__ __align__(16) std::uint64_t own[kBinTile], others[kBinTile];
+    __shared__ std::uint32_t counted[kBinTile];
+    __shared__ std::uint32_t before[kSortWaves];
+    const std::uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    std::uint32_t sum = t < blockIdx.x ? a.totals[t] : 0;
+    const std::uint32_t m = a.totals[blockIdx.x];
 #pragma unroll
-            for (unsigned k = 0; k < kDigits / 64; ++k) smaller_digits += k < w ? wave_sum[k] : 0u;
-            digit_base[t] = smaller_digits;
-        }
-        __syncthreads();
-        const bool last = pass + 1 == static_cast<unsigned>(kPasses);
+    for (int step = 32; step > 0; step /= 2) sum += __shfl_xor(sum, step, 64);
+    if (lane == 0) before[w] = sum;
+    __syncthreads();
+    std::uint32_t start = 0;
 #pragma unroll
-        for (unsigned i = 0; i < kRounds; ++i) {
-            if (chunk + i * 64 + lane < n) {
-                const std::uint32_t digit = (key[i] >> shift) & 255u;
-                const std::uint32_t at = digit_base[digit] + count[w][digit] + place[i];
-                if (at < n) {  // always: the places of n keys are a permutation of [0, n)
-                    if (last) {
-                        by_depth[at] = value[i];
-                        rank[value[i]] = at;
-                    } else {
-                        keys[at] = key[i];
-                        values[at] = value[i];
-                    }
+    for (unsigned k = 0; k < kSortWaves; ++k) start += before[k];
+
+    const auto stage = [&](std::uint64_t* tile, std::uint32_t j0) {  // (keys beyond the end are never below)
+        const std::uint32_t j = j0 + t;
+        tile[t] = j < m ? with_index(keys[start + j], indices[start + j]) : ~std::uint64_t(0);
+    };
+    static_assert(kBinTile == kSortBlock, "a lane stages one key");
+    for (std::uint32_t i0 = 0; i0 < m; i0 += kBinTile) {
+        const std::uint32_t mine = m - i0 < kBinTile ? m - i0 : kBinTile;
+        stage(own, i0);
+        counted[t] = 0;
+        for (std::uint32_t j0 = 0; j0 < m; j0 += kBinTile) {
+            if (j0 != i0) stage(others, j0);
+            __syncthreads();
+            const std::uint64_t* tile = j0 != i0 ? others : own;
+            const std::uint32_t here = m - j0 < kBinTile ? m - j0 : kBinTile;
+            const std::uint32_t share = (here + 2 * kBinParts - 1) / (2 * kBinParts) * 2;
+            for (std::uint32_t unit = w; unit < (mine + 63) / 64 * kBinParts; unit += kSortWaves) {
+                const std::uint32_t i = unit / kBinParts * 64 + lane, begin = unit % kBinParts * share;
+                const std::uint64_t key = own[i];
+                std::uint32_t count = 0;
+#pragma unroll 8
+                for (std::uint32_t j = begin; j < begin + share; j += 2) {
+                    const ulonglong2 k = *reinterpret_cast<const ulonglong2*>(tile + j);
+                    count += k.x < key;
+                    count += k.y < key;
                 }
+                atomicAdd(&counted[i], count);
             }
+            __syncthreads();
         }
-        if (last) break;
-        __syncthreads();  // the block's stores are visible to the block
-#pragma unroll
-        for (unsigned i = 0; i < kRounds; ++i) {
-            const unsigned at = chunk + i * 64 + lane;
-            if (at < n) {
-                key[i] = keys[at];
-                value[i] = values[at];
-            }
+        if (t < mine) {
+            const std::uint32_t at = start + counted[t], index = static_cast<std::uint32_t>(own[t]);
+            by_depth[at] = index;
+            rank[index] = at;
         }
+        __syncthreads();
     }
 }
 
-template <unsigned kRounds>
-void launch_small_sort(hipStream_t s, int G, const float* depth, std::uint32_t* keys, std::uint32_t* values,
-                       std::uint32_t* by_depth, std::uint32_t* rank, float* ordered_depth) {
-    hipLaunchKernelGGL(sort_small_kernel<kRounds>, dim3(1), dim3(kSortBlock), 0, s, G, depth, keys, values, by_depth, rank,
-                       ordered_depth);
+bool sorts_directly(int G) { return static_cast<unsigned>(G) <= kDirectKeys; }
+bool sorts_by_samples(int G) { return !sorts_directly(G) && static_cast<unsigned>(G) <= kSampleSortKeys; }
+
+SampleSort plan_sample_sort(int G, std::uint32_t* work) {
+    SampleSort a{};
+    a.G = static_cast<std::uint32_t>(G);
+    a.bins = (a.G + kBinKeys - 1) / kBinKeys;
+    a.tile = kSortBlock;
+    a.splitters = reinterpret_cast<std::uint64_t*>(work + kStateAt);
+    a.totals = work + kStateAt + 2 * kMostBins;
+    a.base = a.totals + kMostBins;
+    return a;
 }
+unsigned sample_sort_blocks(const SampleSort& a) { return (a.G + a.tile - 1) / a.tile; }
 
 unsigned sort_tiles(int G) { return static_cast<unsigned>((static_cast<std::size_t>(G) + kSortTile - 1) / kSortTile); }
 
@@ -437,6 +571,11 @@ unsigned sort_tiles(int G) { return static_cast<unsigned>((static_cast<std::size
 std::size_t depth_sort_gave_up_offset() { return kGaveUpAt * sizeof(std::uint32_t); }
 
 std::size_t depth_sort_temp_bytes(int G) {
+    if (sorts_directly(G)) return kStateAt * sizeof(std::uint32_t);
+    if (sorts_by_samples(G)) {
+        const SampleSort a = plan_sample_sort(G, nullptr);
+        return (kStateAt + 3 * kMostBins + static_cast<std::size_t>(sample_sort_blocks(a)) * a.bins) * sizeof(std::uint32_t);
+    }
     return (kStateAt + static_cast<std::size_t>(kPasses) * sort_tiles(G) * kDigits) * sizeof(std::uint32_t);
 }
 
@@ -446,16 +585,31 @@ int sort_by_depth(hipStream_t s, void* temp, std::size_t temp_bytes, const float
     XAD_REQUIRE(G > 0 && static_cast<std::uint32_t>(G) <= kCountMask, "depth sort: %d keys do not fit the 30-bit counts", G);
     XAD_REQUIRE(temp && temp_bytes >= depth_sort_temp_bytes(G), "depth sort: workspace of %zu bytes, %zu needed", temp_bytes,
                 depth_sort_temp_bytes(G));
-    if (static_cast<unsigned>(G) <= kSmallSortKeys) {
-        const unsigned rounds = (static_cast<unsigned>(G) + kSortBlock - 1) / kSortBlock;
-        if (rounds <= 2)
-            launch_small_sort<2>(s, G, depth, keys_a, values_a, by_depth, rank, ordered_depth);
-        else
-            launch_small_sort<kSmallSortMaxRounds>(s, G, depth, keys_a, values_a, by_depth, rank, ordered_depth);
+    std::uint32_t* work = static_cast<std::uint32_t*>(temp);
+    const std::uint32_t n = static_cast<std::uint32_t>(G);
+    static_assert(kDirectKeys * sizeof(std::uint32_t) <= (48u << 10) && kMostBins * kPerSplitter <= kDirectKeys, "in LDS beside the counts");
+    const auto lds_of = [](std::uint32_t keys) { return (keys + 4 * kSortWaves - 1) / (4 * kSortWaves) * (4 * kSortWaves) * sizeof(std::uint32_t); };
+    if (sorts_directly(G)) {
+        hipLaunchKernelGGL(rank_directly_kernel<false>, dim3((n + 63) / 64), dim3(kSortBlock), lds_of(n), s, n, n, depth, by_depth, rank,
+                           ordered_depth, nullptr, nullptr, 0u);
         XAD_HIP_TRY(hipGetLastError());
         return XAD_OK;
     }
-    std::uint32_t* work = static_cast<std::uint32_t*>(temp);
+    if (sorts_by_samples(G)) {
+        const SampleSort a = plan_sample_sort(G, work);
+        const std::uint32_t samples = a.bins * kPerSplitter;
+        const dim3 blocks(sample_sort_blocks(a));
+        hipLaunchKernelGGL(rank_directly_kernel<true>, dim3((samples + 63) / 64), dim3(kSortBlock), lds_of(samples), s, samples, n, depth,
+                           nullptr, nullptr, nullptr, a.splitters, a.totals, a.bins);
+        XAD_HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(find_bins_kernel, blocks, dim3(kSortBlock), 0, s, a, depth, values_a, ordered_depth);
+        XAD_HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(fill_bins_kernel, blocks, dim3(kSortBlock), 0, s, a, depth, values_a, keys_b, keys_a);
+        XAD_HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(rank_in_bins_kernel, dim3(a.bins), dim3(kSortBlock), 0, s, a, keys_b, keys_a, by_depth, rank);
+        XAD_HIP_TRY(hipGetLastError());
+        return XAD_OK;
+    }
     const dim3 grid(sort_tiles(G)), block(kSortBlock);
     const std::size_t state_words = static_cast<std::size_t>(kPasses) * sort_tiles(G) * kDigits;
     hipLaunchKernelGGL(sort_prepare_kernel, grid, block, 0, s, G, depth, keys_a, ordered_depth, work, state_words);
