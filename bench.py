@@ -31,10 +31,10 @@ N_FULL = 64 * 1024 * 1024
 # `bench.py --counter-probe splat` / `--counter-probe splat4` (TCC_ATOMIC_sum per kernel, summed over the
 # iteration's kernels); constants from those profiles, not readings of this run.
 ATOMIC_TRAFFIC = {
-    "config4_10k_512": {"l2_atomic_requests_measured": 132_490, "pairs_in_that_run": 129_843,
-                        "source": "profiles/splat_10k_512_kernel_counters.md (TCC_ATOMIC_sum: render_backward_kernel 132 490, nothing else)"},
-    "config5_200k_2048": {"l2_atomic_requests_measured": 3_666_035, "pairs_in_that_run": 5_500_959,
-                          "source": "profiles/splat_200k_2048_kernel_counters.md (TCC_ATOMIC_sum: render_backward_kernel 3 665 877, scans 158)"},
+    "config4_10k_512": {"l2_atomic_requests_measured": 133_099, "pairs_in_that_run": 129_843,
+                        "source": "profiles/splat_10k_512_kernel_counters.md (TCC_ATOMIC_sum: render_backward_kernel 133 059, cover_kernel 40)"},
+    "config5_200k_2048": {"l2_atomic_requests_measured": 3_667_445, "pairs_in_that_run": 5_500_959,
+                          "source": "profiles/splat_200k_2048_kernel_counters.md (TCC_ATOMIC_sum: render_backward_kernel 3 665 877, cover_kernel 1568)"},
 }
 
 

@@ -240,7 +240,7 @@ int xad_splat_get_lists(xad_splat_context* ctx, uint32_t* range_begin, uint32_t*
  * No counterpart in the reference, whose one kernel needs no lists. */
 int xad_splat_overflow_word(xad_splat_context* ctx, const uint32_t** device_word);
 /* The order in which the step composites: order[i] (device, n words) = the i-th
- * Gaussian by (depth, index), rank (device, n words) its inverse.  A stable radix
+ * Gaussian by (depth, index), rank (device, n words) its inverse.  A stable
  * sort on the device (csrc/splat_sort.hip), the one xad_splat_step runs whenever
  * it has to order (every call in XAD_SPLAT_DEPTH_EVERY_STEP mode).  -0.0 and +0.0
  * are one depth; a NaN sorts by its bit pattern (first with the sign bit set, last
